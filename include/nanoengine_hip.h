@@ -104,8 +104,9 @@ int ne_kv_write(const void* vectors, int32_t vec_dtype, int64_t n, int32_t num_h
  * split_len: most keys per work-group (multiple of 128 up to 2048; 0 = choose: the
  * int8 / 8-KV-head path then sizes each sequence's splits from the total work, at
  * least 256 keys each).  head_dim must be 128 and block_size a multiple of 16.  One
- * work-group serves every KV head of a sequence's split; splits are combined by a
- * second kernel on the same stream.
+ * work-group serves every KV head of a sequence's split, or, with more than 32 query rows
+ * per KV head and split_len 0 (prefill), one KV head of a tile of 64 to 256 query rows;
+ * splits are combined by a second kernel on the same stream.
  */
 size_t ne_paged_attention_workspace_size(int32_t num_seqs, int32_t num_q_heads,
                                          int32_t num_kv_heads, int32_t max_q_len,
@@ -128,9 +129,10 @@ int ne_paged_verify_attention(const void* q, int64_t q_token_stride, int64_t q_h
  * results as ne_paged_verify_attention, except that the work plan and split partials live
  * in a library-owned device array of NE_NOALLOC_SCRATCH_BYTES per GPU (held until the
  * process ends), and the error flag is the caller's device word `error_flag` (bits are
- * OR-ed in as in the workspace's flag; the caller clears it).  A call needing more scratch
- * (ne_paged_attention_workspace_size() > NE_NOALLOC_SCRATCH_BYTES) returns NE_EWORKSPACE
- * without launching.  It allocates nothing: the scratch address is looked up once per
+ * OR-ed in as in the workspace's flag; the caller clears it).  A call whose splits need more
+ * scratch than NE_NOALLOC_SCRATCH_BYTES returns NE_EWORKSPACE without launching: with at
+ * most 32 query rows per KV head, one whose ne_paged_attention_workspace_size() is larger;
+ * with more rows, one whose partials of fixed splits (256 keys of int8, 128 of bf16) are.  It allocates nothing: the scratch address is looked up once per
  * device (hipGetSymbolAddress) on the first call with that device current.  Every call on
  * one GPU shares that GPU's scratch, so calls that overlap on one GPU (concurrent streams)
  * race; calls ordered on one stream do not.

@@ -99,6 +99,8 @@ struct AttnParams {
   int32_t plan_whole;  // planned path: one work item per sequence (head-split kernel)
   int32_t plan_grid;   // DMA kernel: work-groups launched
   int32_t max_ctx;     // the caller's bound on ctx_len
+  int32_t rows_kg;     // query-tile kernel: key groups per work-group (0: another kernel serves the call)
+  int32_t row_tiles;   // query-tile kernel: tiles of query rows per sequence
   int32_t* plan_desc;  // precomputed plan: [plan_grid][8] work items (seq < 0: none)
   int32_t* plan_slots; // precomputed plan: [plan_grid][kPlanMaxTiles] first slot of each tile
 };
@@ -792,6 +794,489 @@ __global__ __launch_bounds__(kHeadWaves * KG * kWave) void paged_attention_kerne
         p.part_ml[pbase * 2] = m;
         p.part_ml[pbase * 2 + 1] = l;
       }
+    }
+  }
+}
+
+// ---- query tiles (prefill: more query rows per KV head than the DMA kernel takes) ----
+// One work-group of 8 waves serves one (sequence, KV head, tile of query rows, key
+// split).  The K and V of 128 keys are read from the pool once per work-group, converted
+// once (int8 codes to fp16, exact; bf16 as they are) and written to LDS as MFMA operands,
+// V transposed; every wave then multiplies them with its own 32 query rows.  The
+// fixed-split kernel above holds 16 rows per wave and reads and converts the K/V of its
+// head again for every 16 rows, so at long prompts its time went into the conversions and
+// the L2 traffic of K/V, and 256-key splits wrote fp32 partials 32 times the output.
+//   rows  = row R of a (sequence, KV head) is query R / group, head R % group of the
+//           GQA group, so a tile of consecutive rows spans few queries and its causal
+//           bound is tight.  Tiles run from the last to the first (longest first), with
+//           the KV head fastest: with 8 KV heads every XCD serves one head, whose K/V
+//           its L2 keeps.
+//   waves = KG key groups x 8 / KG row groups of 32 rows: key group kg takes the 32-key
+//           steps kg, kg + KG, .. of a stage, so that tiles of few rows still use every
+//           wave; the groups' (m, l, O) merge through LDS at the end.
+//   loop  = stage t + 1's loads are issued before the products of stage t and written to
+//           the other LDS buffer after them: one barrier per 128 keys.
+// What bounds it: the softmax VALU work (~30 cycles per score and wave), the MFMAs (32
+// cycles of a SIMD per 64 scores x 128 dims) and the fragment reads (128 B per clock) are
+// each ~2,000 cycles per 64 keys of a 256-row tile; two waves per SIMD overlap them.
+// The running maximum moves only when a lane's probabilities show that it must (their sum
+// passes 2^8), so the common path has no row maximum: one multiply-add, one exponential,
+// one sum and one value-scale multiply per score.
+// Measured (int8 pool, 16 / 8 heads): 8,192 queries after 8,192 tokens 4,885 us in the
+// fixed-split kernel and its merge, 960 us here (860 TFLOP/s); eight prompts of 129-895
+// tokens 152 and 44 us; 16 x 200 queries after 4,096 tokens 666 and 154 us.
+constexpr int kQtWaves = 8;
+constexpr int kQtKeys = 128;                     // keys per stage
+constexpr int kQtMT = 2;                         // 16-row MFMA tiles per wave
+constexpr int kQtWaveRows = kQtMT * kRows;
+constexpr int kQtThreads = kQtWaves * kWave;
+constexpr int kQtTileBytes = kQtKeys * kHeadDim * 2;  // one stage's K (or V^T), 16-bit
+constexpr int kQtStage = 2 * kQtTileBytes;
+constexpr int kQtScaleOff = 2 * kQtStage;        // float [2 buffers][K | V][128 keys]
+constexpr int kQtSlotOff = kQtScaleOff + 2 * 2 * kQtKeys * 4;  // int [2][8 tiles]
+constexpr int kQtFlagOff = kQtSlotOff + 2 * 8 * 4;             // int [2 buffers][2 waves]
+constexpr int kQtLds = kQtFlagOff + 2 * 2 * 4;
+static_assert(kQtLds <= 160 * 1024, "LDS of one CU");
+
+constexpr int kQtMinSplit = 256;                 // keys: a shorter split is mostly prologue and partials
+
+constexpr int qt_rows(int kg) { return kQtWaveRows * kQtWaves / kg; }
+
+// One thread's share of a stage on its way to LDS.
+template <bool INT8>
+struct QtRegs;
+template <>
+struct QtRegs<true> {
+  u32x4 k[2];     // keys tid / 8 + 64 j, codes 16 (tid % 8) .. + 16
+  uint32_t v[8];  // the 8 keys of octet tid / 32, codes 4 (tid % 32) .. + 4
+  float sc;       // thread < 128: key scale; < 256: value scale of key tid % 128
+};
+template <>
+struct QtRegs<false> {
+  u32x4 k[4];  // keys tid / 16 + 32 j, dims 8 (tid % 16) .. + 8
+  u32x2 v[8];  // the 8 keys of octet tid / 32, dims 4 (tid % 32) .. + 4
+};
+
+// Key of octet o (0..15), element e: the contraction order of the second product, whose
+// P operand holds keys 16 (e / 4) + 4 g + e % 4 of a 32-key step (o = 4 step + g).
+__device__ __forceinline__ int qt_octet_key(int o, int e) {
+  return 32 * (o >> 2) + 16 * (e >> 2) + 4 * (o & 3) + (e & 3);
+}
+
+// 16-byte chunk position in the LDS rows (256 B: a key's dims, or a dim's keys): spreads
+// both the transposing writes (rows 4 apart) and the fragment reads (rows 1 apart)
+__device__ __forceinline__ int qt_k_pos(int key, int chunk) { return chunk ^ (key & 15); }
+__device__ __forceinline__ int qt_v_pos(int dim, int chunk) { return chunk ^ ((dim ^ ((dim >> 3) & 1)) & 7); }
+
+template <bool INT8, int SDT>
+__device__ __forceinline__ void qt_load(const AttnParams& p, const int* s_slot, int kb, int kend, int head,
+                                        int tid, QtRegs<INT8>& R) {
+  constexpr int kEsz = INT8 ? 1 : 2;
+  const int64_t slot_bytes = (int64_t)p.num_kv_heads * kHeadDim * kEsz;
+  const char* kc = (const char*)p.k_cache + (int64_t)head * kHeadDim * kEsz;
+  const char* vc = (const char*)p.v_cache + (int64_t)head * kHeadDim * kEsz;
+#pragma unroll
+  for (int j = 0; j < (INT8 ? 2 : 4); ++j) {
+    const int key = INT8 ? (tid >> 3) + 64 * j : (tid >> 4) + 32 * j;
+    const int64_t slot = s_slot[key >> 4] + (key & 15);
+    R.k[j] = *(const u32x4*)(kc + slot * slot_bytes + 16 * (tid & (INT8 ? 7 : 15)));
+  }
+  const int o = tid >> 5;
+  const int64_t slot0 = s_slot[2 * (o >> 2)] + 4 * (o & 3);
+  const int64_t slot1 = s_slot[2 * (o >> 2) + 1] + 4 * (o & 3);
+  const char* v0 = vc + slot0 * slot_bytes + 4 * kEsz * (tid & 31);
+  const char* v1 = vc + slot1 * slot_bytes + 4 * kEsz * (tid & 31);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const char* src = (e < 4 ? v0 : v1) + (e & 3) * slot_bytes;
+    if constexpr (INT8) {
+      R.v[e] = *(const uint32_t*)src;
+    } else {
+      R.v[e] = *(const u32x2*)src;
+    }
+  }
+  if constexpr (INT8) {
+    R.sc = 0.f;
+    if (tid < 2 * kQtKeys) {  // whole waves
+      const int key = tid & (kQtKeys - 1);
+      const int64_t slot = s_slot[key >> 4] + (key & 15);
+      const float s = load_scale<SDT>(tid < kQtKeys ? p.k_scale : p.v_scale, slot * p.num_kv_heads + head);
+      R.sc = kb + key < kend ? s : 0.f;  // a slot past the context's end may hold anything
+    }
+  } else {
+    // bf16 values past the context's end may be stale bit patterns: 0 * NaN must not
+    // reach the product (int8 codes are always finite)
+    if (kb + kQtKeys > kend) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (kb + qt_octet_key(o, e) >= kend) R.v[e] = u32x2{0, 0};
+    }
+  }
+}
+
+template <bool INT8>
+__device__ __forceinline__ void qt_store(char* smem, int buf, int tid, int wave, int lane, float qk_scale,
+                                         const QtRegs<INT8>& R) {
+  char* ks = smem + buf * kQtStage;
+  char* vs = ks + kQtTileBytes;
+  const int o = tid >> 5;
+  const int q = tid & 31;
+  if constexpr (INT8) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int key = (tid >> 3) + 64 * j;
+      const int c = 2 * (tid & 7);
+      *(u32x4*)(ks + key * 256 + qt_k_pos(key, c) * 16) = i8x8_f16x8(R.k[j][0], R.k[j][1]);
+      *(u32x4*)(ks + key * 256 + qt_k_pos(key, c + 1) * 16) = i8x8_f16x8(R.k[j][2], R.k[j][3]);
+    }
+    *(u32x4*)(vs + (4 * q + 0) * 256 + qt_v_pos(4 * q + 0, o) * 16) = i8_cols_f16x8<0>(R.v);
+    *(u32x4*)(vs + (4 * q + 1) * 256 + qt_v_pos(4 * q + 1, o) * 16) = i8_cols_f16x8<1>(R.v);
+    *(u32x4*)(vs + (4 * q + 2) * 256 + qt_v_pos(4 * q + 2, o) * 16) = i8_cols_f16x8<2>(R.v);
+    *(u32x4*)(vs + (4 * q + 3) * 256 + qt_v_pos(4 * q + 3, o) * 16) = i8_cols_f16x8<3>(R.v);
+    if (tid < 2 * kQtKeys) {
+      // key scales carry the softmax scale; value scales the fp16 range check
+      float* sc = (float*)(smem + kQtScaleOff) + buf * 2 * kQtKeys;
+      sc[tid] = tid < kQtKeys ? R.sc * qk_scale : R.sc;
+      const bool big = __ballot(R.sc > kLazyMaxVScale) != 0;
+      if (tid >= kQtKeys && lane == 0) ((int*)(smem + kQtFlagOff))[buf * 2 + wave - kQtKeys / kWave] = big;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int key = (tid >> 4) + 32 * j;
+      *(u32x4*)(ks + key * 256 + qt_k_pos(key, tid & 15) * 16) = R.k[j];
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int w = b >> 1;
+      const uint32_t sel = (b & 1) ? 0x07060302u : 0x05040100u;
+      const u32x4 col = {__builtin_amdgcn_perm(R.v[1][w], R.v[0][w], sel), __builtin_amdgcn_perm(R.v[3][w], R.v[2][w], sel),
+                         __builtin_amdgcn_perm(R.v[5][w], R.v[4][w], sel), __builtin_amdgcn_perm(R.v[7][w], R.v[6][w], sel)};
+      *(u32x4*)(vs + (4 * q + b) * 256 + qt_v_pos(4 * q + b, o) * 16) = col;
+    }
+  }
+}
+
+// A wave's running state over its query rows: lane (r, g) has row r of each 16-row tile,
+// this lane's share of the row sum, and dims 16 j + 4 g + i of the output.
+template <bool INT8>
+struct QtState {
+  QFrag<INT8> q[kQtMT];
+  float m[kQtMT], l[kQtMT];
+  floatx4 o[kQtMT][8];
+};
+
+// One 32-key step: keys kb .. + 32 are step u of the stage in LDS.  masked (wave-uniform):
+// some row does not see every key of the step.
+template <bool INT8>
+__device__ __forceinline__ void qt_step(const char* smem, int buf, int u, int kb, const int (&kend_row)[kQtMT],
+                                        bool masked, float limit, float qk_scale, int lane, QtState<INT8>& st) {
+  const int r = lane & 15;
+  const int g = lane >> 4;
+  const char* ks = smem + buf * kQtStage;
+  const char* vs = ks + kQtTileBytes;
+  // ---- S^T = K . Q^T: two tiles of 16 keys x 16 rows per row tile ----
+  floatx4 s[kQtMT][2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+#pragma unroll
+    for (int mt = 0; mt < kQtMT; ++mt) s[mt][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const u32x4 a = *(const u32x4*)(ks + (32 * u + 16 * t + r) * 256 + qt_k_pos(r, 4 * c + g) * 16);
+#pragma unroll
+      for (int mt = 0; mt < kQtMT; ++mt) {
+        if constexpr (INT8) {
+          s[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), st.q[mt].q[c], s[mt][t], 0, 0, 0);
+        } else {
+          s[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), st.q[mt].q[c], s[mt][t], 0, 0, 0);
+        }
+      }
+    }
+  }
+  floatx4 kf[2], vf[2];
+  if constexpr (INT8) {
+    const float* sc = (const float*)(smem + kQtScaleOff) + buf * 2 * kQtKeys + 32 * u + 4 * g;
+    kf[0] = *(const floatx4*)sc;
+    kf[1] = *(const floatx4*)(sc + 16);
+    vf[0] = *(const floatx4*)(sc + kQtKeys);
+    vf[1] = *(const floatx4*)(sc + kQtKeys + 16);
+  }
+  // ---- probabilities; the reference maximum moves only when they outgrow it ----
+  auto factor = [&](int e) { return INT8 ? kf[e >> 2][e & 3] : qk_scale; };
+  auto seen = [&](int mt, int e) { return kb + 16 * (e >> 2) + 4 * g + (e & 3) < kend_row[mt]; };
+  float pr[kQtMT][8], psum[kQtMT];
+  auto probs = [&]() {
+#pragma unroll
+    for (int mt = 0; mt < kQtMT; ++mt)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        pr[mt][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[mt][e >> 2][e & 3], factor(e), -st.m[mt]));
+    if (masked) {
+#pragma unroll
+      for (int mt = 0; mt < kQtMT; ++mt)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pr[mt][e] = seen(mt, e) ? pr[mt][e] : 0.f;
+    }
+#pragma unroll
+    for (int mt = 0; mt < kQtMT; ++mt) {
+      psum[mt] = pr[mt][0];
+#pragma unroll
+      for (int e = 1; e < 8; ++e) psum[mt] += pr[mt][e];
+    }
+  };
+  probs();
+  if (__ballot(psum[0] > limit || psum[1] > limit)) {
+#pragma unroll
+    for (int mt = 0; mt < kQtMT; ++mt) {
+      float mx = kNegBig;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, seen(mt, e) ? s[mt][e >> 2][e & 3] * factor(e) : kNegBig);
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      const float m_new = fmaxf(st.m[mt], mx);
+      const float alpha = __builtin_amdgcn_exp2f(st.m[mt] - m_new);
+      st.l[mt] *= alpha;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) st.o[mt][j] *= alpha;
+      st.m[mt] = m_new;
+    }
+    probs();
+  }
+  u32x4 pb[kQtMT];
+#pragma unroll
+  for (int mt = 0; mt < kQtMT; ++mt) {
+    st.l[mt] += psum[mt];
+    const float(&x)[8] = pr[mt];
+    if constexpr (INT8) {
+      pb[mt] = u32x4{pack_f16x2(x[0] * vf[0][0], x[1] * vf[0][1]), pack_f16x2(x[2] * vf[0][2], x[3] * vf[0][3]),
+                     pack_f16x2(x[4] * vf[1][0], x[5] * vf[1][1]), pack_f16x2(x[6] * vf[1][2], x[7] * vf[1][3])};
+    } else {
+      pb[mt] = u32x4{pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]), pack_bf16x2(x[4], x[5]), pack_bf16x2(x[6], x[7])};
+    }
+  }
+  // ---- O^T += V^T . P^T: eight tiles of 16 dims x 16 rows per row tile ----
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const u32x4 a = *(const u32x4*)(vs + r * 256 + qt_v_pos(r, 4 * u + g) * 16 + j * 16 * 256);
+#pragma unroll
+    for (int mt = 0; mt < kQtMT; ++mt) {
+      if constexpr (INT8) {
+        st.o[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, pb[mt]),
+                                                             st.o[mt][j], 0, 0, 0);
+      } else {
+        st.o[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, pb[mt]),
+                                                              st.o[mt][j], 0, 0, 0);
+      }
+    }
+  }
+}
+
+// Rows, keys and splits of one (sequence, query tile); the same in the merge kernel.
+struct QtItem {
+  int ctx, ql, qs, row0, rows_total, kend, n_splits;
+};
+
+__device__ __forceinline__ QtItem qt_item(const AttnParams& p, int seq, int tile, int tile_rows) {
+  QtItem it;
+  // a context beyond the caller's bound is clipped to it (and flagged by the kernel), so
+  // that no block-table entry past max_ctx is read
+  it.ctx = min(((const ConstI32*)p.ctx_len)[seq], p.max_ctx);
+  it.ql = ((const ConstI32*)p.q_len)[seq];
+  it.qs = ((const ConstI32*)p.q_start)[seq];
+  it.rows_total = p.group * it.ql;
+  it.row0 = tile * tile_rows;
+  it.kend = 0;
+  it.n_splits = 0;
+  if (it.row0 < it.rows_total) {
+    const int last = (min(it.row0 + tile_rows, it.rows_total) - 1) / p.group;  // last query of the tile
+    it.kend = it.ctx - it.ql + last + 1;
+    it.n_splits = it.kend > 0 ? min((it.kend + p.split_len - 1) / p.split_len, p.max_splits) : 0;
+  }
+  return it;
+}
+
+template <bool INT8, int SDT, int KG>
+__global__ __launch_bounds__(kQtThreads) void paged_attention_rows_kernel(AttnParams p) {
+  constexpr int kTileRows_ = qt_rows(KG);
+  constexpr int kRowGroups = kQtWaves / KG;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lane = tid % kWave;
+
+  // ---- work item: KV head fastest, then the sequence, the tiles from the last down ----
+  int b = blockIdx.x;
+  const int head = b % p.num_kv_heads;
+  b /= p.num_kv_heads;
+  const int split = b % p.max_splits;
+  b /= p.max_splits;
+  const int seq = b % p.num_seqs;
+  const int tile = p.row_tiles - 1 - b / p.num_seqs;
+  const QtItem it = qt_item(p, seq, tile, kTileRows_);
+  if (tid == 0 && ((const ConstI32*)p.ctx_len)[seq] > p.max_ctx) atomicOr(p.error_flag, 1u);
+  if (split >= it.n_splits) return;
+  const int kstart = split * p.split_len;
+  const int kend = min(it.kend, kstart + p.split_len);
+  const int n_stages = (kend - kstart + kQtKeys - 1) / kQtKeys;
+
+  // ---- this wave's rows ----
+  const int r = lane & 15;
+  const int g = lane >> 4;
+  const int kg = wave / kRowGroups;
+  const int wrow0 = it.row0 + (wave % kRowGroups) * kQtWaveRows;
+  int kend_row[kQtMT];
+  QtState<INT8> st;
+  int kend_wave = 0, kfull_wave = 0;  // keys some row of the wave sees; keys every row sees
+  if (wrow0 < it.rows_total) {
+    const int last = (min(wrow0 + kQtWaveRows, it.rows_total) - 1) / p.group;
+    kend_wave = min(kend, it.ctx - it.ql + last + 1);
+    kfull_wave = min(kend, it.ctx - it.ql + wrow0 / p.group + 1);
+  }
+
+  // ---- stages of 128 keys ----
+  // first slot of each 16-key tile of a stage, in a ring of two (read one stage before
+  // its data, by 8 threads); tiles past the last key re-read the last key's tile
+  int* s_slot = (int*)(smem + kQtSlotOff);
+  const int32_t* bt = p.block_tables + (int64_t)seq * p.bt_stride;
+  auto tile_slot = [&](int tile16) {
+    const int key = min(kstart + kTileKeys * tile16, (kend - 1) & ~(kTileKeys - 1));
+    return bt[key / p.block_size] * p.block_size + key % p.block_size;
+  };
+  // the first two stages' slots and this wave's Q rows are requested together; Q is
+  // converted behind the first stage's loads
+  int slot0 = 0;
+  if (tid < 16) slot0 = tile_slot(tid);
+  u32x4 raw[kQtMT][4];
+#pragma unroll
+  for (int mt = 0; mt < kQtMT; ++mt) {
+    const int row = wrow0 + kRows * mt + r;
+    const bool valid = row < it.rows_total;
+    const int qi = valid ? row / p.group : 0;
+    kend_row[mt] = valid ? min(kend, it.ctx - it.ql + qi + 1) : kend;
+    // a row past the last reads the sequence's first row; its results are never stored
+    const uint16_t* src = p.q + (int64_t)(it.qs + qi) * p.q_tok_stride +
+                          (int64_t)(head * p.group + (valid ? row - qi * p.group : 0)) * p.q_head_stride + 8 * g;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) raw[mt][c] = *(const u32x4*)(src + 32 * c);
+  }
+  if (tid < 16) s_slot[tid] = slot0;
+  lds_barrier();
+  QtRegs<INT8> R;
+  qt_load<INT8, SDT>(p, s_slot, kstart, kend, head, tid, R);
+  __asm__ __volatile__("" ::: "memory");
+#pragma unroll
+  for (int mt = 0; mt < kQtMT; ++mt) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if constexpr (INT8) {
+        u32x4 h;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          h[i] = pack_f16x2(bf16_to_f32((uint16_t)(raw[mt][c][i] & 0xFFFFu)),
+                            bf16_to_f32((uint16_t)(raw[mt][c][i] >> 16)));
+        st.q[mt].q[c] = __builtin_bit_cast(f16x8, h);
+      } else {
+        st.q[mt].q[c] = __builtin_bit_cast(bf16x8, raw[mt][c]);
+      }
+    }
+    st.m[mt] = kNegBig;
+    st.l[mt] = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) st.o[mt][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  qt_store<INT8>(smem, 0, tid, wave, lane, p.qk_scale, R);
+  __syncthreads();
+  for (int t = 0; t < n_stages; ++t) {
+    const int buf = t & 1;
+    const int kb0 = kstart + t * kQtKeys;
+    const bool more = t + 1 < n_stages;
+    int next_slot = 0;
+    if (more) {
+      qt_load<INT8, SDT>(p, s_slot + 8 * (buf ^ 1), kb0 + kQtKeys, kend, head, tid, R);
+      if (tid < 8) next_slot = tile_slot(8 * (t + 2) + tid);
+    }
+    __asm__ __volatile__("" ::: "memory");  // the loads go out before the products
+    float limit = 256.f;  // 2^kLazyLog2
+    if constexpr (INT8) {
+      // probabilities up to 2^8 times a value scale up to 128 stay inside fp16; a stage
+      // with a larger scale keeps them at 1
+      const int* big = (const int*)(smem + kQtFlagOff) + buf * 2;
+      if (__builtin_amdgcn_readfirstlane(big[0] | big[1])) limit = 1.f;
+    }
+#pragma unroll 1
+    for (int u = kg; u < 4; u += KG) {
+      const int kb = kb0 + 32 * u;
+      if (kb >= kend_wave) break;
+      qt_step<INT8>(smem, buf, u, kb, kend_row, kb + 32 > kfull_wave, limit, p.qk_scale, lane, st);
+    }
+    if (more) {
+      qt_store<INT8>(smem, buf ^ 1, tid, wave, lane, p.qk_scale, R);
+      if (tid < 8) s_slot[8 * buf + tid] = next_slot;
+    }
+    __syncthreads();
+  }
+
+  // ---- merge the key groups through LDS (the stages are done) ----
+#pragma unroll
+  for (int mt = 0; mt < kQtMT; ++mt) {
+    st.l[mt] += __shfl_xor(st.l[mt], 16);
+    st.l[mt] += __shfl_xor(st.l[mt], 32);
+  }
+  if constexpr (KG > 1) {
+    // [key group - 1][row group][mt][9 vectors][64 lanes]: 8 output vectors and (m, l)
+    floatx4* s_part = (floatx4*)smem;
+    auto part_at = [&](int q, int mt, int j) -> floatx4& {
+      return s_part[((((q - 1) * kRowGroups + wave % kRowGroups) * kQtMT + mt) * 9 + j) * kWave + lane];
+    };
+    static_assert((KG - 1) * kRowGroups * kQtMT * 9 * kWave * 16 <= kQtScaleOff, "partials fit the stages");
+    if (kg > 0) {
+#pragma unroll
+      for (int mt = 0; mt < kQtMT; ++mt) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) part_at(kg, mt, j) = st.o[mt][j];
+        part_at(kg, mt, 8) = floatx4{st.m[mt], st.l[mt], 0.f, 0.f};
+      }
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int mt = 0; mt < kQtMT; ++mt) {
+#pragma unroll
+      for (int q = 1; q < KG; ++q) {
+        const floatx4 ml = part_at(q, mt, 8);
+        const float mm = fmaxf(st.m[mt], ml[0]);
+        const float a0 = __builtin_amdgcn_exp2f(st.m[mt] - mm);
+        const float a1 = __builtin_amdgcn_exp2f(ml[0] - mm);
+        st.l[mt] = a0 * st.l[mt] + a1 * ml[1];
+        st.m[mt] = mm;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) st.o[mt][j] = a0 * st.o[mt][j] + a1 * part_at(q, mt, j);
+      }
+    }
+  }
+
+  // ---- outputs (one split) or fp32 partials ----
+#pragma unroll
+  for (int mt = 0; mt < kQtMT; ++mt) {
+    const int row = wrow0 + kRows * mt + r;
+    if (row >= it.rows_total) continue;
+    if (it.n_splits == 1) {
+      const int qi = row / p.group;
+      uint16_t* dst = p.out + (int64_t)(it.qs + qi) * p.o_tok_stride +
+                      (int64_t)(head * p.group + row - qi * p.group) * p.o_head_stride + 4 * g;
+      const float inv = 1.f / st.l[mt];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        *(u32x2*)(dst + 16 * j) = u32x2{pack_bf16x2(st.o[mt][j][0] * inv, st.o[mt][j][1] * inv),
+                                        pack_bf16x2(st.o[mt][j][2] * inv, st.o[mt][j][3] * inv)};
+    } else {
+      const int64_t part = (((int64_t)(seq * p.row_tiles + tile) * p.num_kv_heads + head) * p.max_splits + split) *
+                               kTileRows_ + row - it.row0;
+      float* po = p.part_o + part * kHeadDim + 4 * g;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) *(floatx4*)(po + 16 * j) = st.o[mt][j];
+      if (g == 0) *(float2*)(p.part_ml + part * 2) = float2{st.m[mt], st.l[mt]};
     }
   }
 }
@@ -1889,8 +2374,30 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnParams p) {
   merge_partials(p, n_splits, cd, [&](int s) { return ubase + (int64_t)s * kRows; }, dst);
 }
 
+// Combines the split partials of the query-tile kernel: one work-group per (sequence,
+// tile, KV head, 16 rows), 16 threads per row, 8 dims per thread.
+__global__ __launch_bounds__(256) void attention_rows_merge_kernel(AttnParams p, int tile_rows) {
+  const int blocks = tile_rows / kRows;
+  int b = blockIdx.x;
+  const int row = (b % blocks) * kRows + (threadIdx.x >> 4);
+  b /= blocks;
+  const int head = b % p.num_kv_heads;
+  b /= p.num_kv_heads;
+  const int tile = b % p.row_tiles;
+  const int seq = b / p.row_tiles;
+  const QtItem it = qt_item(p, seq, tile, tile_rows);
+  if (it.n_splits <= 1 || it.row0 + row >= it.rows_total) return;
+  const int cd = (threadIdx.x & 15) * 8;
+  const int64_t base = ((int64_t)(seq * p.row_tiles + tile) * p.num_kv_heads + head) * p.max_splits * tile_rows + row;
+  const int qi = (it.row0 + row) / p.group;
+  uint16_t* dst = p.out + (int64_t)(it.qs + qi) * p.o_tok_stride +
+                  (int64_t)(head * p.group + it.row0 + row - qi * p.group) * p.o_head_stride + cd;
+  merge_partials(p, it.n_splits, cd, [&](int s) { return base + (int64_t)s * tile_rows; }, dst);
+}
+
 struct Layout {
   int group, mtiles, units, split_len, max_splits, plan_grid, plan_w;
+  int rows_kg, row_tiles;  // query-tile kernel: key groups per work-group (0: not its shape), tiles per sequence
   size_t part_o_off, part_ml_off, error_off, plan_off, desc_off, slots_off, total;
 };
 
@@ -1919,12 +2426,55 @@ int default_split_len(int kv_dtype, int max_ctx) {
   return min(split_len, max(128, ceil_div(max(max_ctx, 1), 128) * 128));
 }
 
+// Key groups per work-group of the query-tile kernel: the most (so the smallest tiles)
+// whose tile holds all rows, or, for contexts of up to kQtShortCtx keys, that need no more
+// work-groups than there are CUs: one sequence of 512 queries and no cached token takes
+// 17.5 us in 64-row tiles and 23 us in 256-row ones, 16 of 65 queries after 300 tokens 18
+// and 30 us.  Over longer contexts every tile stages the same K/V again while key splits
+// fill the CUs as well: 16 of 65 after 4,096 tokens take 98 us in 64-row tiles and 89 us in
+// 256-row ones, one of 512 51 and 48 us.
+constexpr int kQtShortCtx = 1024;
+int rows_key_groups(int64_t rows, int64_t seq_heads, int max_ctx) {
+  for (int kg : {4, 2})
+    if (rows <= qt_rows(kg) || (max_ctx <= kQtShortCtx && seq_heads * ceil_div(rows, qt_rows(kg)) <= kPlanCUs))
+      return kg;
+  return 1;
+}
+
+// Whether the query-tile kernel serves a shape: more rows per KV head than the DMA kernel
+// takes and no split length asked for.  Contexts of at most 64 keys stay with the register
+// kernel, which has one split of them and no staging to pay for: 7.4 us against 9.0-9.9 us
+// at 17-32 queries of a bf16 cache, 9.5-9.7 us against 9.0-9.9 us at 17-64 of an int8 one.
+bool rows_serves(int mtiles, int split_len, int max_ctx) {
+  return mtiles > kMaxRowTiles && split_len <= 0 && max_ctx > 4 * kTileKeys;
+}
+
+// rows_path: whether the query-tile kernel may serve the shape.
 Layout make_layout(int num_seqs, int num_q_heads, int num_kv_heads, int max_q_len, int max_ctx,
-                   int split_len, int kv_dtype) {
+                   int split_len, int kv_dtype, bool rows_path = true) {
   Layout L{};
   L.group = num_q_heads / num_kv_heads;
   L.mtiles = ceil_div((int64_t)L.group * max_q_len, kRows);
   L.units = num_seqs * num_kv_heads * L.mtiles;
+  if (rows_path && rows_serves(L.mtiles, split_len, max_ctx)) {
+    // one work-group per CU: where the tiles give fewer, the keys are split over the rest
+    const int64_t rows = (int64_t)L.group * max_q_len;
+    L.rows_kg = rows_key_groups(rows, (int64_t)num_seqs * num_kv_heads, max_ctx);
+    const int tile_rows = qt_rows(L.rows_kg);
+    L.row_tiles = ceil_div(rows, tile_rows);
+    const int64_t groups = (int64_t)num_seqs * num_kv_heads * L.row_tiles;
+    const int want = (int)max((int64_t)1, (int64_t)kPlanCUs / groups);
+    L.split_len = max(kQtMinSplit, ceil_div(ceil_div(max(max_ctx, 1), want), kQtKeys) * kQtKeys);
+    L.max_splits = ceil_div(max(max_ctx, 1), L.split_len);
+    const size_t parts = L.max_splits > 1 ? (size_t)groups * L.max_splits * tile_rows : 0;
+    size_t at = 256;  // the error flag
+    L.part_o_off = at;
+    at += parts * kHeadDim * sizeof(float);
+    L.part_ml_off = at;
+    at += (parts * 2 * sizeof(float) + 255) & ~(size_t)255;
+    L.plan_off = L.desc_off = L.slots_off = L.total = at;
+    return L;
+  }
   const int fixed_split = split_len > 0 ? split_len : 0;  // 0: the caller left it to us
   if (split_len <= 0) split_len = default_split_len(kv_dtype, max_ctx);
   L.split_len = split_len;
@@ -1962,6 +2512,33 @@ Layout make_layout(int num_seqs, int num_q_heads, int num_kv_heads, int max_q_le
   L.slots_off = take(plan ? (size_t)L.plan_grid * kPlanMaxTiles * sizeof(int32_t) : 0);
   L.total = off;
   return L;
+}
+
+template <bool INT8, int SDT, int KG>
+int launch_attention_rows_kg(const AttnParams& p, hipStream_t s) {
+  static const hipError_t attr = hipFuncSetAttribute((const void*)paged_attention_rows_kernel<INT8, SDT, KG>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kQtLds);
+  if (attr != hipSuccess) {
+    set_error("paged_attention_rows_kernel: cannot reserve %d bytes of LDS: %s", kQtLds, hipGetErrorString(attr));
+    return NE_ELAUNCH;
+  }
+  const int64_t tiles = (int64_t)p.num_seqs * p.row_tiles * p.num_kv_heads;
+  const int64_t merges = tiles * (qt_rows(KG) / kRows);
+  NE_CHECK_SUPPORTED(tiles * p.max_splits < (int64_t(1) << 31) && merges < (int64_t(1) << 31),
+                     "too many query tiles (%lld)", (long long)tiles);
+  hipLaunchKernelGGL((paged_attention_rows_kernel<INT8, SDT, KG>), dim3((unsigned)(tiles * p.max_splits)),
+                     dim3(kQtThreads), kQtLds, s, p);
+  const int rc = check_launch("paged_attention_rows_kernel");
+  if (rc != NE_OK || p.max_splits == 1) return rc;
+  hipLaunchKernelGGL(attention_rows_merge_kernel, dim3((unsigned)merges), dim3(256), 0, s, p, qt_rows(KG));
+  return check_launch("attention_rows_merge_kernel");
+}
+
+template <bool INT8, int SDT>
+int launch_attention_rows(const AttnParams& p, hipStream_t s) {
+  if (p.rows_kg == 4) return launch_attention_rows_kg<INT8, SDT, 4>(p, s);
+  if (p.rows_kg == 2) return launch_attention_rows_kg<INT8, SDT, 2>(p, s);
+  return launch_attention_rows_kg<INT8, SDT, 1>(p, s);
 }
 
 template <int KG, bool DB>
@@ -2122,6 +2699,8 @@ int make_params(const void* q, int64_t q_token_stride, int64_t q_head_stride, co
   p.plan_grid = L.plan_grid;
   p.plan_whole = 0;  // the planned entry point decides
   p.max_ctx = max_ctx_len;
+  p.rows_kg = L.rows_kg;
+  p.row_tiles = L.row_tiles;
   return NE_OK;
 }
 
@@ -2161,6 +2740,13 @@ int scratch_for_current_device(void** out) {
 // the unplanned call on a prepared parameter block (shared by both unplanned entry points)
 int run_unplanned(AttnParams& p, int32_t kv_dtype, int32_t scale_dtype, int32_t num_kv_heads,
                   int32_t num_seqs, const void* k_scale, const void* v_scale, hipStream_t stream) {
+  // More than 32 rows per KV head and no fixed split length: the query-tile kernel.
+  if (p.rows_kg > 0) {
+    if (kv_dtype == NE_DTYPE_BF16) return launch_attention_rows<false, NE_DTYPE_BF16>(p, stream);
+    if (scale_dtype == NE_DTYPE_BF16) return launch_attention_rows<true, NE_DTYPE_BF16>(p, stream);
+    if (scale_dtype == NE_DTYPE_FP16) return launch_attention_rows<true, NE_DTYPE_FP16>(p, stream);
+    return launch_attention_rows<true, NE_DTYPE_FP32>(p, stream);
+  }
   // 8 KV heads, up to two M tiles, bf16 or int8 with 2-byte scales: the DMA kernel on
   // the balanced plan.  Other int8 shapes: one wave per KV head, registers
   // double-buffered (154 VGPRs); other bf16 shapes: single-buffered (double-buffered it
@@ -2228,7 +2814,10 @@ extern "C" int ne_paged_verify_attention_noalloc(
   NE_CHECK_ARG(num_q_heads > 0 && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 && max_q_len > 0 &&
                    max_ctx_len > 0,
                "bad attention shape");
-  const Layout L = make_layout(num_seqs, num_q_heads, num_kv_heads, max_q_len, max_ctx_len, split_len, kv_dtype);
+  // the limit is the fixed-split layout's, whichever kernel serves the shape (the query-tile
+  // kernel's layout is the smaller one)
+  const Layout L = make_layout(num_seqs, num_q_heads, num_kv_heads, max_q_len, max_ctx_len, split_len, kv_dtype,
+                               /*rows_path=*/false);
   if (L.total > kNoAllocScratchBytes) {
     set_error("this call needs %zu bytes of scratch; the allocation-free entry point holds at most %zu "
               "(%d sequences, max_q_len %d, max_ctx_len %d): use ne_paged_verify_attention with a workspace",

@@ -1,0 +1,156 @@
+"""A6 at prefill shapes: the query-tile attention kernel (more than 32 query rows per KV head)
+against the oracle (fp32 restatement of ne/models/attention_context.py:57-109).
+
+Bar: 6e-3 relative (2-norm).  The roundings that differ from the oracle's are each uniform
+relative errors of at most 2^-9 (1.1e-3 rms): the bf16 output, the 16-bit probabilities, and
+the oracle's own 16-bit dequantised keys and values; four of them add up to 2.3e-3 and the
+bar leaves a factor of 2.6.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from helpers import make_batch, make_pool, real_rows, rel_err
+from oracle.attention import paged_attention_reference
+from nanoengine_amd import _native, kernels
+
+pytestmark = pytest.mark.gpu
+
+TOL = 6e-3
+
+
+def run(device, q_lens, pasts, kv, scale_dtype=torch.bfloat16, heads=(16, 8), block_size=16, padded_q=None,
+        spoil=False, value_scale=1.0, workspace=None, strided=False):
+    """(result, oracle) on the real rows.  spoil: slots outside every context hold NaN (bf16
+    values, int8 scales)."""
+    hq, hkv = heads
+    ctx_lens = [q + p for q, p in zip(q_lens, pasts)]
+    num_blocks = sum(-(-c // block_size) for c in ctx_lens) + 3
+    kc, vc, ks, vs = make_pool(num_blocks, block_size, hkv, "bf16" if kv == "bf16" else "int8", scale_dtype, seed=21)
+    tables, ctx, qs, ql, rows = make_batch(ctx_lens, q_lens, num_blocks, block_size, seed=22, padded_q=padded_q)
+    q = torch.randn(rows, hq, 128, generator=torch.Generator().manual_seed(23)).to(torch.bfloat16)
+    if vs is not None:
+        vs = (vs.float() * value_scale).to(vs.dtype)
+    ref = paged_attention_reference(q, kc, vc, ks, vs, tables, block_size, ctx, qs, ql,
+                                    model_dtype=scale_dtype if kv != "bf16" else torch.bfloat16)
+    if spoil:
+        used = torch.zeros(kc.shape[0], dtype=torch.bool)
+        for i, c in enumerate(ctx_lens):
+            at = torch.arange(c)
+            used[tables[i, at // block_size].long() * block_size + at % block_size] = True
+        for t in ((kc, vc) if kv == "bf16" else (ks, vs)):
+            t[~used] = float("nan")
+    d = lambda t: None if t is None else t.to(device)
+    qd = d(q)
+    out = None
+    if strided:  # rows of a wider tensor, heads apart: strides of their own for q and out
+        wide = torch.zeros(rows, 2 * hq + 1, 128, dtype=torch.bfloat16, device=device)
+        wide[:, :2 * hq:2] = qd
+        qd = wide[:, :2 * hq:2]
+        out = torch.empty(rows, hq + 3, 128, dtype=torch.bfloat16, device=device)[:, 1:1 + hq]
+    got = kernels.paged_verify_attention(qd, d(kc), d(vc), d(ks), d(vs), d(tables), block_size, d(ctx), d(qs), d(ql),
+                                         max_q_len=max(q_lens), max_ctx_len=max(ctx_lens), out=out,
+                                         workspace=workspace)
+    torch.cuda.synchronize()
+    idx = real_rows(qs, ql)
+    return got.cpu()[idx], ref[idx]
+
+
+# rows per KV head (2 heads): 34 and 64 (four key groups), 66 and 128 (two), 130, 256 and 258
+# (one tile, one past it); contexts of less than a 32-key step, on and next to a stage's end
+@pytest.mark.parametrize("kv", ["bf16", "int8"])
+@pytest.mark.parametrize("q_lens,pasts", [
+    ([17], [0]), ([32, 17, 31], [0, 95, 97]), ([33, 20], [95, 236]), ([64, 1, 63], [64, 500, 1]),
+    ([65, 65, 5], [0, 63, 0]), ([128, 127], [0, 129]), ([129, 3, 257], [0, 40, 127]), ([512], [0]),
+])
+def test_row_tiles(device, kv, q_lens, pasts):
+    got, ref = run(device, q_lens, pasts, kv)
+    assert torch.isfinite(got.float()).all()
+    assert rel_err(got, ref) < TOL
+
+
+@pytest.mark.parametrize("kv", ["bf16", "int8"])
+@pytest.mark.parametrize("q_lens,pasts", [([20], [1500]), ([150], [700]), ([40, 17], [2000, 256])])
+def test_key_splits_and_their_merge(device, kv, q_lens, pasts):
+    """Few tiles: the keys are split over the idle CUs; the last split's keys are hidden from
+    the first rows, and the shorter sequence has fewer splits than the longer one."""
+    got, ref = run(device, q_lens, pasts, kv)
+    assert rel_err(got, ref) < TOL
+
+
+@pytest.mark.parametrize("scale_dtype", [torch.float16, torch.float32])
+def test_scale_types(device, scale_dtype):
+    got, ref = run(device, [70, 40], [30, 300], "int8", scale_dtype)
+    assert rel_err(got, ref) < TOL
+
+
+@pytest.mark.parametrize("heads", [(8, 8), (8, 2), (6, 1), (12, 3)])
+def test_head_counts(device, heads):
+    group = heads[0] // heads[1]
+    got, ref = run(device, [140 // group + 1, 36], [11, 45], "int8", heads=heads)
+    assert rel_err(got, ref) < TOL
+
+
+@pytest.mark.parametrize("kv", ["bf16", "int8"])
+def test_stale_slots_strides_and_layout(device, kv):
+    got, ref = run(device, [37, 50], [7, 90], kv, block_size=32, padded_q=64, spoil=True, strided=True)
+    assert torch.isfinite(got.float()).all()
+    assert rel_err(got, ref) < TOL
+
+
+def test_large_value_scales_stay_in_range(device):
+    """Value scales up to ~20,000: probabilities may not pass 1 before they are scaled in fp16."""
+    got, ref = run(device, [90], [200], "int8", value_scale=6e5)
+    assert torch.isfinite(got.float()).all()
+    assert rel_err(got, ref) < TOL
+
+
+def test_scores_that_keep_growing_move_the_maximum(device):
+    """Keys ordered so that the row maximum grows by far more than the lazy limit, every step."""
+    n, bs, hkv = 300, 16, 8
+    g = torch.Generator().manual_seed(31)
+    direction = torch.randn(128, generator=g)
+    growth = torch.linspace(0.0, 40.0, 19 * bs + 1)
+    for kv in ("bf16", "int8"):
+        kc, vc, ks, vs = make_pool(19, bs, hkv, kv, torch.bfloat16, seed=32)
+        steep = (growth[:, None, None] * direction / direction.norm() * 4.0).expand(-1, hkv, -1).to(torch.bfloat16)
+        if kv == "bf16":
+            kc = steep.contiguous()
+        else:
+            from oracle.quant import quantize_vectors
+            kc, ks = quantize_vectors(steep)
+            ks = ks.reshape(-1, hkv)
+        q = (direction + 0.1 * torch.randn(n, 16, 128, generator=g)).to(torch.bfloat16)
+        tables = torch.arange(19, dtype=torch.int32)[None]
+        one = lambda v: torch.tensor([v], dtype=torch.int32)
+        args = (tables, bs, one(n), one(0), one(n))
+        # scores reach ~160: keys dequantised to bf16 (2^-9 each) would move them by ~0.02, the
+        # probabilities by 2e-2; so the oracle dequantises in fp32 here
+        ref = paged_attention_reference(q, kc, vc, ks, vs, *args, model_dtype=torch.float32)
+        d = lambda t: t.to(device) if torch.is_tensor(t) else t
+        got = kernels.paged_verify_attention(*map(d, (q, kc, vc, ks, vs) + args), max_q_len=n, max_ctx_len=n)
+        torch.cuda.synchronize()
+        assert torch.isfinite(got.float()).all()
+        assert rel_err(got, ref) < TOL
+
+
+def test_context_past_the_bound_is_flagged(device):
+    ws = kernels.AttentionWorkspace()
+    kc, vc, ks, vs = make_pool(64, 16, 8, "int8")
+    tables, ctx, qs, ql, rows = make_batch([500, 60], [40, 40], 64, 16)
+    q = torch.randn(rows, 16, 128).to(torch.bfloat16)
+    d = lambda t: t.to(device)
+    args = [d(t) for t in (q, kc, vc, ks, vs, tables)] + [16] + [d(t) for t in (ctx, qs, ql)]
+    kernels.paged_verify_attention(*args, max_q_len=40, max_ctx_len=500, workspace=ws)
+    assert ws.error_flag() == 0
+    kernels.paged_verify_attention(*args, max_q_len=40, max_ctx_len=400, workspace=ws)
+    assert ws.error_flag() != 0
+
+
+def test_workspace_holds_partials_only_where_the_keys_are_split(device):
+    size = _native.load().ne_paged_attention_workspace_size
+    assert size(1, 16, 8, 8192, 16384, 0) == 256  # 512 tiles: no split
+    # 8 work-groups of 64 rows, 32 splits: 130 floats per row
+    assert size(1, 16, 8, 20, 8192, 0) >= 8 * 32 * 64 * 130 * 4
