@@ -19,6 +19,8 @@
 // work-group's chain (first weight fetch from HBM, then per stage a barrier, the copy
 // issue, the fragment reads and the MFMAs, then the k-group exchange), not L2 -> CU
 // bandwidth (~30 TB/s with enough loads in flight), HBM or the MFMAs.
+#include <type_traits>
+
 #include "ne_common.hpp"
 #include "qk_rope_kv.hpp"
 
@@ -36,6 +38,7 @@ struct GemmParams {
   int64_t ldy;
   uint64_t* argmax;  // [m][n / BN] packed (ordered value, ~index)
   int tiles_m, tiles_n;
+  int scale_dtype;   // of the projections' row scales
 };
 
 __device__ __forceinline__ float sbyte(uint32_t w, int k) { return (float)(int8_t)(w >> (8 * k)); }
@@ -69,6 +72,20 @@ __device__ __forceinline__ float scale_at(const void* s, int64_t i) {
   } else {
     return load_scale<SDT>(s, i);
   }
+}
+
+// bf16(silu(gate)) * up of four paired outputs, each rounded to bf16 first
+__device__ __forceinline__ u32x2 swiglu4(const floatx4& gate4, const floatx4& up4, const float (&gs)[4],
+                                         const float (&us)[4]) {
+  float out[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float gate = bf16_round(gate4[i] * gs[i]);
+    const float up = bf16_round(up4[i] * us[i]);
+    const float silu = bf16_round(gate / (1.f + __expf(-gate)));
+    out[i] = silu * up;
+  }
+  return u32x2{pack_bf16x2(out[0], out[1]), pack_bf16x2(out[2], out[3])};
 }
 
 // ---- shared pieces -------------------------------------------------------------
@@ -549,16 +566,9 @@ __global__ __launch_bounds__((ProjLayout<NSUB, PM, KG, NPW>::kThreads)) void pro
       }
     } else if constexpr (EPI == 1) {
       static_assert(NPW == 2, "a wave holds paired gate / up subtiles");
-      float out[4];  // gate rows are subtile 2 nw, the paired up rows subtile 2 nw + 1
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float gate = bf16_round(v[0][i] * sc[0][i]);
-        const float up = bf16_round(v[1][i] * sc[1][i]);
-        const float silu = bf16_round(gate / (1.f + __expf(-gate)));
-        out[i] = silu * up;
-      }
+      // gate rows are subtile 2 nw, the paired up rows subtile 2 nw + 1
       const int ncol = (n0 + 2 * nw * 16) / 2 + 4 * g;
-      const u32x2 bits = {pack_bf16x2(out[0], out[1]), pack_bf16x2(out[2], out[3])};
+      const u32x2 bits = swiglu4(v[0], v[1], sc[0], sc[1]);
       *(u32x2*)(p.y + (int64_t)m * p.ldy + ncol) = bits;
     } else {
 #pragma unroll
@@ -623,6 +633,547 @@ int launch_proj(GemmParams p, int splits, float* partial, hipStream_t stream, co
   return launch_proj_kt<NSUB, SDT, EPI, KV, PM, KG, NPW, 0>(p, splits, partial, stream, name, qa);
 }
 
+// ---- W8A16 projections over many rows (prefill) ---------------------------------------
+// The kernel above is built for a verify step: every wave takes all rows of a tile, 80 at
+// most.  Over thousands of rows its 80 x 64 tiles read each X row 64 times and each weight
+// 52-100 times, and a wave reads 1.2 LDS fragments per MFMA.  Here a work-group of 8 waves
+// owns 256 x 256, 128 x 256 or 128 x 128 outputs and a wave 128 x 64 or 64 x 64 of them:
+// 0.38 or 0.5 fragments per MFMA.
+//   waves = KG k-groups x MW row groups x NW column groups.  The 128 x 128 tile has two
+//           k-groups (each takes half of every stage's k, the halves of the sum meet in LDS
+//           at the end), the others one.
+//   ring  = three stages of KG blocks of 64 k, copied by DMA: X rows of 128 B and int8
+//           weight rows of 64 B, chunk-swizzled so that the fragment reads are free of bank
+//           conflicts.  Every wave issues the same number of copies per stage, so one vmcnt
+//           wait covers the stage.
+//   loop  = a wave holds the fragments of the next k-step while the MFMAs of the current
+//           one run; the barrier that admits stage t + 1 sits before the last MFMAs of stage
+//           t, so its wait and the first reads of t + 1 hide under them.
+//   k order: in k-step q of a block, lane group g holds logical k = 16 g + 8 q + e, so one
+//           16-byte weight read feeds both k-steps.
+// Measured (four weights in turn from a HIP graph; us, before -> here): 8,192 rows QKV
+// N = 4,096 154 -> 72, gate|up N = 6,144 183 -> 104 (990 TFLOP/s), o K = 2,048 83 -> 39,
+// down K = 3,072 119 -> 54; 4,096 rows 83 -> 39, 102 -> 62, 49 -> 25, 68 -> 34; the QKV
+// product with its epilogue, in the layer, 195 -> 100 and 110 -> 56.  A 256 x 256
+// tile's 64 k take ~2.3 us for 2,048 cycles of MFMAs per SIMD: the int8 conversions (48 VALU
+// per 32 MFMAs, both waves of a SIMD at once) and the LDS (208 KB per block at 128 B per
+// clock) share that time with them.
+template <int BM_, int BN_, int MW_, int NW_, int KG_>
+struct TileLayout {
+  static constexpr int BM = BM_, BN = BN_, MW = MW_, NW = NW_, KG = KG_;
+  static constexpr int kWaves = 8;
+  static_assert(MW * NW * KG == kWaves && (KG == 1 || KG == 2), "waves");
+  static constexpr int PM = BM / MW / 16;   // token subtiles per wave
+  static constexpr int NPW = BN / NW / 16;  // weight subtiles per wave
+  static constexpr int kXBlock = BM * 128, kWBlock = BN * 64;
+  static constexpr int kBlock = kXBlock + kWBlock;  // 64 k of X and W
+  static constexpr int kStage = KG * kBlock;
+  static constexpr int kStageK = 64 * KG;
+  static constexpr int kRing = 3;
+  static constexpr int kPerBlock = kBlock / 1024 / kWaves;  // copies per wave and block
+  static constexpr int kXPerBlock = kXBlock / 1024 / kWaves;
+  static constexpr int kCopies = KG * kPerBlock;  // copies per wave and stage
+  static constexpr int kRed = KG > 1 ? kWaves * (PM / 2) * NPW * 1024 : 0;
+  static constexpr int kRowB = BN * 2 + 16;       // bytes per row of the staged bf16 tile (QKV epilogue)
+  static constexpr int kLds = kRing * kStage;
+  static_assert(kBlock % (1024 * kWaves) == 0 && kXBlock % (1024 * kWaves) == 0, "copies split evenly over the waves");
+  static_assert(kRed <= kLds && BM * kRowB <= kLds && kLds <= 160 * 1024, "LDS");
+};
+
+template <typename L>
+struct TileWave {
+  uint32_t off[L::kCopies];  // lane offsets of this wave's copies
+  uint32_t xr, wr;           // fragment read positions within a block (k-step 0, subtile 0)
+  int wave, mw, nw, kg;
+};
+
+template <typename L>
+__device__ __forceinline__ void tile_mainloop(const GemmParams& p, char* smem, int n0, const TileWave<L>& w,
+                                              floatx4 (&acc)[L::PM][L::NPW]) {
+  constexpr int PM = L::PM, NPW = L::NPW, D = L::kCopies;
+  const int n_stages = p.k / L::kStageK;
+  const char* xbase = (const char*)p.x;
+  const char* wbase = (const char*)p.w + (int64_t)n0 * p.k;
+  // copy j of this wave is KiB 8 j + wave of the stage; a block is X rows, then weight rows
+  auto issue = [&](int t) {
+    char* slot = smem + (t % L::kRing) * L::kStage;
+    const char* xs = uniform_ptr(xbase + (int64_t)t * (L::kStageK * 2));
+    const char* ws = uniform_ptr(wbase + (int64_t)t * L::kStageK);
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      uint32_t o = w.off[j];
+      __asm__("" : "+v"(o));  // keep the lane offset 32-bit: scalar base + offset addressing
+      lds_dma16((j % L::kPerBlock < L::kXPerBlock ? xs : ws) + o, slot + (j * L::kWaves + w.wave) * 1024);
+    }
+  };
+  using XFrag = u32x4[PM];
+  using AFrag = bf16x8[NPW];
+  auto block_at = [&](int t) { return smem + (t % L::kRing) * L::kStage + w.kg * L::kBlock; };
+  // X chunk 2 g + q of a 128-byte row sits at position chunk ^ (row % 8): k-step q flips bit 4
+  auto read_x = [&](int t, int q, XFrag& xf) {
+    const char* xs = block_at(t) + (w.xr ^ (uint32_t)(q * 16));
+#pragma unroll
+    for (int mi = 0; mi < PM; ++mi) xf[mi] = *(const u32x4*)(xs + mi * 16 * 128);
+  };
+  u32x4 wf[NPW];  // both k-steps of a block
+  auto read_w = [&](int t) {
+    const char* ws = block_at(t) + w.wr;
+#pragma unroll
+    for (int ns = 0; ns < NPW; ++ns) wf[ns] = *(const u32x4*)(ws + ns * 16 * 64);
+  };
+  auto convert = [&](int q, AFrag& a) {
+#pragma unroll
+    for (int ns = 0; ns < NPW; ++ns) a[ns] = int8x8_to_bf16x8(wf[ns][2 * q], wf[ns][2 * q + 1]);
+  };
+  auto mma = [&](const XFrag& xf, const AFrag& a) {
+#pragma unroll
+    for (int mi = 0; mi < PM; ++mi)
+#pragma unroll
+      for (int ns = 0; ns < NPW; ++ns)
+        acc[mi][ns] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ns], __builtin_bit_cast(bf16x8, xf[mi]), acc[mi][ns],
+                                                              0, 0, 0);
+  };
+
+#pragma unroll
+  for (int s = 0; s < L::kRing; ++s)
+    if (s < n_stages) issue(s);
+  wait_pending<D, L::kRing - 1>(min(n_stages, L::kRing) - 1);  // stage 0 has landed
+  asm volatile("s_barrier" ::: "memory");
+
+  XFrag x0, x1;
+  AFrag a0, a1;
+  read_w(0);
+  read_x(0, 0, x0);
+  for (int t = 0; t + 1 < n_stages; ++t) {
+    read_x(t, 1, x1);
+    __builtin_amdgcn_sched_barrier(0);  // the reads go out before the multiplies
+    convert(0, a0);
+    mma(x0, a0);
+    convert(1, a1);
+    __builtin_amdgcn_sched_barrier(0);
+    // stage t + 1 has landed and every wave has read stage t: its slot takes stage t + 3
+    if (t + 2 < n_stages) {
+      wait_vmcnt<D>();
+    } else {
+      wait_vmcnt<0>();
+    }
+    wait_lgkmcnt0();
+    asm volatile("s_barrier" ::: "memory");
+    if (t + L::kRing < n_stages) issue(t + L::kRing);
+    read_w(t + 1);
+    read_x(t + 1, 0, x0);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(x1, a1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  read_x(n_stages - 1, 1, x1);
+  convert(0, a0);
+  mma(x0, a0);
+  convert(1, a1);
+  mma(x1, a1);
+}
+
+// the weight rows' scales first + 16 ns + i in the caller's dtype (one uniform branch)
+template <int NPW>
+__device__ __forceinline__ void tile_scales(const GemmParams& p, int first, float (&sc)[NPW][4]) {
+  auto load = [&](auto dtype) {
+#pragma unroll
+    for (int ns = 0; ns < NPW; ++ns)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sc[ns][i] = load_scale<decltype(dtype)::value>(p.scale, first + ns * 16 + i);
+  };
+  if (p.scale_dtype == NE_DTYPE_BF16) {
+    load(std::integral_constant<int, NE_DTYPE_BF16>{});
+  } else if (p.scale_dtype == NE_DTYPE_FP16) {
+    load(std::integral_constant<int, NE_DTYPE_FP16>{});
+  } else {
+    load(std::integral_constant<int, NE_DTYPE_FP32>{});
+  }
+}
+
+// Sum / maximum over the 16 lanes of a DPP row, every lane ending with the result.  With
+// a lane holding the sum of four consecutive leaves, the additions pair up exactly as
+// wave_reduce_n pairs 64 lanes of one leaf each.
+template <bool MAX, int N>
+__device__ __forceinline__ void row16_reduce(float (&v)[N]) {
+  auto op = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = op(v[i], dpp_f32<0xB1>(v[i]));  // quad_perm [1, 0, 3, 2]
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = op(v[i], dpp_f32<0x4E>(v[i]));  // quad_perm [2, 3, 0, 1]
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = op(v[i], dpp_f32<0x141>(v[i]));  // row_half_mirror
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = op(v[i], dpp_f32<0x140>(v[i]));  // row_mirror
+}
+
+__device__ __forceinline__ void unpack4(const u32x2 v, float (&f)[4]) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    f[2 * i] = __uint_as_float(v[i] << 16);
+    f[2 * i + 1] = __uint_as_float(v[i] & 0xFFFF0000u);
+  }
+}
+
+// four values rounded to bf16
+__device__ __forceinline__ u32x2 pack4(const float (&f)[4]) {
+  return u32x2{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3])};
+}
+
+__device__ __forceinline__ void round4(float (&f)[4]) { unpack4(pack4(f), f); }
+
+// four int8 codes of quotients: rounded to even, clamped to +-127
+__device__ __forceinline__ uint32_t codes4(const float (&t)[4]) {
+  uint32_t b[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) b[e] = (uint32_t)(int)fminf(fmaxf(rintf(t[e]), -127.f), 127.f);
+  const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u);
+  return __builtin_amdgcn_perm(__builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u), lo, 0x05040100u);
+}
+
+// QK-norm + RoPE + KV write of the tile's head vectors, staged as bf16 in LDS (the bits the
+// plain epilogue stores): the arithmetic of qk_norm_rope_kv_vectors on 16 lanes per vector,
+// lane c with elements 4 c .. + 4 and 64 + 4 c .. + 4, so that a wave takes four vectors at
+// once, RoPE pairs meet in a lane and stores are 4 or 8 bytes wide.
+template <typename L, int KV>
+__device__ __forceinline__ void tile_qkv_epilogue(const QkvRopeArgs& qa, const char* smem, int m, int m0, int n0,
+                                                  int wave, int lane) {
+  constexpr bool kInt8 = KV >= 2;
+  constexpr int kSdt = KV == 3 ? NE_DTYPE_FP16 : NE_DTYPE_BF16;
+  constexpr int kHeads = L::BN / 128;
+  constexpr int kHeadWaves = L::kWaves / kHeads;   // waves per head of the tile
+  constexpr int kWaveRows = L::BM / kHeadWaves;    // rows per wave
+  constexpr int kSteps = kWaveRows / 4;            // four rows at a time
+  constexpr int kBatch = 4;                        // steps whose RoPE loads are in flight together
+  static_assert(kSteps % kBatch == 0, "whole batches");
+  const int hl = wave / kHeadWaves;
+  const int h = n0 / 128 + hl;
+  const int c = lane & 15;
+  const bool is_q = h < qa.hq;
+  const bool is_v = h >= qa.hq + qa.hkv;
+  const int kh = is_v ? h - qa.hq - qa.hkv : h - qa.hq;
+  void* cache = is_v ? qa.v_cache : qa.k_cache;
+  const int wrow0 = (wave % kHeadWaves) * kWaveRows + (lane >> 4);
+  // slots and positions of all the wave's rows, then the RoPE values one batch ahead
+  int slot[kSteps], pos[kSteps];
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i) {
+    const int row = min(m0 + wrow0 + 4 * i, m - 1);
+    slot[i] = is_q ? 0 : qa.slot_mapping[row];
+    pos[i] = is_v ? 0 : qa.positions[row];
+  }
+  float wa[4], wb[4];
+  {
+    const uint16_t* w = is_q ? qa.q_norm_w : qa.k_norm_w;  // v heads do not use it
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      wa[i] = bf16_to_f32(w[4 * c + i]);
+      wb[i] = bf16_to_f32(w[64 + 4 * c + i]);
+    }
+  }
+  u32x2 rope[2][kBatch][2];
+  auto load_rope = [&](int b, u32x2 (&dst)[kBatch][2]) {
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const int64_t at = min(max(pos[b * kBatch + i], 0), qa.rope_positions - 1);
+      dst[i][0] = *(const u32x2*)(qa.rope + at * 128 + 4 * c);
+      dst[i][1] = *(const u32x2*)(qa.rope + at * 128 + 64 + 4 * c);
+    }
+  };
+  load_rope(0, rope[0]);
+  lds_barrier();  // the staged tile is complete
+#pragma unroll
+  for (int b = 0; b < kSteps / kBatch; ++b) {
+    const int lrow0 = wrow0 + b * 4 * kBatch;
+    if (m0 + lrow0 - (lane >> 4) >= m) return;  // wave-uniform: no rows left
+    if (b + 1 < kSteps / kBatch) load_rope(b + 1, rope[(b + 1) & 1]);
+    // the batch's vectors stage by stage, so that the steps' chains overlap
+    float x[kBatch][4], y[kBatch][4];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const char* src = smem + (lrow0 + 4 * i) * L::kRowB + hl * 256 + 8 * c;
+      unpack4(*(const u32x2*)src, x[i]);
+      unpack4(*(const u32x2*)(src + 128), y[i]);
+    }
+    if (!is_v) {
+      float ss[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        float leaf[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) leaf[e] = x[i][e] * x[i][e] + y[i][e] * y[i][e];
+        ss[i] = (leaf[0] + leaf[1]) + (leaf[2] + leaf[3]);
+      }
+      row16_reduce<false, kBatch>(ss);
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const float inv = rsqrtf(ss[i] / 128.f + qa.eps);
+        float cs[4], sn[4], xc[4], xs[4], yc[4], ys[4];
+        unpack4(rope[b & 1][i][0], cs);
+        unpack4(rope[b & 1][i][1], sn);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[i][e] *= inv;
+          y[i][e] *= inv;
+        }
+        round4(x[i]);
+        round4(y[i]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[i][e] *= wa[e];
+          y[i][e] *= wb[e];
+        }
+        round4(x[i]);
+        round4(y[i]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          xc[e] = x[i][e] * cs[e];
+          xs[e] = x[i][e] * sn[e];
+          yc[e] = y[i][e] * cs[e];
+          ys[e] = -y[i][e] * sn[e];
+        }
+        round4(xc);
+        round4(xs);
+        round4(yc);
+        round4(ys);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[i][e] = xc[e] + ys[e];
+          y[i][e] = yc[e] + xs[e];
+        }
+      }
+    }
+    if (is_q || !kInt8) {
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const int row = m0 + lrow0 + 4 * i;
+        uint16_t* dst = (is_q ? qa.q_out + ((int64_t)row * qa.hq + h) * 128
+                              : (uint16_t*)cache + ((int64_t)slot[b * kBatch + i] * qa.hkv + kh) * 128) + 4 * c;
+        if (row < m) {
+          *(u32x2*)dst = pack4(x[i]);
+          *(u32x2*)(dst + 64) = pack4(y[i]);
+        }
+      }
+    } else {
+      // write_vectors' quantisation: the quotient by the reciprocal (within 3e-5 of the exact
+      // one), exact divisions where a lane of the batch is near a rounding tie
+      float s[kBatch], tx[kBatch][4], ty[kBatch][4];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        round4(x[i]);
+        round4(y[i]);
+        s[i] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[i] = fmaxf(s[i], fmaxf(fabsf(x[i][e]), fabsf(y[i][e])));
+      }
+      row16_reduce<true, kBatch>(s);
+      float dist = 0.f;  // the farthest of this lane's quotients from a whole number
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        s[i] = fmaxf(s[i], 1e-8f) / 127.f;
+        const float rcp = __builtin_amdgcn_rcpf(s[i]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          tx[i][e] = x[i][e] * rcp;
+          ty[i][e] = y[i][e] * rcp;
+          dist = fmaxf(dist, fmaxf(fabsf(tx[i][e] - rintf(tx[i][e])), fabsf(ty[i][e] - rintf(ty[i][e]))));
+        }
+      }
+      if (__builtin_amdgcn_ballot_w64(dist > 0.49996f) != 0) {
+#pragma unroll
+        for (int i = 0; i < kBatch; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            tx[i][e] = x[i][e] / s[i];
+            ty[i][e] = y[i][e] / s[i];
+          }
+      }
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const uint32_t px = codes4(tx[i]), py = codes4(ty[i]);
+        const int64_t vec = (int64_t)slot[b * kBatch + i] * qa.hkv + kh;
+        if (m0 + lrow0 + 4 * i < m) {
+          int8_t* dst = (int8_t*)cache + vec * 128 + 4 * c;
+          *(uint32_t*)dst = px;
+          *(uint32_t*)(dst + 64) = py;
+          if (c == 0) store_scale<kSdt>(is_v ? qa.v_scale : qa.k_scale, vec, s[i]);
+        }
+      }
+    }
+  }
+}
+
+// EPI and KV as proj_kernel's (0: store, 1: SwiGLU, 4: QK-norm + RoPE + KV write).
+template <typename L, int EPI, int KV>
+__global__ __launch_bounds__(L::kWaves* kWave) void proj_tile_kernel(GemmParams p, QkvRopeArgs qa) {
+  constexpr int PM = L::PM, NPW = L::NPW;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  asm volatile("" ::"s"(p.x), "s"(p.ldx), "s"(p.w), "s"(p.scale), "s"(p.m), "s"(p.k), "s"(p.tiles_m),
+               "s"(p.tiles_n), "s"(p.y), "s"(p.ldy));
+  // Each XCD takes a contiguous eighth of the tiles, in an order that walks all weight
+  // tiles against groups of four row tiles: the group's X rows stay in that XCD's L2.
+  const int total = p.tiles_m * p.tiles_n;
+  const int per = (total + kNumXcd - 1) / kNumXcd;
+  const int idx = (blockIdx.x % kNumXcd) * per + blockIdx.x / kNumXcd;
+  if (idx >= total) return;
+  constexpr int kGroup = 4;
+  const int grp = idx / (kGroup * p.tiles_n);
+  const int in_grp = idx - grp * (kGroup * p.tiles_n);
+  const int rows_in = min(kGroup, p.tiles_m - grp * kGroup);
+  const int tn = in_grp / rows_in;
+  const int m0 = (grp * kGroup + in_grp - tn * rows_in) * L::BM;
+  const int n0 = tn * L::BN;
+  const int lane = threadIdx.x % kWave;
+  const int r = lane & 15;
+  const int g = lane >> 4;
+  TileWave<L> w;
+  w.wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  w.kg = w.wave / (L::MW * L::NW);
+  w.mw = (w.wave / L::NW) % L::MW;
+  w.nw = w.wave % L::NW;
+#pragma unroll
+  for (int j = 0; j < L::kCopies; ++j) {
+    const int block = j / L::kPerBlock;
+    const int i = (j % L::kPerBlock) * L::kWaves + w.wave;  // KiB of the block
+    if (j % L::kPerBlock < L::kXPerBlock) {                 // 8 X rows x 8 chunks of 16 B
+      const int row = i * 8 + (lane >> 3);
+      const int chunk = (lane & 7) ^ (row & 7);
+      // rows past m re-read row m - 1 and are never stored
+      w.off[j] = (uint32_t)min(m0 + row, p.m - 1) * (uint32_t)(p.ldx * 2) + (uint32_t)(block * 128 + chunk * 16);
+    } else {  // 16 weight rows x 4 chunks
+      const int row = (i - L::kXBlock / 1024) * 16 + (lane >> 2);
+      const int chunk = (lane & 3) ^ ((row >> 1) & 3);
+      w.off[j] = (uint32_t)row * (uint32_t)p.k + (uint32_t)(block * 64 + chunk * 16);
+    }
+  }
+  w.xr = (uint32_t)((w.mw * PM * 16 + r) * 128 + (((2 * g) ^ (r & 7)) * 16));
+  w.wr = (uint32_t)(L::kXBlock + (w.nw * NPW * 16 + r) * 64 + ((g ^ ((r >> 1) & 3)) * 16));
+
+  floatx4 acc[PM][NPW];
+#pragma unroll
+  for (int mi = 0; mi < PM; ++mi)
+#pragma unroll
+    for (int ns = 0; ns < NPW; ++ns) acc[mi][ns] = floatx4{0.f, 0.f, 0.f, 0.f};
+  tile_mainloop<L>(p, smem, n0, w, acc);
+
+  // the weight rows' scales: lane (r, g) stores columns 16 ns + 4 g + i of its subtiles
+  float sc[NPW][4];
+  tile_scales<NPW>(p, n0 + w.nw * NPW * 16 + 4 * g, sc);
+
+  // two k-groups: group kg finishes token subtiles [kg PM / 2, + PM / 2), summed kg 0 + kg 1
+  constexpr int kMine = L::KG > 1 ? PM / 2 : PM;
+  if constexpr (L::KG > 1) {
+    floatx4* red = (floatx4*)smem;
+    auto at = [&](int from, int mi, int ns) -> floatx4& {
+      return red[(((from * L::MW * L::NW + w.wave % (L::MW * L::NW)) * kMine + mi) * NPW + ns) * kWave + lane];
+    };
+    lds_barrier();  // every wave is past its last fragment read
+#pragma unroll
+    for (int mi = 0; mi < kMine; ++mi)
+#pragma unroll
+      for (int ns = 0; ns < NPW; ++ns) at(w.kg, mi, ns) = w.kg == 0 ? acc[kMine + mi][ns] : acc[mi][ns];
+    lds_barrier();
+#pragma unroll
+    for (int mi = 0; mi < kMine; ++mi)
+#pragma unroll
+      for (int ns = 0; ns < NPW; ++ns) {
+        const floatx4 other = at(1 - w.kg, mi, ns);
+        acc[mi][ns] = w.kg == 0 ? acc[mi][ns] + other : other + acc[kMine + mi][ns];
+      }
+  }
+  const int lrow0 = (w.mw * PM + (L::KG > 1 ? w.kg * kMine : 0)) * 16 + r;  // first of this lane's tile rows
+  if constexpr (EPI == 4) {
+    lds_barrier();  // every wave is past its last read of the ring, or of the partial sums
+#pragma unroll
+    for (int mi = 0; mi < kMine; ++mi)
+#pragma unroll
+      for (int ns = 0; ns < NPW; ++ns) {
+        const floatx4 v = acc[mi][ns];
+        *(u32x2*)(smem + (lrow0 + mi * 16) * L::kRowB + ((w.nw * NPW + ns) * 16 + 4 * g) * 2) =
+            u32x2{pack_bf16x2(v[0] * sc[ns][0], v[1] * sc[ns][1]), pack_bf16x2(v[2] * sc[ns][2], v[3] * sc[ns][3])};
+      }
+    tile_qkv_epilogue<L, KV>(qa, smem, p.m, m0, n0, w.wave, lane);
+    return;
+  }
+#pragma unroll
+  for (int mi = 0; mi < kMine; ++mi) {
+    const int m = m0 + lrow0 + mi * 16;
+    if (m >= p.m) continue;
+    if constexpr (EPI == 0) {
+#pragma unroll
+      for (int ns = 0; ns < NPW; ++ns) {
+        const int n = n0 + (w.nw * NPW + ns) * 16 + 4 * g;
+        const floatx4 v = acc[mi][ns];
+        *(u32x2*)(p.y + (int64_t)m * p.ldy + n) =
+            u32x2{pack_bf16x2(v[0] * sc[ns][0], v[1] * sc[ns][1]), pack_bf16x2(v[2] * sc[ns][2], v[3] * sc[ns][3])};
+      }
+    } else if constexpr (EPI == 1) {
+      static_assert(NPW % 2 == 0, "a wave holds paired gate / up subtiles");
+#pragma unroll
+      for (int ns = 0; ns < NPW; ns += 2) {
+        const u32x2 bits = swiglu4(acc[mi][ns], acc[mi][ns + 1], sc[ns], sc[ns + 1]);
+        *(u32x2*)(p.y + (int64_t)m * p.ldy + (n0 + (w.nw * NPW + ns) * 16) / 2 + 4 * g) = bits;
+      }
+    }
+  }
+}
+
+template <typename L, int EPI, int KV>
+int launch_proj_tile_as(GemmParams p, hipStream_t stream, const char* name, const QkvRopeArgs& qa) {
+  p.tiles_m = ceil_div(p.m, L::BM);
+  p.tiles_n = p.n / L::BN;
+  const int per = ceil_div((int64_t)p.tiles_m * p.tiles_n, kNumXcd);
+  static const hipError_t attr = hipFuncSetAttribute((const void*)proj_tile_kernel<L, EPI, KV>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, L::kLds);
+  if (attr != hipSuccess) {
+    set_error("%s: cannot reserve %d bytes of LDS: %s", name, L::kLds, hipGetErrorString(attr));
+    return NE_ELAUNCH;
+  }
+  hipLaunchKernelGGL((proj_tile_kernel<L, EPI, KV>), dim3((unsigned)(per * kNumXcd)), dim3(L::kWaves * kWave),
+                     L::kLds, stream, p, qa);
+  return check_launch(name);
+}
+
+using Tile256x256 = TileLayout<256, 256, 2, 4, 1>;
+using Tile128x256 = TileLayout<128, 256, 2, 4, 1>;
+using Tile128x128 = TileLayout<128, 128, 2, 2, 2>;
+
+enum class ProjTile { kVerify, k128x128, k128x256, k256x256 };
+
+// The kernel of a product without split-K: the least rounds of one tile per CU times what a
+// round costs per 64 k.  Costs in us, measured at N = 1,024-6,144, K = 1,024-3,072 and 320-
+// 8,192 rows: 2.3 (256 x 256), 1.32 (128 x 256), 0.8 (128 x 128) and, for the verify step's
+// kernel, 0.39 (80 x 64) or 0.45 (SwiGLU's 80 x 96) with rounds that overlap.  At 512 rows
+// of N = 4,096 that kernel takes 12.6 us and 128 x 128 tiles 14.0, at 1,024 rows 22.9 and
+// 15.7; 2,048 rows of o 24.3 and 23.3, 4,096 rows 49 and 25.  The fused QKV product follows
+// the plain product's choice, so that both sum in one order and round to the same bits.
+ProjTile choose_proj_tile(int m, int n, bool swiglu) {
+  const auto rounds = [&](int bm, int bn) {
+    return (int64_t)ceil_div((int64_t)ceil_div(m, bm) * (n / bn), kNumCu);
+  };
+  const int verify_n = swiglu && n % 96 == 0 ? 96 : 64;
+  const double verify_tiles = (double)ceil_div(m, kPM * 16) * (n / verify_n) / kNumCu;
+  double best = (verify_tiles > 1.0 ? verify_tiles : 1.0) * (verify_n == 96 ? 0.45 : 0.39);
+  ProjTile tile = ProjTile::kVerify;
+  const auto offer = [&](ProjTile t, int bm, int bn, double cost) {
+    if (n % bn != 0 || rounds(bm, bn) * cost >= best) return;
+    best = rounds(bm, bn) * cost;
+    tile = t;
+  };
+  offer(ProjTile::k128x128, 128, 128, 0.8);
+  offer(ProjTile::k128x256, 128, 256, 1.32);
+  offer(ProjTile::k256x256, 256, 256, 2.3);
+  return tile;
+}
+
+template <int EPI, int KV>
+int launch_proj_tile(ProjTile tile, const GemmParams& p, hipStream_t s, const char* name,
+                     const QkvRopeArgs& qa = QkvRopeArgs{}) {
+  if (tile == ProjTile::k256x256) return launch_proj_tile_as<Tile256x256, EPI, KV>(p, s, name, qa);
+  if (tile == ProjTile::k128x256) return launch_proj_tile_as<Tile128x256, EPI, KV>(p, s, name, qa);
+  return launch_proj_tile_as<Tile128x128, EPI, KV>(p, s, name, qa);
+}
+
 // Wave layouts (k-groups, weight subtiles per wave).  The plain and split-K products and
 // the fused QKV projection share two k-groups, so the fused epilogue sums every output in
 // the order the plain GEMM does and both round to the same bits; SwiGLU pairs gate and
@@ -633,6 +1184,14 @@ constexpr int kKgSwiglu = 4, kNpwSwiglu = 2;
 
 template <int SDT>
 int dispatch_qkv_fused(GemmParams p, const QkvRopeArgs& qa, int kv_mode, hipStream_t s) {
+  // the tiles' epilogue stores 4 or 8 bytes at a time where the row kernel's stores elements
+  const bool aligned = (((uintptr_t)qa.q_out | (uintptr_t)qa.rope | (uintptr_t)qa.k_cache | (uintptr_t)qa.v_cache) % 8) == 0;
+  const ProjTile tile = aligned ? choose_proj_tile(p.m, p.n, false) : ProjTile::kVerify;
+  if (tile != ProjTile::kVerify) {
+    if (kv_mode == 1) return launch_proj_tile<4, 1>(tile, p, s, "w8a16_qkv_norm_rope_kv", qa);
+    if (kv_mode == 2) return launch_proj_tile<4, 2>(tile, p, s, "w8a16_qkv_norm_rope_kv", qa);
+    return launch_proj_tile<4, 3>(tile, p, s, "w8a16_qkv_norm_rope_kv", qa);
+  }
   switch (kv_mode) {
     // 48-row tiles: 7 x 32 = 224 work-groups for 320 rows, 3 rows per wave in the epilogue
     case 1: return launch_proj<8, SDT, 4, 1, 3, kKgQkv, kNpwQkv>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
@@ -643,6 +1202,12 @@ int dispatch_qkv_fused(GemmParams p, const QkvRopeArgs& qa, int kv_mode, hipStre
 
 template <int SDT>
 int dispatch_w8a16(GemmParams p, int epilogue, int splits, float* partial, hipStream_t s) {
+  if (partial == nullptr) {
+    const bool swiglu = epilogue == NE_EPILOGUE_SWIGLU;
+    const ProjTile tile = choose_proj_tile(p.m, p.n, swiglu);
+    if (tile != ProjTile::kVerify)
+      return swiglu ? launch_proj_tile<1, 0>(tile, p, s, "w8a16_swiglu") : launch_proj_tile<0, 0>(tile, p, s, "w8a16_gemm");
+  }
   if (epilogue == NE_EPILOGUE_SWIGLU) {
     if (p.n % 96 == 0)
       return launch_proj<6, SDT, 1, 0, kPM, kKgSwiglu, kNpwSwiglu>(p, 1, nullptr, s, "w8a16_swiglu");
@@ -1106,6 +1671,7 @@ int w8a16_common(const void* x, int64_t ldx, const int8_t* w, const void* scale,
   p.ldx = ldx;
   p.w = w;
   p.scale = scale;
+  p.scale_dtype = scale_dtype;
   p.m = m;
   p.n = n;
   p.k = k;
@@ -1197,6 +1763,7 @@ extern "C" int ne_w8a16_qkv_norm_rope_kv(
   p.ldx = ldx;
   p.w = w;
   p.scale = scale;
+  p.scale_dtype = scale_dtype;
   p.m = m;
   p.n = (num_q_heads + 2 * num_kv_heads) * 128;
   p.k = k;

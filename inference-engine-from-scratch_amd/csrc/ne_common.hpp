@@ -25,6 +25,7 @@ constexpr int kWave = 64;
 using ConstI32 = __attribute__((address_space(4))) const int32_t;
 
 constexpr int kNumXcd = 8;  // MI355X: 8 XCDs, work-groups dispatched round-robin
+constexpr int kNumCu = 256;
 
 // ---- error state (per calling thread) ------------------------------------
 void set_error(const char* fmt, ...);

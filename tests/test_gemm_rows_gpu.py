@@ -1,0 +1,118 @@
+"""A8 over many rows (prefill): the large-tile projection kernels against Int8Linear in fp32.
+
+Sizes reach each tile (128 x 128, 128 x 256, 256 x 256) with row counts one below, at and one
+past its edges.  Bars: 2.5e-3 relative for a plain product, whose only rounding beside fp32
+sums is the bf16 output (2^-9, 1.1e-3 rms); 5e-3 for SwiGLU, which rounds gate, up, silu and
+the product (four such, 2.3e-3).
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from helpers import rel_err
+from nanoengine_amd import kernels
+from nanoengine_amd._native import EPILOGUE_SWIGLU
+
+pytestmark = pytest.mark.gpu
+
+
+def weight(n, k, device, scale_dtype=torch.bfloat16, seed=0):
+    g = torch.Generator(device=device).manual_seed(seed + n + k)
+    codes = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=device, generator=g)
+    scales = torch.rand(n, device=device, generator=g) * 3e-4 + 1e-4
+    return codes, scales.to(scale_dtype)
+
+
+def product(x, w, s):
+    return (x.float() @ w.float().t()) * s.float()
+
+
+# N = 4,096 at 897-1,024 rows: 128 x 128; at 2,047-2,048: 128 x 256; at 3,841-4,096: 256 x 256
+@pytest.mark.parametrize("m,n,k", [
+    (897, 4096, 1024), (1024, 4096, 128), (1023, 4096, 256), (1000, 4096, 384), (2047, 4096, 1024), (2048, 4096, 128),
+    (2000, 4096, 384), (3841, 4096, 1024), (4096, 4096, 128), (4095, 4096, 256), (4097, 1024, 2048), (8191, 1024, 3072),
+])
+def test_product(device, m, n, k):
+    w, s = weight(n, k, device)
+    x = torch.randn(m, k, device=device, generator=torch.Generator(device=device).manual_seed(m)).to(torch.bfloat16)
+    out = kernels.w8a16_gemm(x, w, s)
+    assert rel_err(out, product(x, w, s)) < 2.5e-3
+
+
+@pytest.mark.parametrize("scale_dtype", [torch.float16, torch.float32])
+def test_scale_types_and_strides(device, scale_dtype):
+    w, s = weight(4096, 512, device, scale_dtype)
+    wide = torch.randn(1001, 640, device=device).to(torch.bfloat16)
+    x = wide[:, 64:576]
+    out = torch.zeros(1002, 4096, dtype=torch.bfloat16, device=device)
+    kernels.w8a16_gemm(x, w, s, out=out[:1001])
+    assert rel_err(out[:1001], product(x, w, s)) < 2.5e-3
+    assert not out[1001].any()  # the row after the last
+
+
+@pytest.mark.parametrize("m", [1025, 1537, 2049])
+def test_swiglu(device, m):
+    gate, gs = weight(3072, 1024, device, seed=1)
+    up, us = weight(3072, 1024, device, seed=2)
+    pair = lambda a, b: torch.stack([a.view(-1, 16, *a.shape[1:]), b.view(-1, 16, *b.shape[1:])], 1).flatten(0, 2)
+    x = torch.randn(m, 1024, device=device).to(torch.bfloat16)
+    out = kernels.w8a16_gemm(x, pair(gate, up).contiguous(), pair(gs, us).contiguous(), epilogue=EPILOGUE_SWIGLU)
+    ref = torch.nn.functional.silu(product(x, gate, gs)) * product(x, up, us)
+    assert out.shape == (m, 3072) and rel_err(out, ref) < 5e-3
+
+
+@pytest.mark.parametrize("kv", ["int8-bf16-scales", "int8-fp16-scales", "bf16"])
+@pytest.mark.parametrize("m", [1000, 2047, 3900])
+def test_fused_qkv_equals_gemm_then_row_kernel(device, kv, m):
+    """The tiles' QK-norm + RoPE + KV-write epilogue gives the bits of the plain product
+    followed by the row kernel, rows past the last written nowhere."""
+    hq, hkv, k, slots_n = 16, 8, 1024, 5000
+    g = torch.Generator(device=device).manual_seed(m)
+    w, s = weight(4096, k, device)
+    x = torch.randn(m, k, device=device, generator=g).to(torch.bfloat16)
+    x[5] = 0  # a zero row: zero vectors, the smallest scale
+    q_norm, k_norm = ((1 + 0.1 * torch.randn(128, device=device, generator=g)).to(torch.bfloat16) for _ in range(2))
+    positions = torch.randint(0, 6000, (m,), generator=g, dtype=torch.int32, device=device)
+    rope = kernels.rope_table(6000, 1e6).to(device)
+    slots = torch.randperm(slots_n, generator=g, device=device)[:m].to(torch.int32)
+
+    def pool():
+        if kv == "bf16":
+            return [torch.zeros(slots_n, hkv, 128, dtype=torch.bfloat16, device=device) for _ in range(2)] + [None, None]
+        sdt = torch.bfloat16 if kv == "int8-bf16-scales" else torch.float16
+        return ([torch.zeros(slots_n, hkv, 128, dtype=torch.int8, device=device) for _ in range(2)]
+                + [torch.zeros(slots_n, hkv, dtype=sdt, device=device) for _ in range(2)])
+
+    a, b = pool(), pool()
+    q_ref = kernels.qk_norm_rope_kv_write(kernels.w8a16_gemm(x, w, s), hq, hkv, q_norm, k_norm, 1e-6, positions, rope,
+                                          slots, *a)
+    q_out = torch.zeros(m + 1, hq, 128, dtype=torch.bfloat16, device=device)
+    kernels.w8a16_qkv_norm_rope_kv(x, w, s, hq, hkv, q_norm, k_norm, 1e-6, positions, rope, slots, *b, q_out=q_out[:m])
+    assert torch.equal(q_out[:m].view(torch.int16), q_ref.view(torch.int16)) and not q_out[m].any()
+    for ta, tb in zip(a, b):
+        if ta is not None:
+            assert torch.equal(ta.view(torch.uint8), tb.view(torch.uint8))
+    assert int(a[0].view(torch.uint8).ne(0).sum()) > 0
+
+
+def test_unaligned_cache_takes_the_other_kernel(device):
+    """A pool that starts at an odd byte (the row kernel stores single codes) is still written."""
+    hq, hkv, k, m, n_slots = 16, 8, 256, 1000, 1100
+    w, s = weight(4096, k, device)
+    x = torch.randn(m, k, device=device).to(torch.bfloat16)
+    ones = torch.ones(128, dtype=torch.bfloat16, device=device)
+    pos = torch.arange(m, dtype=torch.int32, device=device)
+    rope = kernels.rope_table(1024, 1e6).to(device)
+    size = n_slots * hkv * 128
+    raw = [torch.zeros(size + 1, dtype=torch.int8, device=device) for _ in range(2)]
+    odd = [t[1:].view(n_slots, hkv, 128) for t in raw]
+    even = [torch.zeros(n_slots, hkv, 128, dtype=torch.int8, device=device) for _ in range(2)]
+    for caches in (odd, even):
+        scales = [torch.zeros(n_slots, hkv, dtype=torch.bfloat16, device=device) for _ in range(2)]
+        kernels.w8a16_qkv_norm_rope_kv(x, w, s, hq, hkv, ones, ones, 1e-6, pos, rope, pos, *caches, *scales,
+                                       q_out=torch.empty(m, hq, 128, dtype=torch.bfloat16, device=device))
+    # another summation order: a code may differ by the rounding of a tie
+    for o, e in zip(odd, even):
+        assert int((o.int() - e.int()).abs().max()) <= 2 and float((o != e).float().mean()) < 0.02
