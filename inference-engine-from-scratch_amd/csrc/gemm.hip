@@ -200,6 +200,16 @@ __device__ __forceinline__ void wait_pending(int pend) {
   }
 }
 
+// Two adjacent 16-column subtiles of a 16-row MFMA result, lane (r, g) with columns 4 g ..
+// + 4 of each as packed bf16 (a, b): regrouped so that the lane holds 8 consecutive columns
+// from column 16 (g % 2) + 8 (g / 2) of the pair, one 16-byte store instead of two of 8.
+__device__ __forceinline__ u32x4 pair_columns(const u32x2& a, const u32x2& b) {
+  const auto x = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto y = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return u32x4{x[0], y[0], x[1], y[1]};
+}
+__device__ __forceinline__ int pair_column(int g) { return 16 * (g & 1) + 8 * (g >> 1); }
+
 __device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4)); }
 
 // The k loop of a work-group: kt_n stages of 128 from k = kbase (KT > 0: kt_n = KT).  X rows m0.. (rows past
@@ -654,7 +664,9 @@ int launch_proj(GemmParams p, int splits, float* partial, hipStream_t stream, co
 // Measured (four weights in turn from a HIP graph; us, before -> here): 8,192 rows QKV
 // N = 4,096 154 -> 72, gate|up N = 6,144 183 -> 104 (990 TFLOP/s), o K = 2,048 83 -> 39,
 // down K = 3,072 119 -> 54; 4,096 rows 83 -> 39, 102 -> 62, 49 -> 25, 68 -> 34; the QKV
-// product with its epilogue, in the layer, 195 -> 100 and 110 -> 56.  A 256 x 256
+// product with its epilogue, in the layer, 195 -> 100 and 110 -> 56.  16-byte stores (two
+// output subtiles regrouped by pair_columns) instead of 8: QKV 72 -> 65 us at 8,192 rows, o
+// 25 -> 23 us at 4,096.  A 256 x 256
 // tile's 64 k take ~2.3 us for 2,048 cycles of MFMAs per SIMD: the int8 conversions (48 VALU
 // per 32 MFMAs, both waves of a SIMD at once) and the LDS (208 KB per block at 128 B per
 // clock) share that time with them.
@@ -1095,24 +1107,28 @@ __global__ __launch_bounds__(L::kWaves* kWave) void proj_tile_kernel(GemmParams 
     tile_qkv_epilogue<L, KV>(qa, smem, p.m, m0, n0, w.wave, lane);
     return;
   }
+  const bool wide = ((uintptr_t)p.y % 16) == 0 && p.ldy % 8 == 0;
 #pragma unroll
   for (int mi = 0; mi < kMine; ++mi) {
     const int m = m0 + lrow0 + mi * 16;
-    if (m >= p.m) continue;
-    if constexpr (EPI == 0) {
+    // the row's 16-column output subtiles in pairs: with 16-byte aligned rows one store each
+    constexpr int kOut = EPI == 1 ? NPW / 2 : NPW;
+    static_assert(kOut % 2 == 0, "output subtiles in pairs");
+    uint16_t* dst = p.y + (int64_t)m * p.ldy + (EPI == 1 ? n0 / 2 : n0) + w.nw * kOut * 16;
+    auto out4 = [&](int o) {
+      if constexpr (EPI == 1) return swiglu4(acc[mi][2 * o], acc[mi][2 * o + 1], sc[2 * o], sc[2 * o + 1]);
+      const floatx4 v = acc[mi][o];
+      return u32x2{pack_bf16x2(v[0] * sc[o][0], v[1] * sc[o][1]), pack_bf16x2(v[2] * sc[o][2], v[3] * sc[o][3])};
+    };
 #pragma unroll
-      for (int ns = 0; ns < NPW; ++ns) {
-        const int n = n0 + (w.nw * NPW + ns) * 16 + 4 * g;
-        const floatx4 v = acc[mi][ns];
-        *(u32x2*)(p.y + (int64_t)m * p.ldy + n) =
-            u32x2{pack_bf16x2(v[0] * sc[ns][0], v[1] * sc[ns][1]), pack_bf16x2(v[2] * sc[ns][2], v[3] * sc[ns][3])};
-      }
-    } else if constexpr (EPI == 1) {
-      static_assert(NPW % 2 == 0, "a wave holds paired gate / up subtiles");
-#pragma unroll
-      for (int ns = 0; ns < NPW; ns += 2) {
-        const u32x2 bits = swiglu4(acc[mi][ns], acc[mi][ns + 1], sc[ns], sc[ns + 1]);
-        *(u32x2*)(p.y + (int64_t)m * p.ldy + (n0 + (w.nw * NPW + ns) * 16) / 2 + 4 * g) = bits;
+    for (int o = 0; o < kOut; o += 2) {
+      const u32x2 x = out4(o), y = out4(o + 1);
+      if (wide) {
+        const u32x4 both = pair_columns(x, y);
+        if (m < p.m) *(u32x4*)(dst + o * 16 + pair_column(g)) = both;
+      } else if (m < p.m) {
+        *(u32x2*)(dst + o * 16 + 4 * g) = x;
+        *(u32x2*)(dst + (o + 1) * 16 + 4 * g) = y;
       }
     }
   }
@@ -1236,10 +1252,15 @@ int dispatch_w8a16(GemmParams p, int epilogue, int splits, float* partial, hipSt
 // of W, then runs its 80 MFMAs on the current one.  Spreading the weight copies (HBM
 // misses) over all waves keeps any one wave from queueing behind them; the two waves of
 // a SIMD still finish a stage apart, the older one ahead.  Stages run on across
-// blocks.  A range of ~9.3 groups ends in a short block of one or two groups: there the
-// waves whose 128 columns are all past the end skip their MFMAs and the weight copies of
-// absent rows are not issued (~23 % of the MFMAs were on such columns).  Rows beyond m
-// re-read row m - 1 and are never stored; more than 320 rows take further passes.
+// blocks.  The logits leave in 16-byte stores (two subtiles regrouped by pair_columns), and
+// the stage after a full block waits for its copies only, not for those stores: 320 rows'
+// logits 127 -> 122.5 us (their argmax partials alone take ~115).  Holding each next k-step's
+// fragments in registers through the current one's MFMAs, as the prefill tiles do, was
+// slower (151 us): a wave's reads then wait for each other in order.  A range of ~9.3 groups
+// ends in a short block of one or two groups: there the waves whose 128 columns are all past
+// the end skip their MFMAs and the weight copies of absent rows are not issued (~23 % of the
+// MFMAs were on such columns).  Rows beyond m re-read row m - 1 and are never stored; more
+// than 320 rows take further passes.
 constexpr int kLmMaxGrid = 256;  // persistent work-groups (one per CU)
 constexpr int kLmRows = 320;
 constexpr int kLmCols = 256;
@@ -1262,6 +1283,7 @@ struct LmStage {
 // scalar base for the stage (X: k0; W: the block's first column and k0) plus a 32-bit
 // lane offset that depends only on the pass's first row (X) or the block's width (W), so
 // a stage's copies need no 64-bit arithmetic.
+constexpr int kLmFullStores = 40;  // 16-byte stores per wave of a full block's logits (5 x 8 / 2 subtile pairs)
 constexpr int kLmXCopies = kLmXBytes / 1024 / kLmWaves;  // 5
 static_assert(kLmXBytes % (1024 * kLmWaves) == 0, "X slots split evenly over the waves");
 
@@ -1389,8 +1411,16 @@ __global__ __launch_bounds__(kLmWaves * kWave) void lm_head_kernel(GemmParams p)
   lm_offsets(p, cur, wave, lane, copies);
   int off_m0 = cur.m0, off_cols = cur.ccols;  // what the offsets were built for
   lm_issue(p, smem, cur, copies, wave);
+  const bool wide = p.y != nullptr && ((uintptr_t)p.y % 16) == 0 && p.ldy % 8 == 0;
+  bool stores = false;  // the last block's stores may still be in flight
   for (int u = 0; u < total; ++u) {
-    wait_vmcnt<0>();                                   // this wave's copies of stage u
+    // this wave's copies of stage u (older than the last block's stores, if any)
+    if (stores) {
+      wait_vmcnt<kLmFullStores>();
+      stores = false;
+    } else {
+      wait_vmcnt<0>();
+    }
     asm volatile("s_barrier" ::: "memory");           // everyone's; stage u - 1 fully read
     const bool more = u + 1 < total;
     int npass = pass, nbi = bi, nt = t + 1;
@@ -1424,6 +1454,23 @@ __global__ __launch_bounds__(kLmWaves * kWave) void lm_head_kernel(GemmParams p)
     // position 4 ns + i in column order, then turned into a range column once per row
     const int ngrp = st.ccols / kArgmaxCols;
     const uint32_t col0 = (uint32_t)(st.c0 - rc0 + nw * 128 + 4 * g);
+    if (wide) {
+      // a block whose rows and columns are all there: its 40 stores per wave are known, so
+      // the next stage waits for its copies (issued before them) and not for the stores
+      stores = st.m0 + kLmRows <= p.m && ngrp == 4;
+      const int row = st.m0 + mw * 80 + r;
+      uint16_t* dst = p.y + (int64_t)row * p.ldy + st.c0 + nw * 128 + pair_column(g);
+#pragma unroll
+      for (int mi = 0; mi < 5; ++mi)
+#pragma unroll
+        for (int ns = 0; ns < 8; ns += 2) {
+          const floatx4 v = acc[mi][ns], w = acc[mi][ns + 1];
+          const u32x4 both = pair_columns(u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])},
+                                          u32x2{pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3])});
+          if (row + mi * 16 < p.m && 2 * nw + ns / 4 < ngrp)
+            *(u32x4*)(dst + (int64_t)mi * 16 * p.ldy + ns * 16) = both;
+        }
+    }
 #pragma unroll
     for (int mi = 0; mi < 5; ++mi) {
       const int m = st.m0 + mw * 80 + mi * 16 + r;
@@ -1437,8 +1484,8 @@ __global__ __launch_bounds__(kLmWaves * kWave) void lm_head_kernel(GemmParams p)
           const int n = st.c0 + nw * 128 + ns * 16 + 4 * g;
           const floatx4 v = acc[mi][ns];
           const u32x2 bits = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-          if (p.y != nullptr && m < p.m && grp < ngrp) *(u32x2*)(p.y + (int64_t)m * p.ldy + n) = bits;
-          if (grp < ngrp) {
+          if (p.y != nullptr && !wide && m < p.m && grp < ngrp) *(u32x2*)(p.y + (int64_t)m * p.ldy + n) = bits;
+          if (p.argmax != nullptr && grp < ngrp) {
             const uint32_t o0 = bf16x2_order(bits[0]);
             const uint32_t o1 = bf16x2_order(bits[1]);
             const uint32_t rank = 31u - 4u * ns;
