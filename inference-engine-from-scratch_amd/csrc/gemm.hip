@@ -1365,6 +1365,11 @@ __device__ __forceinline__ uint32_t bf16x2_order(uint32_t pair) {
   return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, t) - __builtin_bit_cast(u16x2, sgn));
 }
 
+// What a block's end writes, each in a kernel without the others' code (a call of one short
+// block per work-group feels the instruction fetches): the argmax partials alone, logits in
+// 8-byte stores, or logits whose full blocks leave in 16-byte stores.
+enum class LmOut { kArgmax, kLogits, kWideLogits };
+template <LmOut OUT>
 __global__ __launch_bounds__(kLmWaves * kWave) void lm_head_kernel(GemmParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -1411,11 +1416,11 @@ __global__ __launch_bounds__(kLmWaves * kWave) void lm_head_kernel(GemmParams p)
   lm_offsets(p, cur, wave, lane, copies);
   int off_m0 = cur.m0, off_cols = cur.ccols;  // what the offsets were built for
   lm_issue(p, smem, cur, copies, wave);
-  const bool wide = p.y != nullptr && ((uintptr_t)p.y % 16) == 0 && p.ldy % 8 == 0;
+  constexpr bool LOGITS = OUT != LmOut::kArgmax, WIDE = OUT == LmOut::kWideLogits;
   bool stores = false;  // the last block's stores may still be in flight
   for (int u = 0; u < total; ++u) {
     // this wave's copies of stage u (older than the last block's stores, if any)
-    if (stores) {
+    if (WIDE && stores) {
       wait_vmcnt<kLmFullStores>();
       stores = false;
     } else {
@@ -1454,10 +1459,11 @@ __global__ __launch_bounds__(kLmWaves * kWave) void lm_head_kernel(GemmParams p)
     // position 4 ns + i in column order, then turned into a range column once per row
     const int ngrp = st.ccols / kArgmaxCols;
     const uint32_t col0 = (uint32_t)(st.c0 - rc0 + nw * 128 + 4 * g);
-    if (wide) {
+    const bool pairs = WIDE && ngrp == 4;  // a range's short last block keeps 8-byte stores
+    if (pairs) {
       // a block whose rows and columns are all there: its 40 stores per wave are known, so
       // the next stage waits for its copies (issued before them) and not for the stores
-      stores = st.m0 + kLmRows <= p.m && ngrp == 4;
+      stores = st.m0 + kLmRows <= p.m;
       const int row = st.m0 + mw * 80 + r;
       uint16_t* dst = p.y + (int64_t)row * p.ldy + st.c0 + nw * 128 + pair_column(g);
 #pragma unroll
@@ -1467,7 +1473,7 @@ __global__ __launch_bounds__(kLmWaves * kWave) void lm_head_kernel(GemmParams p)
           const floatx4 v = acc[mi][ns], w = acc[mi][ns + 1];
           const u32x4 both = pair_columns(u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])},
                                           u32x2{pack_bf16x2(w[0], w[1]), pack_bf16x2(w[2], w[3])});
-          if (row + mi * 16 < p.m && 2 * nw + ns / 4 < ngrp)
+          if (row + mi * 16 < p.m)
             *(u32x4*)(dst + (int64_t)mi * 16 * p.ldy + ns * 16) = both;
         }
     }
@@ -1484,8 +1490,8 @@ __global__ __launch_bounds__(kLmWaves * kWave) void lm_head_kernel(GemmParams p)
           const int n = st.c0 + nw * 128 + ns * 16 + 4 * g;
           const floatx4 v = acc[mi][ns];
           const u32x2 bits = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-          if (p.y != nullptr && !wide && m < p.m && grp < ngrp) *(u32x2*)(p.y + (int64_t)m * p.ldy + n) = bits;
-          if (p.argmax != nullptr && grp < ngrp) {
+          if (LOGITS && !pairs && m < p.m && grp < ngrp) *(u32x2*)(p.y + (int64_t)m * p.ldy + n) = bits;
+          if ((!LOGITS || p.argmax != nullptr) && grp < ngrp) {
             const uint32_t o0 = bf16x2_order(bits[0]);
             const uint32_t o1 = bf16x2_order(bits[1]);
             const uint32_t rank = 31u - 4u * ns;
@@ -1678,6 +1684,19 @@ __global__ __launch_bounds__(kLmWaves * kWave) void lm_head_small_kernel(GemmPar
   }
 }
 
+template <LmOut OUT>
+int launch_lm_head_rows(const GemmParams& p, int grid, hipStream_t stream) {
+  static const hipError_t attr = hipFuncSetAttribute(
+      (const void*)lm_head_kernel<OUT>, hipFuncAttributeMaxDynamicSharedMemorySize, kLmRing * kLmStage);
+  if (attr != hipSuccess) {
+    set_error("lm_head: cannot reserve %d bytes of LDS: %s", kLmRing * kLmStage, hipGetErrorString(attr));
+    return NE_ELAUNCH;
+  }
+  hipLaunchKernelGGL((lm_head_kernel<OUT>), dim3((unsigned)grid), dim3(kLmWaves * kWave), kLmRing * kLmStage,
+                     stream, p);
+  return check_launch("lm_head");
+}
+
 int launch_lm_head(GemmParams p, hipStream_t stream) {
   const int groups = p.n / kArgmaxCols;
   const int grid = groups < kLmMaxGrid ? groups : kLmMaxGrid;
@@ -1692,14 +1711,11 @@ int launch_lm_head(GemmParams p, hipStream_t stream) {
                        stream, p);
     return check_launch("lm_head");
   }
-  static const hipError_t attr = hipFuncSetAttribute(
-      (const void*)lm_head_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLmRing * kLmStage);
-  if (attr != hipSuccess) {
-    set_error("lm_head: cannot reserve %d bytes of LDS: %s", kLmRing * kLmStage, hipGetErrorString(attr));
-    return NE_ELAUNCH;
-  }
-  hipLaunchKernelGGL(lm_head_kernel, dim3((unsigned)grid), dim3(kLmWaves * kWave), kLmRing * kLmStage, stream, p);
-  return check_launch("lm_head");
+  if (p.y == nullptr) return launch_lm_head_rows<LmOut::kArgmax>(p, grid, stream);
+  // 16-byte stores: rows that start on 16 bytes, and ranges with a full block of 4 groups
+  if (((uintptr_t)p.y % 16) == 0 && p.ldy % 8 == 0 && groups >= 4 * grid)
+    return launch_lm_head_rows<LmOut::kWideLogits>(p, grid, stream);
+  return launch_lm_head_rows<LmOut::kLogits>(p, grid, stream);
 }
 
 }  // namespace

@@ -118,20 +118,22 @@ def test_unaligned_cache_takes_the_other_kernel(device):
         assert int((o.int() - e.int()).abs().max()) <= 2 and float((o != e).float().mean()) < 0.02
 
 
-@pytest.mark.parametrize("m,ld,first", [(321, 4096 + 4, 0), (330, 4096 + 8, 4), (320, 4096 + 8, 0)])
-def test_outputs_of_every_row_alignment(device, m, ld, first):
+@pytest.mark.parametrize("m,pad,first", [(321, 4, 0), (330, 8, 4), (320, 8, 0), (640, 8, 0)])
+def test_outputs_of_every_row_alignment(device, m, pad, first):
     """Rows that do not start on 16 bytes leave in 8-byte stores: the same bits, and nothing
-    beyond the columns, from the projection tiles and the LM head."""
+    beyond the columns, from the projection tiles and the LM head (full and short blocks)."""
     g = torch.Generator(device=device).manual_seed(m)
     w, s = weight(4096, 256, device)
-    embed = (torch.randn(4096, 256, device=device, generator=g) * 0.02).to(torch.bfloat16)
-    for rows, call in ((1000, lambda x, out: kernels.w8a16_gemm(x, w, s, out=out)),
-                       (m, lambda x, out: kernels.lm_head(x, embed, logits=out))):
+    embed = (torch.randn(65664, 256, device=device, generator=g) * 0.02).to(torch.bfloat16)
+    for rows, n, call in ((1000, 4096, lambda x, out: kernels.w8a16_gemm(x, w, s, out=out)),
+                          (m, 65664, lambda x, out: kernels.lm_head(x, embed, logits=out))):
         x = torch.randn(rows, 256, device=device, generator=g).to(torch.bfloat16)
-        plain = torch.empty(rows, 4096, dtype=torch.bfloat16, device=device)
+        plain = torch.empty(rows, n, dtype=torch.bfloat16, device=device)
         call(x, plain)
+        assert rel_err(plain, product(x, w, s) if n == 4096 else x.float() @ embed.float().t()) < 2.5e-3
+        ld = n + pad
         flat = torch.zeros(rows * ld + 16, dtype=torch.bfloat16, device=device)
         view = flat[first:first + rows * ld].view(rows, ld)
-        call(x, view[:, :4096])
-        assert torch.equal(view[:, :4096], plain)
-        assert not view[:, 4096:].any() and not flat[:first].any() and not flat[first + rows * ld:].any()
+        call(x, view[:, :n])
+        assert torch.equal(view[:, :n], plain)
+        assert not view[:, n:].any() and not flat[:first].any() and not flat[first + rows * ld:].any()
