@@ -97,7 +97,9 @@ struct AttnParams {
   int32_t* plan;       // DMA kernel: first work-group of each sequence, then the total
   int32_t plan_w;      // DMA kernel: tiles per split (0: derived from the total work)
   int32_t plan_whole;  // planned path: one work item per sequence (head-split kernel)
-  int32_t plan_grid;   // DMA kernel: work-groups launched
+  int32_t plan_grid;   // DMA kernel: work items of the plan (the grid, with one wave per KV head)
+  int32_t plan_ks;     // DMA kernel: waves per KV head of a split plan (split_plan_ks)
+  int32_t plan_floor;  // DMA kernel: least tiles per split
   int32_t max_ctx;     // the caller's bound on ctx_len
   int32_t rows_kg;     // query-tile kernel: key groups per work-group (0: another kernel serves the call)
   int32_t row_tiles;   // query-tile kernel: tiles of query rows per sequence
@@ -1336,10 +1338,38 @@ constexpr int kPlanFloorTiles = 8;                    // no split shorter than 1
 constexpr int kPlanCUs = 256;                         // work-groups the plan aims to fill
 constexpr int kWholeMaxTiles = 64;                    // longest context of a whole-sequence plan
 
+// Waves per KV head of a split plan (4, 2 or 1).  With KS, an item covers KS times the tiles
+// and is served by KS work-groups of 8 / KS KV heads, whose waves take a part of its tiles
+// each and merge through LDS: the same work-groups in flight, 1 / KS of the fp32 partials to
+// write and merge, and items cut finer per wave (16 sequences of 256-2,048 keys had 152
+// work-groups of 8-tile items on 256 CUs, and have ~224 of 6 tiles per wave).
+// Measured per planned call with its merge, one wave per head -> here: that shape in bf16
+// 27.9 -> 24.5 us; one sequence of 17,408 keys 41.8 -> 26.9 us (int8); 8 of 2,000-8,000 34.0
+// -> 28.8; 24 of 300-2,000 24.3 -> 24.2 (bf16 33.0 -> 31.4).  32 such sequences lose with 4
+// (28.8 -> 29.5) and gain with 2 (25.8); 48 are even with 2 (34.4, 34.8) and 64 lose
+// (200-1,500 keys 34.2 -> 37.1).  From 641 keys on 4 also beats one whole item per sequence
+// (16 sequences of 200-800 keys 15.6 -> 14.8, bf16 20.3 -> 15.8; at 640 13.7 and 14.1, bf16
+// 16.8 and 14.3; at 512 12.4 and 13.8).
+constexpr int kSplitKs4MaxSeqs = 24;
+constexpr int kSplitKs2MaxSeqs = 40;
+constexpr int kSplitKs4MinTiles = 40;
+constexpr int kSplitKsFloorTiles = 4;  // per wave: its ring
+int split_plan_grid(int num_seqs, int ks) { return max(kPlanCUs / ks, 2 * num_seqs); }  // items
+int split_plan_ks(int num_seqs, int max_ctx, int split_len, int mtiles) {
+  const int64_t tiles = ((int64_t)max_ctx + kTileKeys - 1) / kTileKeys;
+  if (split_len != 0 || mtiles != 1) return 1;
+  const int ks = num_seqs <= kSplitKs4MaxSeqs ? 4 : num_seqs <= kSplitKs2MaxSeqs ? 2 : 1;
+  if (tiles <= (ks == 4 ? kSplitKs4MinTiles : kWholeMaxTiles)) return 1;
+  // every item's slot list holds its tiles
+  const int64_t need = num_seqs + (num_seqs * tiles + kPlanMaxTiles - 1) / kPlanMaxTiles;
+  return need <= split_plan_grid(num_seqs, ks) ? ks : 1;
+}
+
 // Waves per KV head (4 or 2) when the precomputed plan gives every sequence one
 // whole work item, served by that many work-groups (one per CU at most): no split
 // partials and no merge kernel.  0 when the split plan serves the shape better.
 int whole_plan_ks(int num_seqs, int max_ctx, int split_len, int mtiles) {
+  if (split_plan_ks(num_seqs, max_ctx, split_len, mtiles) > 1) return 0;
   if (split_len != 0 || mtiles != 1 || (max_ctx + kTileKeys - 1) / kTileKeys > kWholeMaxTiles) return 0;
   if (num_seqs * 4 <= kPlanCUs) return 4;
   if (num_seqs * 2 <= kPlanCUs) return 2;
@@ -1351,9 +1381,9 @@ int whole_plan_ks(int num_seqs, int max_ctx, int split_len, int mtiles) {
 // covers tiles [tiles_b s / n_b, tiles_b (s+1) / n_b)).  W is p.plan_w when the
 // caller fixed the split length; else 16 when every context fits in 16 tiles (one
 // split per sequence, so no partials and no merge kernel); else
-// max(8, ceil(T / (G - B))) for T = sum_b tiles_b, G = p.plan_grid work-groups and
-// B sequences -- splitting is paid for already, so W only balances the longest
-// split against the mean.  Both keep sum_b n_b <= G:
+// max(8, ceil(T / (G - B))) (16 with four waves per KV head) for T = sum_b tiles_b, G =
+// p.plan_grid items and B sequences -- splitting is paid for already, so W only balances
+// the longest split against the mean.  Both keep sum_b n_b <= G:
 // the longest sequence is spread over as many work-groups as its share of T asks
 // for instead of one per fixed-length split, and no CU waits for a second round
 // of work-groups.  Work-group w serves split w - N_b of the sequence with
@@ -1418,7 +1448,7 @@ __device__ PlanScan plan_scan(const AttnParams& p, int* s_plan) {
     if (p.plan_whole)
       W = max(max_tiles, 1);  // every sequence in one item
     else
-      W = max_tiles <= kPlanMinTiles ? kPlanMinTiles : max(kPlanFloorTiles, (T + (G - B) - 1) / (G - B));
+      W = max_tiles <= kPlanMinTiles ? kPlanMinTiles : max(p.plan_floor, (T + (G - B) - 1) / (G - B));
   }
   if (W > kPlanMaxTiles) {
     if (tid == 0 && blockIdx.x == 0) atomicOr(p.error_flag, 1u);
@@ -1454,12 +1484,11 @@ __device__ PlanScan plan_scan(const AttnParams& p, int* s_plan) {
   return ps;
 }
 
-// Called by all threads of the work-group; false when the work-group has no work.
-__device__ bool plan_item(const AttnParams& p, int* s_plan, PlanItem& item) {
+// Item w.  Called by all threads of the work-group; false when the item has no work.
+__device__ bool plan_item(const AttnParams& p, int* s_plan, int w, PlanItem& item) {
   const int tid = threadIdx.x;
   if (tid == 0) s_plan[16] = -1;  // ordered before the owner's write by plan_scan's barriers
   const PlanScan ps = plan_scan(p, s_plan);
-  const int w = blockIdx.x;
   const int k = (w >= ps.first[0] && w < ps.first[1]) ? 0
                 : ((w >= ps.first[1] && w < ps.first[1] + ps.n[1]) ? 1 : -1);
   if (k >= 0) {
@@ -1817,7 +1846,7 @@ __device__ __forceinline__ void compute_iter_bf(const IterRegs<false>& R, const 
 // BF16: a bf16 cache (SDT unused): two-tile rings, bf16 MFMA scores (compute_iter_bf).
 template <int SDT, bool PLANNED, int MT, int KS = 1, bool BF16 = false>
 __global__ __launch_bounds__((DmaShape<KS, BF16>::waves * kWave)) void paged_attention_dma_kernel(AttnParams p) {
-  static_assert(KS == 1 || (PLANNED && MT == 1), "head split: planned, one row tile");
+  static_assert(KS == 1 || MT == 1, "head split: one row tile");
   using Shape = DmaShape<KS, BF16>;
   constexpr int HG = Shape::heads;  // KV heads per work-group
   constexpr int RING = Shape::ring;
@@ -1867,7 +1896,7 @@ __global__ __launch_bounds__((DmaShape<KS, BF16>::waves * kWave)) void paged_att
     }
     planned_slot = my_slot;
   } else {
-    if (!plan_item(p, s_plan, item)) return;
+    if (!plan_item(p, s_plan, widx, item)) return;
   }
   // the item is the same for the whole work-group: keep it in scalar registers, so
   // that the loop and its waits are compiled as uniform
@@ -1929,8 +1958,8 @@ __global__ __launch_bounds__((DmaShape<KS, BF16>::waves * kWave)) void paged_att
   }
   if constexpr (!PLANNED) {
     const int32_t* bt_row = p.block_tables + (int64_t)seq * p.bt_stride;
-    for (int t = tid; t < n_tiles; t += kThreads) {
-      const int key0 = kstart + kTileKeys * t;
+    for (int t = tid; t < j1 - j0; t += kThreads) {
+      const int key0 = kTileKeys * (j0 + t);
       s_slot[t] = bt_row[key0 / p.block_size] * p.block_size + key0 % p.block_size;
     }
   } else {
@@ -2578,6 +2607,13 @@ int launch_attention_dma_ks(const AttnParams& p, unsigned grid, hipStream_t s) {
   return check_launch("paged_attention_dma_kernel");
 }
 
+// the split plan of a call: the same for ne_paged_attention_plan and the calls that read it
+void set_split_plan(AttnParams& p, int split_len) {
+  p.plan_ks = split_plan_ks(p.num_seqs, p.max_ctx, split_len, p.mtiles);
+  p.plan_floor = p.plan_ks > 1 ? kSplitKsFloorTiles * p.plan_ks : kPlanFloorTiles;
+  if (p.plan_ks > 1) p.plan_grid = split_plan_grid(p.num_seqs, p.plan_ks);
+}
+
 template <int SDT, bool PLANNED, int MT, bool BF16>
 int launch_attention_dma_mt(const AttnParams& p, hipStream_t s) {
   if constexpr (PLANNED && MT == 1) {
@@ -2592,7 +2628,17 @@ int launch_attention_dma_mt(const AttnParams& p, hipStream_t s) {
   // no sequence is split when every context fits in one split's minimum length
   const int min_w = p.plan_w > 0 ? p.plan_w : kPlanMinTiles;
   const bool no_splits = ceil_div(p.max_ctx, kTileKeys) <= min_w;
-  const int rc = launch_attention_dma_ks<SDT, PLANNED, MT, 1, BF16>(p, (unsigned)p.plan_grid, s);
+  int rc = NE_OK;
+  if constexpr (MT == 1) {
+    if (p.plan_ks == 4)
+      rc = launch_attention_dma_ks<SDT, PLANNED, MT, 4, BF16>(p, (unsigned)p.plan_grid * DmaShape<4>::groups, s);
+    else if (p.plan_ks == 2)
+      rc = launch_attention_dma_ks<SDT, PLANNED, MT, 2, BF16>(p, (unsigned)p.plan_grid * DmaShape<2>::groups, s);
+    else
+      rc = launch_attention_dma_ks<SDT, PLANNED, MT, 1, BF16>(p, (unsigned)p.plan_grid, s);
+  } else {
+    rc = launch_attention_dma_ks<SDT, PLANNED, MT, 1, BF16>(p, (unsigned)p.plan_grid, s);
+  }
   if (rc != NE_OK || no_splits) return rc;
   hipLaunchKernelGGL(attention_plan_merge_kernel, dim3((unsigned)p.num_seqs * kHeadWaves),
                      dim3(kPartRows * 16), 0, s, p);
@@ -2699,6 +2745,7 @@ int make_params(const void* q, int64_t q_token_stride, int64_t q_head_stride, co
   p.plan_grid = L.plan_grid;
   p.plan_whole = 0;  // the planned entry point decides
   p.max_ctx = max_ctx_len;
+  set_split_plan(p, split_len);
   p.rows_kg = L.rows_kg;
   p.row_tiles = L.row_tiles;
   return NE_OK;
@@ -2875,6 +2922,7 @@ extern "C" int ne_paged_attention_plan(const int32_t* block_tables, int32_t bloc
   p.max_ctx = max_ctx_len;
   p.plan_w = L.plan_w;
   p.plan_grid = L.plan_grid;
+  set_split_plan(p, split_len);
   p.plan_whole = whole_plan_ks(num_seqs, max_ctx_len, split_len, L.mtiles) > 0;
   char* ws = (char*)workspace;
   p.error_flag = (uint32_t*)(ws + L.error_off);
@@ -2936,6 +2984,8 @@ int launch_kv_stream(const AttnParams& p, hipStream_t s) {
       return launch_kv_stream_ks<4, BF16>(p, (unsigned)p.num_seqs * DmaShape<4>::groups, s);
     return launch_kv_stream_ks<2, BF16>(p, (unsigned)p.num_seqs * DmaShape<2>::groups, s);
   }
+  if (p.plan_ks == 4) return launch_kv_stream_ks<4, BF16>(p, (unsigned)p.plan_grid * DmaShape<4>::groups, s);
+  if (p.plan_ks == 2) return launch_kv_stream_ks<2, BF16>(p, (unsigned)p.plan_grid * DmaShape<2>::groups, s);
   return launch_kv_stream_ks<1, BF16>(p, (unsigned)p.plan_grid, s);
 }
 }  // namespace
@@ -2972,6 +3022,7 @@ extern "C" int ne_paged_kv_stream_planned(const void* k_cache, const void* v_cac
   p.max_ctx = max_ctx_len;
   p.plan_w = L.plan_w;
   p.plan_grid = L.plan_grid;
+  set_split_plan(p, split_len);
   p.plan_whole = whole_plan_ks(num_seqs, max_ctx_len, split_len, L.mtiles) > 0;
   char* ws = (char*)workspace;
   p.error_flag = (uint32_t*)(ws + L.error_off);

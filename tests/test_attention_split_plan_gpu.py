@@ -1,0 +1,47 @@
+"""A6 on split plans with several waves per KV head (up to 24 sequences past 640 keys: four;
+up to 40 past 1,024: two) against the oracle, planned and unplanned (the same items and sums,
+so the same bits), at the rule's edges and with sequences far shorter than the longest.
+
+Bar: 6e-3 relative, four roundings of 2^-9 (output, probabilities, the oracle's dequantised
+keys and values; 1.1e-3 rms each) with a factor of 2.6 to spare.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from helpers import make_batch, make_pool, real_rows, rel_err
+from oracle.attention import paged_attention_reference
+from nanoengine_amd import kernels
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kv", ["bf16", "int8"])
+@pytest.mark.parametrize("seqs,longest", [(1, 641), (1, 2500), (3, 640), (24, 700), (25, 1024), (25, 1025), (40, 1100),
+                                          (41, 1100)])
+def test_split_items(device, kv, seqs, longest):
+    ctx = [longest] + [1 + 37 * i % 300 for i in range(seqs - 1)]
+    ctx[-1] = longest - 1 if seqs > 1 else longest
+    q_lens = [min(c, 1 + i % 8) for i, c in enumerate(ctx)]
+    num_blocks = sum(-(-c // 16) for c in ctx) + 4
+    kc, vc, ks, vs = make_pool(num_blocks, 16, 8, kv, torch.float16, seed=41)
+    tables, ctx_t, qs, ql, rows = make_batch(ctx, q_lens, num_blocks, 16, seed=42)
+    q = torch.randn(rows, 16, 128, generator=torch.Generator().manual_seed(43)).to(torch.bfloat16)
+    d = lambda t: None if t is None else t.to(device)
+    tables_d, ctx_d, qs_d, ql_d = map(d, (tables, ctx_t, qs, ql))
+    args = (d(q), d(kc), d(vc), d(ks), d(vs), tables_d, 16, ctx_d, qs_d, ql_d)
+    ws = kernels.AttentionWorkspace()
+    unplanned = kernels.paged_verify_attention(*args, max_q_len=8, max_ctx_len=longest, workspace=ws)
+    kernels.paged_attention_plan(tables_d, 16, ctx_d, qs_d, ql_d, 16, 8, 8, longest, ws)
+    planned = kernels.paged_verify_attention(*args, max_q_len=8, max_ctx_len=longest, workspace=ws, planned=True)
+    torch.cuda.synchronize()
+    assert ws.error_flag() == 0
+    idx = real_rows(qs, ql)
+    ref = paged_attention_reference(q, kc, vc, ks, vs, tables, 16, ctx_t, qs, ql,
+                                    model_dtype=torch.bfloat16 if kv == "bf16" else torch.float16)
+    assert rel_err(planned.cpu()[idx], ref[idx]) < 6e-3
+    assert rel_err(unplanned.cpu()[idx], ref[idx]) < 6e-3
+    if not (25 <= seqs and longest <= 1024) and longest > 640:
+        assert torch.equal(planned.cpu()[idx], unplanned.cpu()[idx])
