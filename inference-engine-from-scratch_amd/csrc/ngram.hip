@@ -13,6 +13,11 @@
 // which is the common case in long histories; without one, the same pass has already
 // found the smaller n's answers.  The guesses are the tokens that followed
 // the window, clipped to the history, so they are never empty.
+// A call is a chain of memory round trips (the length, the history, the guesses): the
+// stretch's loads go out together, the guesses of a single pass come from LDS, and a thread
+// stops at its first full match: 64 sequences of 64-2,048 tokens 10.8 -> 7.0 us.
+#include <type_traits>
+
 #include "ne_common.hpp"
 
 namespace ne {
@@ -80,15 +85,25 @@ __global__ __launch_bounds__(256) void ngram_kernel(const int32_t* history, int6
 #pragma unroll
   for (int i = 0; i < kMaxNgram; ++i) found[i] = -1;
   if (!scan) __syncthreads();  // uniform: publishes s_want
+  // history positions [staged_from, len - 1) are in s_hist after a scan of one pass
+  const int first_base = len - 2 - kScanChunk - kMaxNgram + 2;
+  int staged_from = max(first_base, 0);
   for (int hi = scan ? len - 2 : -1; hi >= 0; hi -= kScanChunk) {
     // the pass's ends are hi - 4095 .. hi and their windows reach 15 tokens further back:
     // s_hist[k] = h[base + k] for the history positions 0 .. hi among them.  The previous
     // pass's reads of s_hist ended before its last barrier.
     const int base = hi - kScanChunk - kMaxNgram + 2;
-    for (int k = tid; k < kStage; k += 256) {
-      const int pos = base + k;
-      s_hist[k] = (pos >= 0 && pos <= hi) ? h[pos] : 0;
+    // (every load of the stretch is requested before the first is stored)
+    int stage[kScanPerThread + 1];
+#pragma unroll
+    for (int j = 0; j <= kScanPerThread; ++j) {
+      const int pos = base + tid + j * 256;
+      const bool in = pos >= 0 && pos <= hi && tid + j * 256 < kStage;
+      stage[j] = in ? h[pos] : 0;
     }
+#pragma unroll
+    for (int j = 0; j <= kScanPerThread; ++j)
+      if (tid + j * 256 < kStage) s_hist[tid + j * 256] = stage[j];
     __syncthreads();
     // thread tid tests ends hi - tid, hi - tid - 256, ...: its first hit for each n is
     // its largest, and the owner of the chunk's largest hit has no larger one
@@ -103,29 +118,39 @@ __global__ __launch_bounds__(256) void ngram_kernel(const int32_t* history, int6
       const int e = hi - j * 256 - tid;
       if (e >= 0 && s_hist[e - base] == suffix[0]) hit |= 1u << j;
     }
-    while (hit != 0) {
-      const int j = __builtin_ctz(hit);
-      hit &= hit - 1;
-      const int e = hi - j * 256 - tid;
-      // the window's tokens are all read before the first comparison, so the LDS reads
-      // overlap (e - i - base >= 0 for every i: the stage reaches 15 tokens below the
-      // pass's lowest end)
-      int tok[kMaxNgram];
+    // the window's tokens are all read before the first comparison, so the LDS reads
+    // overlap (e - i - base >= 0 for every i: the stage reaches 15 tokens below the
+    // pass's lowest end); a window of nmax tokens ends the thread's search, since no
+    // smaller end can be the largest for any n
+    auto windows = [&](auto width) {
+      constexpr int N = decltype(width)::value;  // nmax <= N
+      while (hit != 0) {
+        const int j = __builtin_ctz(hit);
+        hit &= hit - 1;
+        const int e = hi - j * 256 - tid;
+        int tok[N];
 #pragma unroll
-      for (int i = 0; i < kMaxNgram; ++i) tok[i] = s_hist[e - i - base];
-      int c = 0;  // tokens ending at e that equal those ending at len - 1
-      bool same = true;
+        for (int i = 0; i < N; ++i) tok[i] = s_hist[e - i - base];
+        int c = 0;  // tokens ending at e that equal those ending at len - 1
+        bool same = true;
 #pragma unroll
-      for (int i = 0; i < kMaxNgram; ++i) {
-        if (same && i < nmax && e - i >= 0 && tok[i] == suffix[i]) {
-          ++c;
-        } else {
-          same = false;
+        for (int i = 0; i < N; ++i) {
+          if (same && i < nmax && e - i >= 0 && tok[i] == suffix[i]) {
+            ++c;
+          } else {
+            same = false;
+          }
         }
-      }
 #pragma unroll
-      for (int i = 0; i < kMaxNgram; ++i)
-        if (i < c && best[i] < 0) best[i] = e;
+        for (int i = 0; i < N; ++i)
+          if (i < c && best[i] < 0) best[i] = e;
+        if (c == nmax) break;
+      }
+    };
+    if (nmax <= 4) {
+      windows(std::integral_constant<int, 4>{});
+    } else {
+      windows(std::integral_constant<int, kMaxNgram>{});
     }
 #pragma unroll
     for (int i = 0; i < kMaxNgram; ++i) {
@@ -145,13 +170,14 @@ __global__ __launch_bounds__(256) void ngram_kernel(const int32_t* history, int6
         if (found[i] < 0) found[i] = top;
       }
     }
-    __syncthreads();
     bool done = false;
 #pragma unroll
     for (int i = 0; i < kMaxNgram; ++i)
       if (i == nmax - 1) done = found[i] >= 0;
     if (done) break;  // uniform: the largest n has its answer
     if (adv.num_out != nullptr && s_want <= 0) break;  // uniform: published before the barriers above
+    if (hi > kScanChunk - 1) staged_from = len;        // another pass takes the stage
+    __syncthreads();                                   // s_best and s_hist free for it
   }
   if (adv.num_out != nullptr) requested = s_want;
   const int want = min(requested, max_drafts);
@@ -170,7 +196,11 @@ __global__ __launch_bounds__(256) void ngram_kernel(const int32_t* history, int6
   }
   const int follow = e + 1;
   const int count = min(want, len - follow);
-  for (int i = tid; i < count; i += 256) drafts[(int64_t)b * max_drafts + i] = h[follow + i];
+  for (int i = tid; i < count; i += 256) {
+    const int pos = follow + i;
+    drafts[(int64_t)b * max_drafts + i] =
+        pos == len - 1 ? suffix[0] : (pos >= staged_from ? s_hist[pos - first_base] : h[pos]);
+  }
   if (tid == 0) num_drafts[b] = count;
 }
 
