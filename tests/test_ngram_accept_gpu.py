@@ -450,3 +450,47 @@ def test_history_append_stops_at_the_row_capacity(device):
     assert h.cpu()[0].tolist() == [-9] * 8 + [3, 4]
     assert h.cpu()[1].tolist() == [-9] * 10
     assert hld.cpu().tolist() == [10, 0]
+
+
+@pytest.mark.parametrize("num_tiles", [1, 63, 65, 511, 513, 1100])
+@pytest.mark.parametrize("k", [1, 4, 16])
+def test_greedy_partials_of_any_key_count(device, num_tiles, k):
+    """Greedy acceptance from argmax partials: rows are reduced a wave each, up to 8 keys per
+    lane at a time; the winner may sit at any key, the first and the last included."""
+    g = torch.Generator().manual_seed(num_tiles * 17 + k)
+    n, vocab = 6, 151936
+    rows = n * (k + 1)
+    keys = (torch.randint(0, 1 << 31, (rows, num_tiles), generator=g) << 32) | (
+        0xFFFFFFFF - torch.randint(0, vocab, (rows, num_tiles), generator=g))
+    at = torch.randint(0, num_tiles, (rows,), generator=g)
+    at[::3], at[1::3] = 0, num_tiles - 1
+    target = torch.randint(0, vocab, (rows,), generator=g)
+    keys[torch.arange(rows), at] = (0x7FFFFFFF << 32) | (0xFFFFFFFF - target)
+    drafts = target.view(n, k + 1)[:, :k].clone()
+    stop = [min(i, k) for i in range(n)]  # sequence i keeps its first min(i, k) guesses
+    for i, s in enumerate(stop):
+        if s < k:
+            drafts[i, s] = (drafts[i, s] + 1) % vocab
+    i32 = lambda t: t.to(torch.int32).contiguous().to(device)
+    out, num = kernels.accept(i32(drafts), i32(torch.full((n,), k)), i32(torch.arange(n) * (k + 1)), vocab,
+                              argmax_partials=keys.to(device))
+    for i, s in enumerate(stop):
+        assert int(num[i]) == s + 1
+        assert out[i, : s + 1].tolist() == target.view(n, k + 1)[i, : s + 1].tolist()
+
+
+@pytest.mark.parametrize("length", [5, 20, 257, 4097, 4098, 9000])
+@pytest.mark.parametrize("max_ngram", [2, 4, 5, 16])
+def test_ngram_guesses_at_the_end_of_the_history(device, length, max_ngram):
+    """The guesses end at the history's last token (which the staged stretch does not hold) or
+    come from a pass older than the newest one: equal to the oracle's."""
+    g = torch.Generator().manual_seed(length)
+    filler = torch.randint(100, 10_000_000, (length,), generator=g).tolist()
+    recent, old = list(filler), list(filler)
+    recent[-1] = recent[-2] = recent[-3]  # the match ends one before the last token
+    old[1] = old[-1]  # the only match is at the start
+    for history in (recent, old):
+        hist = torch.tensor([history], dtype=torch.int32, device=device)
+        drafts, num = kernels.ngram_propose(hist, torch.tensor([length], dtype=torch.int32, device=device),
+                                            torch.tensor([8], dtype=torch.int32, device=device), max_ngram, 8)
+        assert drafts[0, : int(num[0])].tolist() == propose(history, 8, max_ngram)
