@@ -493,4 +493,4 @@ def test_ngram_guesses_at_the_end_of_the_history(device, length, max_ngram):
         hist = torch.tensor([history], dtype=torch.int32, device=device)
         drafts, num = kernels.ngram_propose(hist, torch.tensor([length], dtype=torch.int32, device=device),
                                             torch.tensor([8], dtype=torch.int32, device=device), max_ngram, 8)
-        assert drafts[0, : int(num[0])].tolist() == propose(history, 8, max_ngram)
+        assert drafts[0, : int(num[0])].tolist() == oracle_ngram.propose(history, 8, max_ngram)
