@@ -1190,6 +1190,223 @@ int launch_proj_tile(ProjTile tile, const GemmParams& p, hipStream_t s, const ch
   return launch_proj_tile_as<Tile128x128, EPI, KV>(p, s, name, qa);
 }
 
+// ---- W8A16 projections of few rows -----------------------------------------------------
+// At up to 16 rows a work-group of the kernel above spends its time in a chain of stages
+// (copy, barrier, read, convert, multiply, ~0.5 us each) that hold a dozen MFMAs.  Here
+// nothing is staged: X (all of K, at most 32 KB) is copied to LDS once, every wave loads all
+// of its weight rows' K into registers in one burst, in the MFMA operand order, and then
+// multiplies as they arrive.  One barrier, one memory round trip.
+//   wave  = NPW weight subtiles of 16 rows x all PM token subtiles x K = 128 KT
+//   sums  = KG accumulators per output (k-step kk of a stage goes to accumulator kk KG / 4),
+//           added in order: the k-groups of the kernel above, so the results are its bits
+// Measured at 5 rows (kernel trace, fastest of 28; us, before -> here): QKV 8.7 -> 7.8,
+// gate|up 7.0 -> 6.4, o 4.5 -> 2.9, down 4.6 -> 3.9; four layers from a HIP graph 176.7 ->
+// 167.2.  What is left is the launch, one round trip to HBM and, for QKV, 128 KB of weights
+// into each of 32 CUs.
+template <int PM_, int NPW_, int KG_, int WAVES_, int KT_>
+struct FewLayout {
+  static constexpr int PM = PM_, NPW = NPW_, KG = KG_, WAVES = WAVES_, KT = KT_;
+  static constexpr int kRows = PM * 16;
+  static constexpr int kStage = kRows * 256;         // X rows of a 128-wide stage
+  static constexpr int kX = KT * kStage;
+  static constexpr int kCopies = KT * PM * 4;        // 1 KiB copies: 4 rows of 256 B
+  static constexpr int kPerWave = kCopies / WAVES;
+  static constexpr int kLoads = NPW * KT * 2;        // 16-byte weight loads per lane
+  static_assert(kCopies % WAVES == 0 && kLoads < 64, "copies split evenly; vmcnt range");
+  static_assert(kX <= 160 * 1024, "LDS");
+};
+
+template <typename L, int EPI, int KV>
+__global__ __launch_bounds__(L::WAVES* kWave) void proj_few_rows_kernel(GemmParams p, float* partial, QkvRopeArgs qa) {
+  constexpr int PM = L::PM, NPW = L::NPW, KG = L::KG, KT = L::KT;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  asm volatile("" ::"s"(p.x), "s"(p.ldx), "s"(p.w), "s"(p.scale), "s"(p.m), "s"(p.k), "s"(p.n), "s"(p.y), "s"(p.ldy));
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int lane = threadIdx.x % kWave;
+  const int r = lane & 15;
+  const int g = lane >> 4;
+  const int n0 = (blockIdx.x * L::WAVES + wave) * NPW * 16;  // this wave's first weight row
+  const int kbase = blockIdx.y * KT * kStageK;
+
+  // ---- X to LDS: stage t, row, 16-byte chunk c at position c ^ (row % 16) ----
+  {
+    const char* xsrc = uniform_ptr((const char*)p.x + (int64_t)kbase * 2);
+#pragma unroll
+    for (int j = 0; j < L::kPerWave; ++j) {
+      const int i = j * L::WAVES + wave;  // KiB: stage i / (4 PM), rows 4 (i % (4 PM)) .. + 4
+      const int t = i / (4 * PM);
+      const int row = (i % (4 * PM)) * 4 + (lane >> 4);
+      // rows past m re-read row m - 1 and are never stored
+      const uint32_t off = (uint32_t)min(row, p.m - 1) * (uint32_t)(p.ldx * 2) +
+                           (uint32_t)(t * 256 + (((lane & 15) ^ (row & 15)) * 16));
+      lds_dma16(xsrc + off, smem + i * 1024);
+    }
+  }
+  __asm__ __volatile__("" ::: "memory");  // the X copies are older than the weight loads
+  // ---- weights: bytes 128 t + 64 h + 16 g of row r of each subtile feed k-steps 2 h, 2 h + 1 ----
+  u32x4 wf[KT][2][NPW];
+  {
+    const char* wsrc = (const char*)p.w + (int64_t)(n0 + r) * p.k + kbase + 16 * g;
+#pragma unroll
+    for (int t = 0; t < KT; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int ns = 0; ns < NPW; ++ns)
+          wf[t][h][ns] = *(const u32x4*)(wsrc + (int64_t)ns * 16 * p.k + t * 128 + 64 * h);
+  }
+  __asm__ __volatile__("" ::: "memory");
+  // EPI 4: wave w finishes rows w, w + WAVES, .. of the head; their slots and positions
+  // (scalar loads) now, their RoPE values behind the weights
+  constexpr int N = EPI == 4 ? L::kRows / L::WAVES : 1;
+  const int head = blockIdx.x;
+  int64_t slot_e[N];
+  int pos_e[N];
+  if constexpr (EPI == 4) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int m = min(wave + L::WAVES * i, p.m - 1);
+      slot_e[i] = ((const ConstI32*)qa.slot_mapping)[m];
+      pos_e[i] = ((const ConstI32*)qa.positions)[m];
+    }
+  }
+  wait_vmcnt<L::kLoads>();  // this wave's X copies have landed
+  asm volatile("s_barrier" ::: "memory");
+  uint16_t rc_e[N], rs_e[N], nw_e[2] = {0, 0};
+  if constexpr (EPI == 4) {
+    const uint16_t* w = head < qa.hq ? qa.q_norm_w : qa.k_norm_w;  // v heads do not use it
+    nw_e[0] = w[lane];
+    nw_e[1] = w[lane + 64];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int64_t pos = min(max(pos_e[i], 0), qa.rope_positions - 1);
+      rc_e[i] = qa.rope[pos * 128 + lane];
+      rs_e[i] = qa.rope[pos * 128 + 64 + lane];
+    }
+  }
+  // the weight rows' scales as they are, behind the weights too (converted at the end: a
+  // conversion here would wait for every load)
+  uint32_t raw_sc[NPW][4];
+#pragma unroll
+  for (int ns = 0; ns < NPW; ++ns)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int at = n0 + 4 * g + ns * 16 + i;
+      raw_sc[ns][i] = p.scale_dtype == NE_DTYPE_FP32 ? ((const uint32_t*)p.scale)[at] : ((const uint16_t*)p.scale)[at];
+    }
+
+  floatx4 acc[KG][PM][NPW];
+#pragma unroll
+  for (int q = 0; q < KG; ++q)
+#pragma unroll
+    for (int mi = 0; mi < PM; ++mi)
+#pragma unroll
+      for (int ns = 0; ns < NPW; ++ns) acc[q][mi][ns] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < KT; ++t)
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      u32x4 xf[PM];
+#pragma unroll
+      for (int mi = 0; mi < PM; ++mi)
+        xf[mi] = *(const u32x4*)(smem + t * L::kStage + (mi * 16 + r) * 256 +
+                                 (((8 * (kk >> 1) + 2 * g + (kk & 1)) ^ r) * 16));
+#pragma unroll
+      for (int ns = 0; ns < NPW; ++ns) {
+        const u32x4 w = wf[t][kk >> 1][ns];
+        const bf16x8 a = int8x8_to_bf16x8(w[2 * (kk & 1)], w[2 * (kk & 1) + 1]);
+#pragma unroll
+        for (int mi = 0; mi < PM; ++mi)
+          acc[kk * KG / 4][mi][ns] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a, __builtin_bit_cast(bf16x8, xf[mi]), acc[kk * KG / 4][mi][ns], 0, 0, 0);
+      }
+    }
+
+  float sc[NPW][4];
+#pragma unroll
+  for (int ns = 0; ns < NPW; ++ns)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t b = raw_sc[ns][i];
+      sc[ns][i] = p.scale_dtype == NE_DTYPE_FP32   ? __uint_as_float(b)
+                  : p.scale_dtype == NE_DTYPE_BF16 ? bf16_to_f32((uint16_t)b)
+                                                   : f16_to_f32((uint16_t)b);
+    }
+  floatx4 v[PM][NPW];
+#pragma unroll
+  for (int mi = 0; mi < PM; ++mi)
+#pragma unroll
+    for (int ns = 0; ns < NPW; ++ns) {
+      v[mi][ns] = acc[0][mi][ns];
+#pragma unroll
+      for (int q = 1; q < KG; ++q) v[mi][ns] += acc[q][mi][ns];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if constexpr (EPI != 1) v[mi][ns][i] *= sc[ns][i];
+    }
+
+  if constexpr (EPI == 4) {
+    // the head's rows through LDS (fp32 [row][128 + 4], over X once every wave has read it),
+    // then wave w takes rows w, w + WAVES, .. as the row kernel does
+    static_assert(NPW == 1 && L::WAVES == 8, "one head per work-group");
+    constexpr int kRowF = 132;
+    static_assert(L::kRows * kRowF * 4 <= L::kX, "the rows fit over X");
+    float* rows = (float*)smem;
+    lds_barrier();
+#pragma unroll
+    for (int mi = 0; mi < PM; ++mi) *(floatx4*)(rows + (mi * 16 + r) * kRowF + wave * 16 + 4 * g) = v[mi][0];
+    lds_barrier();
+    int rows_e[N];
+    bool valid_e[N];
+    float a_e[N], b_e[N], c_e[N], s_e[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      rows_e[i] = wave + L::WAVES * i;
+      valid_e[i] = rows_e[i] < p.m;
+      a_e[i] = bf16_round(rows[rows_e[i] * kRowF + lane]);
+      b_e[i] = bf16_round(rows[rows_e[i] * kRowF + 64 + lane]);
+      c_e[i] = bf16_to_f32(rc_e[i]);
+      s_e[i] = bf16_to_f32(rs_e[i]);
+    }
+    qk_norm_rope_kv_vectors<(KV >= 2), KV == 3 ? NE_DTYPE_FP16 : NE_DTYPE_BF16, N>(
+        qa, rows_e, valid_e, head, lane, a_e, b_e, slot_e, bf16_to_f32(nw_e[0]), bf16_to_f32(nw_e[1]), c_e, s_e);
+    return;
+  }
+#pragma unroll
+  for (int mi = 0; mi < PM; ++mi) {
+    const int m = mi * 16 + r;
+    if (m >= p.m) continue;
+    if constexpr (EPI == 0) {
+#pragma unroll
+      for (int ns = 0; ns < NPW; ++ns)
+        *(u32x2*)(p.y + (int64_t)m * p.ldy + n0 + ns * 16 + 4 * g) =
+            u32x2{pack_bf16x2(v[mi][ns][0], v[mi][ns][1]), pack_bf16x2(v[mi][ns][2], v[mi][ns][3])};
+    } else if constexpr (EPI == 1) {
+      static_assert(NPW == 2, "a wave holds paired gate / up subtiles");
+      *(u32x2*)(p.y + (int64_t)m * p.ldy + n0 / 2 + 4 * g) = swiglu4(v[mi][0], v[mi][1], sc[0], sc[1]);
+    } else {
+#pragma unroll
+      for (int ns = 0; ns < NPW; ++ns)
+        *(floatx4*)(partial + ((int64_t)blockIdx.y * p.m + m) * p.n + n0 + ns * 16 + 4 * g) = v[mi][ns];
+    }
+  }
+}
+
+template <typename L, int EPI, int KV>
+int launch_few_as(const GemmParams& p, int splits, float* partial, hipStream_t stream, const char* name,
+                  const QkvRopeArgs& qa) {
+  static const hipError_t attr = hipFuncSetAttribute((const void*)proj_few_rows_kernel<L, EPI, KV>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, L::kX);
+  if (attr != hipSuccess) {
+    set_error("%s: cannot reserve %d bytes of LDS: %s", name, L::kX, hipGetErrorString(attr));
+    return NE_ELAUNCH;
+  }
+  hipLaunchKernelGGL((proj_few_rows_kernel<L, EPI, KV>),
+                     dim3((unsigned)(p.n / (L::WAVES * L::NPW * 16)), (unsigned)splits), dim3(L::WAVES * kWave), L::kX,
+                     stream, p, partial, qa);
+  return check_launch(name);
+}
+
 // Wave layouts (k-groups, weight subtiles per wave).  The plain and split-K products and
 // the fused QKV projection share two k-groups, so the fused epilogue sums every output in
 // the order the plain GEMM does and both round to the same bits; SwiGLU pairs gate and
@@ -1197,6 +1414,26 @@ int launch_proj_tile(ProjTile tile, const GemmParams& p, hipStream_t s, const ch
 constexpr int kKgPlain = 2, kNpwPlain = 1;
 constexpr int kKgQkv = 2, kNpwQkv = 2;
 constexpr int kKgSwiglu = 4, kNpwSwiglu = 2;
+
+// Whether the few-rows kernel serves a product: one token subtile, and a K (per split) of
+// 1,024 (or 512 / 768 of a split one), i.e. 8, 4 or 6 stages.  With three subtiles it lost to
+// the staged kernel at 48 rows (QKV 10.4 -> 12.2 us, gate|up 8.2 -> 9.4, down 5.6 -> 6.8:
+// every wave then waits for 96 KB of X before its first product).
+bool few_rows(const GemmParams& p, int splits) {
+  const int kt = p.k / splits / kStageK;
+  return p.m <= 16 && (splits > 1 ? kt == 4 || kt == 6 || kt == 8 : kt == 8);
+}
+
+template <int NPW, int KG, int WAVES, int EPI, int KV>
+int launch_few(const GemmParams& p, int splits, float* partial, hipStream_t s, const char* name,
+               const QkvRopeArgs& qa = QkvRopeArgs{}) {
+  const int kt = p.k / splits / kStageK;
+  if constexpr (EPI == 3) {
+    if (kt == 4) return launch_few_as<FewLayout<1, NPW, KG, WAVES, 4>, EPI, KV>(p, splits, partial, s, name, qa);
+    if (kt == 6) return launch_few_as<FewLayout<1, NPW, KG, WAVES, 6>, EPI, KV>(p, splits, partial, s, name, qa);
+  }
+  return launch_few_as<FewLayout<1, NPW, KG, WAVES, 8>, EPI, KV>(p, splits, partial, s, name, qa);
+}
 
 template <int SDT>
 int dispatch_qkv_fused(GemmParams p, const QkvRopeArgs& qa, int kv_mode, hipStream_t s) {
@@ -1207,6 +1444,11 @@ int dispatch_qkv_fused(GemmParams p, const QkvRopeArgs& qa, int kv_mode, hipStre
     if (kv_mode == 1) return launch_proj_tile<4, 1>(tile, p, s, "w8a16_qkv_norm_rope_kv", qa);
     if (kv_mode == 2) return launch_proj_tile<4, 2>(tile, p, s, "w8a16_qkv_norm_rope_kv", qa);
     return launch_proj_tile<4, 3>(tile, p, s, "w8a16_qkv_norm_rope_kv", qa);
+  }
+  if (few_rows(p, 1)) {
+    if (kv_mode == 1) return launch_few<1, kKgQkv, 8, 4, 1>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
+    if (kv_mode == 2) return launch_few<1, kKgQkv, 8, 4, 2>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
+    return launch_few<1, kKgQkv, 8, 4, 3>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
   }
   switch (kv_mode) {
     // 48-row tiles: 7 x 32 = 224 work-groups for 320 rows, 3 rows per wave in the epilogue
@@ -1223,6 +1465,11 @@ int dispatch_w8a16(GemmParams p, int epilogue, int splits, float* partial, hipSt
     const ProjTile tile = choose_proj_tile(p.m, p.n, swiglu);
     if (tile != ProjTile::kVerify)
       return swiglu ? launch_proj_tile<1, 0>(tile, p, s, "w8a16_swiglu") : launch_proj_tile<0, 0>(tile, p, s, "w8a16_gemm");
+  }
+  if (few_rows(p, partial != nullptr ? splits : 1)) {
+    if (epilogue == NE_EPILOGUE_SWIGLU) return launch_few<2, kKgSwiglu, 2, 1, 0>(p, 1, nullptr, s, "w8a16_swiglu");
+    if (partial != nullptr) return launch_few<1, kKgPlain, 2, 3, 0>(p, splits, partial, s, "w8a16_splitk");
+    return launch_few<1, kKgPlain, 2, 0, 0>(p, 1, nullptr, s, "w8a16_gemm");
   }
   if (epilogue == NE_EPILOGUE_SWIGLU) {
     if (p.n % 96 == 0)

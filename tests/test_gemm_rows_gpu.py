@@ -137,3 +137,47 @@ def test_outputs_of_every_row_alignment(device, m, pad, first):
         call(x, view[:, :n])
         assert torch.equal(view[:, :n], plain)
         assert not view[:, n:].any() and not flat[:first].any() and not flat[first + rows * ld:].any()
+
+
+@pytest.mark.parametrize("m", [1, 5, 16, 17])
+def test_few_rows_give_the_bits_of_many(device, m):
+    """Up to 16 rows run their own kernel; it adds every output in the order of the kernel
+    that 320 rows run, so a row's results do not depend on how many there are: plain,
+    SwiGLU, split-K (K 512, 768 and 1,024 a split) and, with the cache, the fused QKV."""
+    g = torch.Generator(device=device).manual_seed(m)
+    for n, k, splits in ((4096, 1024, 0), (1024, 2048, 4), (1024, 3072, 4), (1024, 2048, 2)):
+        for scale_dtype in (torch.bfloat16, torch.float16, torch.float32):
+            w, s = weight(n, k, device, scale_dtype)
+            x = torch.randn(320, k, device=device, generator=g).to(torch.bfloat16)
+            if splits:
+                few = kernels.w8a16_gemm_splitk(x[:m], w, s, splits)
+                many = kernels.w8a16_gemm_splitk(x, w, s, splits)
+                assert torch.equal(few.view(splits, m, n), many.view(splits, 320, n)[:, :m])
+            else:
+                assert torch.equal(kernels.w8a16_gemm(x[:m], w, s), kernels.w8a16_gemm(x, w, s)[:m])
+    w, s = weight(6144, 1024, device)
+    x = torch.randn(320, 1024, device=device, generator=g).to(torch.bfloat16)
+    assert torch.equal(kernels.w8a16_gemm(x[:m], w, s, epilogue=EPILOGUE_SWIGLU),
+                       kernels.w8a16_gemm(x, w, s, epilogue=EPILOGUE_SWIGLU)[:m])
+    w, s = weight(4096, 1024, device)
+    norms = [(1 + 0.1 * torch.randn(128, device=device, generator=g)).to(torch.bfloat16) for _ in range(2)]
+    positions = torch.randint(0, 3000, (320,), generator=g, dtype=torch.int32, device=device)
+    rope = kernels.rope_table(3000, 1e6).to(device)
+    slots = torch.randperm(400, generator=g, device=device)[:320].to(torch.int32)
+    for dtype in (torch.int8, torch.bfloat16):
+        results = []
+        for rows in (m, 320):
+            caches = [torch.zeros(400, 8, 128, dtype=dtype, device=device) for _ in range(2)]
+            scales = [torch.zeros(400, 8, dtype=torch.bfloat16, device=device) for _ in range(2)]
+            q = torch.zeros(rows + 1, 16, 128, dtype=torch.bfloat16, device=device)
+            kernels.w8a16_qkv_norm_rope_kv(x[:rows], w, s, 16, 8, *norms, 1e-6, positions[:rows], rope, slots[:rows],
+                                           *caches, *(scales if dtype == torch.int8 else (None, None)), q_out=q[:rows])
+            assert not q[rows].any()
+            mine = slots[:m].long()
+            results.append([q[:m]] + [c[mine] for c in caches] + [t[mine] for t in scales])
+            if rows == m:
+                other = torch.ones(400, dtype=torch.bool, device=device)
+                other[mine] = False
+                assert not any(c[other].any() for c in caches)
+        for a, b in zip(*results):
+            assert torch.equal(a, b)
