@@ -34,11 +34,11 @@ struct GemmParams {
   const void* w;
   const void* scale;
   int m, n, k;
+  int scale_dtype;   // of the projections' row scales
   uint16_t* y;
   int64_t ldy;
   uint64_t* argmax;  // [m][n / BN] packed (ordered value, ~index)
   int tiles_m, tiles_n;
-  int scale_dtype;   // of the projections' row scales
 };
 
 __device__ __forceinline__ float sbyte(uint32_t w, int k) { return (float)(int8_t)(w >> (8 * k)); }
