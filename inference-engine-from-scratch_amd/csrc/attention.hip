@@ -20,6 +20,8 @@
 //           heads, one M tile) sizes the splits from a work plan that every
 //           work-group derives from the context lengths (plan_item); the register
 //           kernels use fixed `split_len` splits.
+//           Prefill (more than 32 rows per KV head) runs a kernel of its own, one KV
+//           head of a tile of query rows per work-group (paged_attention_rows_kernel).
 //   merge = splits store fp32 partials (reference max, sum, unnormalised output;
 //           real rows only) and a second kernel combines them.  No fences or
 //           atomics order the work-groups: the kernel boundary does, which on an
