@@ -1200,8 +1200,8 @@ int launch_proj_tile(ProjTile tile, const GemmParams& p, hipStream_t s, const ch
 //   sums  = KG accumulators per output (k-step kk of a stage goes to accumulator kk KG / 4),
 //           added in order: the k-groups of the kernel above, so the results are its bits
 // Measured at 5 rows (kernel trace, fastest of 28; us, before -> here): QKV 8.7 -> 7.8,
-// gate|up 7.0 -> 6.4, o 4.5 -> 2.9, down 4.6 -> 3.9; four layers from a HIP graph 176.7 ->
-// 167.2.  What is left is the launch, one round trip to HBM and, for QKV, 128 KB of weights
+// gate|up 7.0 -> 6.4, o 4.5 -> 2.9, down 4.6 -> 3.9; four layers from a HIP graph 174-177
+// -> 167-171.  What is left is the launch, one round trip to HBM and, for QKV, 128 KB of weights
 // into each of 32 CUs.
 template <int PM_, int NPW_, int KG_, int WAVES_, int KT_>
 struct FewLayout {
