@@ -1083,9 +1083,7 @@ struct QtItem {
 
 __device__ __forceinline__ QtItem qt_item(const AttnParams& p, int seq, int tile, int tile_rows) {
   QtItem it;
-  // a context beyond the caller's bound is clipped to it (and flagged by the kernel), so
-  // that no block-table entry past max_ctx is read
-  it.ctx = min(((const ConstI32*)p.ctx_len)[seq], p.max_ctx);
+  it.ctx = ((const ConstI32*)p.ctx_len)[seq];
   it.ql = ((const ConstI32*)p.q_len)[seq];
   it.qs = ((const ConstI32*)p.q_start)[seq];
   it.rows_total = p.group * it.ql;
@@ -1094,7 +1092,9 @@ __device__ __forceinline__ QtItem qt_item(const AttnParams& p, int seq, int tile
   it.n_splits = 0;
   if (it.row0 < it.rows_total) {
     const int last = (min(it.row0 + tile_rows, it.rows_total) - 1) / p.group;  // last query of the tile
-    it.kend = it.ctx - it.ql + last + 1;
+    // keys past the caller's bound are dropped (and the context flagged by the kernel): no
+    // block-table entry beyond it is read; the queries keep their positions
+    it.kend = min(it.ctx - it.ql + last + 1, p.max_ctx);
     it.n_splits = it.kend > 0 ? min((it.kend + p.split_len - 1) / p.split_len, p.max_splits) : 0;
   }
   return it;

@@ -149,6 +149,30 @@ def test_context_past_the_bound_is_flagged(device):
     assert ws.error_flag() != 0
 
 
+# contexts past the bound: the first rows see keys up to their own position, the others those
+# below the bound; a bound shorter than the queries
+@pytest.mark.parametrize("kv", ["bf16", "int8"])
+@pytest.mark.parametrize("q_lens,ctx_lens,bound", [([40, 40], [500, 60], 400), ([300, 70], [330, 70], 200)])
+def test_keys_past_the_bound_are_dropped(device, kv, q_lens, ctx_lens, bound):
+    ws = kernels.AttentionWorkspace()
+    kc, vc, ks, vs = make_pool(64, 16, 8, kv)
+    tables, ctx, qs, ql, rows = make_batch(ctx_lens, q_lens, 64, 16)
+    q = torch.randn(rows, 16, 128, generator=torch.Generator().manual_seed(51)).to(torch.bfloat16)
+    # every query as a sequence of its own, which sees min(position + 1, bound) keys
+    seq = torch.repeat_interleave(torch.arange(len(q_lens)), ql.long())
+    position = torch.cat([torch.arange(c - n, c) for c, n in zip(ctx_lens, q_lens)])
+    seen = (position + 1).clamp(max=bound).to(torch.int32)
+    ref = paged_attention_reference(q, kc, vc, ks, vs, tables[seq], 16, seen, torch.arange(rows, dtype=torch.int32),
+                                    torch.ones(rows, dtype=torch.int32), model_dtype=torch.bfloat16)
+    d = lambda t: None if t is None else t.to(device)
+    args = [d(t) for t in (q, kc, vc, ks, vs, tables)] + [16] + [d(t) for t in (ctx, qs, ql)]
+    kernels.paged_verify_attention(*args, max_q_len=max(q_lens), max_ctx_len=max(ctx_lens), workspace=ws)
+    assert ws.error_flag() == 0
+    got = kernels.paged_verify_attention(*args, max_q_len=max(q_lens), max_ctx_len=bound, workspace=ws)
+    assert ws.error_flag() != 0
+    assert rel_err(got, ref) < TOL
+
+
 def test_workspace_holds_partials_only_where_the_keys_are_split(device):
     size = _native.load().ne_paged_attention_workspace_size
     assert size(1, 16, 8, 8192, 16384, 0) == 256  # 512 tiles: no split
