@@ -105,6 +105,10 @@ struct AttnParams {
   int32_t max_ctx;     // the caller's bound on ctx_len
   int32_t rows_kg;     // query-tile kernel: key groups per work-group (0: another kernel serves the call)
   int32_t row_tiles;   // query-tile kernel: tiles of query rows per sequence
+  int32_t row_slots;   // query-tile kernel: partials of split tiles (0: no splits)
+  int32_t row_share;   // query-tile kernel: least stages per work-group of a split tile
+  int32_t row_extra;   // query-tile kernel: work-groups for the parts after a tile's first
+  int32_t* rows_list;  // query-tile kernel: the split tiles' merges, [1 + row_slots / 2][kQtListInts], the count first
   int32_t* plan_desc;  // precomputed plan: [plan_grid][8] work items (seq < 0: none)
   int32_t* plan_slots; // precomputed plan: [plan_grid][kPlanMaxTiles] first slot of each tile
 };
@@ -839,10 +843,31 @@ constexpr int kQtStage = 2 * kQtTileBytes;
 constexpr int kQtScaleOff = 2 * kQtStage;        // float [2 buffers][K | V][128 keys]
 constexpr int kQtSlotOff = kQtScaleOff + 2 * 2 * kQtKeys * 4;  // int [2][8 tiles]
 constexpr int kQtFlagOff = kQtSlotOff + 2 * 8 * 4;             // int [2 buffers][2 waves]
-constexpr int kQtLds = kQtFlagOff + 2 * 2 * 4;
+constexpr int kQtScanOff = kQtFlagOff + 2 * 2 * 4;             // int [3][8 waves], [4]
+constexpr int kQtLds = kQtScanOff + 28 * 4;
 static_assert(kQtLds <= 160 * 1024, "LDS of one CU");
 
-constexpr int kQtMinSplit = 256;                 // keys: a shorter split is mostly prologue and partials
+// Key splits.  A tile's work is its stages of keys; with T stages in the batch (all tiles of
+// all heads), a work-group's share is S = ceil(T / 256), at least row_share stages, and a tile
+// of n >= 1.5 S stages is cut into n / S parts, rounded to nearest: at most 4/3 n / S of them,
+// so 341 in all and 256 beside the tiles' first ones.  The sequences' lengths decide and not
+// the call's bounds, because a batch is seldom even: splits of the bounds left the tail of a
+// long prompt beside short prompts, or one long sequence in a graph's many slots, to one
+// work-group per head (us, int8, bounds -> lengths): 100 queries after 15,900 keys beside
+// twelve prompts of 300 522 -> 69, 64 slots of 17 queries with one sequence of 16,384 keys
+// 253 -> 44 (the fixed-split kernel: 208 and 50), eight times 64 queries after 0-6,000 keys
+// 47 -> 32.
+// Every work-group derives S from the lengths (a load per thread, a sum in registers and one
+// in LDS, under the first loads).  A tile's own work-group serves its first part, which needs S
+// only to know where to end; the other parts have work-groups at the end of the grid, so that
+// those without a part (most calls split nothing) leave while the last tiles run.  In front of
+// the tiles they balance a little better (63 instead of 69 us above) and cost every call
+// ~3 us; as a second pass of the tiles' own work-groups they cost the main loop 13 % (the
+// lane addresses of both passes held in registers or computed again).
+constexpr int kQtMinSplitStages = 2;             // a shorter part is mostly prologue and partials
+constexpr int kQtManySplitStages = 4;            // where the tiles may fill the chip: tiles of up to 5 need no S
+constexpr int kQtMaxSlots = 4 * kNumCu / 3;      // parts of split tiles, each with a partial's room
+constexpr int kQtListInts = 8;                   // sequence, tile, head, first slot, parts of a merge
 
 constexpr int qt_rows(int kg) { return kQtWaveRows * kQtWaves / kg; }
 
@@ -1076,28 +1101,166 @@ __device__ __forceinline__ void qt_step(const char* smem, int buf, int u, int kb
   }
 }
 
-// Rows, keys and splits of one (sequence, query tile); the same in the merge kernel.
+// Rows and keys of one (sequence, query tile).
 struct QtItem {
-  int ctx, ql, qs, row0, rows_total, kend, n_splits;
+  int ctx, ql, row0, rows_total, kend, stages;
 };
 
-__device__ __forceinline__ QtItem qt_item(const AttnParams& p, int seq, int tile, int tile_rows) {
+// ... of a sequence of ctx keys and ql queries
+__device__ __forceinline__ QtItem qt_item_of(const AttnParams& p, int ctx, int ql, int tile, int tile_rows) {
   QtItem it;
-  it.ctx = ((const ConstI32*)p.ctx_len)[seq];
-  it.ql = ((const ConstI32*)p.q_len)[seq];
-  it.qs = ((const ConstI32*)p.q_start)[seq];
-  it.rows_total = p.group * it.ql;
+  it.ctx = ctx;
+  it.ql = ql;
+  it.rows_total = p.group * ql;
   it.row0 = tile * tile_rows;
   it.kend = 0;
-  it.n_splits = 0;
+  it.stages = 0;
   if (it.row0 < it.rows_total) {
     const int last = (min(it.row0 + tile_rows, it.rows_total) - 1) / p.group;  // last query of the tile
     // keys past the caller's bound are dropped (and the context flagged by the kernel): no
     // block-table entry beyond it is read; the queries keep their positions
-    it.kend = min(it.ctx - it.ql + last + 1, p.max_ctx);
-    it.n_splits = it.kend > 0 ? min((it.kend + p.split_len - 1) / p.split_len, p.max_splits) : 0;
+    it.kend = min(ctx - ql + last + 1, p.max_ctx);
+    it.stages = it.kend > 0 ? (it.kend - 1) / kQtKeys + 1 : 0;
   }
   return it;
+}
+
+__device__ __forceinline__ QtItem qt_item(const AttnParams& p, int seq, int tile, int tile_rows) {
+  return qt_item_of(p, ((const ConstI32*)p.ctx_len)[seq], ((const ConstI32*)p.q_len)[seq], tile, tile_rows);
+}
+
+// Parts of a tile of n stages when a work-group's share is S.
+__device__ __forceinline__ int qt_parts(int n, int S) { return 2 * (int64_t)n >= 3 * (int64_t)S ? (n + S / 2) / S : 1; }
+
+// The batch's tiles f = sequence * row_tiles + tile, a consecutive range for each thread (one
+// tile, up to kQtThreads of them), and the lengths of the first one's sequence.
+struct QtTiles {
+  int begin, end, ctx, ql;
+};
+__device__ __forceinline__ QtTiles qt_my_tiles(const AttnParams& p) {
+  const int tiles = p.num_seqs * p.row_tiles;
+  const int per = (tiles + kQtThreads - 1) / kQtThreads;
+  QtTiles my;
+  my.begin = min(tiles, (int)threadIdx.x * per);
+  my.end = min(tiles, my.begin + per);
+  const int seq = min(my.begin, tiles - 1) / p.row_tiles;
+  my.ctx = p.ctx_len[seq];
+  my.ql = p.q_len[seq];
+  return my;
+}
+// Calls fn(tile, its stages) for the thread's tiles.
+template <typename F>
+__device__ __forceinline__ void qt_each(const AttnParams& p, const QtTiles& my, int tile_rows, F fn) {
+  int ctx = my.ctx, ql = my.ql;
+  for (int f = my.begin; f < my.end; ++f) {
+    const int seq = f / p.row_tiles;
+    if (f > my.begin) {
+      ctx = p.ctx_len[seq];
+      ql = p.q_len[seq];
+    }
+    fn(f, qt_item_of(p, ctx, ql, f - seq * p.row_tiles, tile_rows).stages);
+  }
+}
+
+// S in two steps, called by all threads of the work-group with a barrier between them: the
+// waves' sums and longest tiles to LDS, and S from them.
+__device__ __forceinline__ void qt_sum_stages(const AttnParams& p, const QtTiles& my, int tile_rows, int wave, int lane,
+                                              int* s_sum) {
+  int sum = 0, most = 0;  // the host bounds the batch's stages to 31 bits
+  qt_each(p, my, tile_rows, [&](int, int n) {
+    sum += n;
+    most = max(most, n);
+  });
+  auto step = [&](auto ctrl) {
+    constexpr int C = decltype(ctrl)::value;
+    sum += __builtin_amdgcn_mov_dpp(sum, C, 0xF, 0xF, false);
+    most = max(most, __builtin_amdgcn_mov_dpp(most, C, 0xF, 0xF, false));
+  };
+  step(std::integral_constant<int, 0xB1>{});   // quad_perm [1, 0, 3, 2]
+  step(std::integral_constant<int, 0x4E>{});   // quad_perm [2, 3, 0, 1]
+  step(std::integral_constant<int, 0x141>{});  // row_half_mirror
+  step(std::integral_constant<int, 0x140>{});  // row_mirror
+  int total = 0, longest = 0;
+#pragma unroll
+  for (int row = 0; row < kWave; row += 16) {
+    total += __builtin_amdgcn_readlane(sum, row);
+    longest = max(longest, __builtin_amdgcn_readlane(most, row));
+  }
+  if (lane == 0) {
+    s_sum[wave] = total;
+    s_sum[kQtWaves + wave] = longest;
+  }
+}
+__device__ __forceinline__ int qt_share(const AttnParams& p, const int* s_sum, int& longest) {
+  int64_t sum = 0;
+  longest = 0;
+#pragma unroll
+  for (int w = 0; w < kQtWaves; ++w) {
+    sum += s_sum[w];
+    longest = max(longest, s_sum[kQtWaves + w]);
+  }
+  longest = __builtin_amdgcn_readfirstlane(longest);
+  const int64_t share = (sum * p.num_kv_heads + kNumCu - 1) / kNumCu;
+  return __builtin_amdgcn_readfirstlane((int)min(max(share, (int64_t)p.row_share), (int64_t)1 << 30));
+}
+
+// Finds one split tile among the batch's: the one whose parts after the first hold number
+// `extra` (in the order of the tiles), or tile number `want` if that is split.  Called by all
+// threads of the work-group; s_scan: 12 ints.  False when there is none.
+struct QtSplit {
+  int tile;          // f
+  int parts;         // its parts
+  int parts_before;  // parts and split tiles before it
+  int tiles_before;
+  int tiles_total;   // split tiles of the batch
+};
+__device__ bool qt_find_split(const AttnParams& p, const QtTiles& my, int tile_rows, int S, int extra, int want,
+                              int wave, int lane, int* s_scan, QtSplit& out) {
+  // parts in the low half, split tiles in the high half: at most kQtMaxSlots of them
+  int mine = 0;
+  qt_each(p, my, tile_rows, [&](int, int stages) {
+    const int n = qt_parts(stages, S);
+    if (n > 1) mine += n + (1 << 16);
+  });
+  int incl = mine;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int below = __shfl_up(incl, o);
+    if (lane >= o) incl += below;
+  }
+  if (lane == kWave - 1) s_scan[wave] = incl;
+  int* found = s_scan + kQtWaves;
+  if (threadIdx.x == 0) found[0] = -1;
+  __syncthreads();
+  int before = incl - mine, total = 0;
+#pragma unroll
+  for (int w = 0; w < kQtWaves; ++w) {
+    if (w < wave) before += s_scan[w];
+    total += s_scan[w];
+  }
+  out.tiles_total = __builtin_amdgcn_readfirstlane(total >> 16);
+  if (mine != 0) {
+    int parts = before & 0xFFFF, tiles = before >> 16;
+    qt_each(p, my, tile_rows, [&](int f, int stages) {
+      const int n = qt_parts(stages, S);
+      if (n <= 1) return;
+      const int at = parts - tiles;  // parts after the first ones, before this tile's
+      if (want >= 0 ? f == want : (extra >= at && extra < at + n - 1)) {
+        found[0] = f;
+        found[1] = n;
+        found[2] = parts;
+        found[3] = tiles;
+      }
+      parts += n;
+      ++tiles;
+    });
+  }
+  __syncthreads();
+  out.tile = __builtin_amdgcn_readfirstlane(found[0]);
+  out.parts = __builtin_amdgcn_readfirstlane(found[1]);
+  out.parts_before = __builtin_amdgcn_readfirstlane(found[2]);
+  out.tiles_before = __builtin_amdgcn_readfirstlane(found[3]);
+  return out.tile >= 0;
 }
 
 template <bool INT8, int SDT, int KG>
@@ -1109,63 +1272,103 @@ __global__ __launch_bounds__(kQtThreads) void paged_attention_rows_kernel(AttnPa
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int lane = tid % kWave;
 
-  // ---- work item: KV head fastest, then the sequence, the tiles from the last down ----
-  int b = blockIdx.x;
-  const int head = b % p.num_kv_heads;
-  b /= p.num_kv_heads;
-  const int split = b % p.max_splits;
-  b /= p.max_splits;
-  const int seq = b % p.num_seqs;
-  const int tile = p.row_tiles - 1 - b / p.num_seqs;
+  // ---- work item: a tile, or its first part (KV head fastest, then the sequence, the tiles
+  // from the last down); behind the tiles, the further parts ----
+  const int tiles = p.num_seqs * p.row_tiles * p.num_kv_heads;
+  int* s_scan = (int*)(smem + kQtScanOff);
+  int seq, tile, head, part = 0, parts = 1, slot = 0;
+  if ((int)blockIdx.x < tiles) {
+    int b = blockIdx.x;
+    head = b % p.num_kv_heads;
+    b /= p.num_kv_heads;
+    seq = b % p.num_seqs;
+    tile = p.row_tiles - 1 - b / p.num_seqs;
+  } else {
+    const int x = blockIdx.x - tiles;
+    head = x % p.num_kv_heads;
+    const QtTiles my = qt_my_tiles(p);
+    qt_sum_stages(p, my, kTileRows_, wave, lane, s_scan);
+    __syncthreads();
+    int longest;
+    const int S = qt_share(p, s_scan, longest);
+    const int extra = x / p.num_kv_heads;
+    QtSplit sp{};
+    const bool any = qt_parts(longest, S) > 1 &&  // most calls split nothing
+                     qt_find_split(p, my, kTileRows_, S, extra, -1, wave, lane, s_scan + 2 * kQtWaves, sp);
+    if (x == 0 && tid == 0) p.rows_list[0] = sp.tiles_total * p.num_kv_heads;  // merges
+    if (!any) return;
+    seq = sp.tile / p.row_tiles;
+    tile = sp.tile % p.row_tiles;
+    part = extra - (sp.parts_before - sp.tiles_before) + 1;
+    parts = sp.parts;
+    slot = (sp.parts_before + part) * p.num_kv_heads + head;
+  }
   const QtItem it = qt_item(p, seq, tile, kTileRows_);
-  if (tid == 0 && ((const ConstI32*)p.ctx_len)[seq] > p.max_ctx) atomicOr(p.error_flag, 1u);
-  if (split >= it.n_splits) return;
-  const int kstart = split * p.split_len;
-  const int kend = min(it.kend, kstart + p.split_len);
-  const int n_stages = (kend - kstart + kQtKeys - 1) / kQtKeys;
+  const int qs = ((const ConstI32*)p.q_start)[seq];
+  if (it.stages == 0) return;
+  if (tid == 0 && it.ctx > p.max_ctx) atomicOr(p.error_flag, 1u);
+  const int kstart = (int)((int64_t)it.stages * part / parts) * kQtKeys;
+  // whether S decides where this tile's work-group ends
+  const bool whole = part == 0 && p.row_slots > 0 && qt_parts(it.stages, p.row_share) > 1;
 
   // ---- this wave's rows ----
   const int r = lane & 15;
   const int g = lane >> 4;
   const int kg = wave / kRowGroups;
   const int wrow0 = it.row0 + (wave % kRowGroups) * kQtWaveRows;
-  int kend_row[kQtMT];
   QtState<INT8> st;
-  int kend_wave = 0, kfull_wave = 0;  // keys some row of the wave sees; keys every row sees
-  if (wrow0 < it.rows_total) {
-    const int last = (min(wrow0 + kQtWaveRows, it.rows_total) - 1) / p.group;
-    kend_wave = min(kend, it.ctx - it.ql + last + 1);
-    kfull_wave = min(kend, it.ctx - it.ql + wrow0 / p.group + 1);
-  }
 
   // ---- stages of 128 keys ----
   // first slot of each 16-key tile of a stage, in a ring of two (read one stage before
-  // its data, by 8 threads); tiles past the last key re-read the last key's tile
+  // its data, by 8 threads); tiles past the tile's last key re-read its 16 keys
   int* s_slot = (int*)(smem + kQtSlotOff);
   const int32_t* bt = p.block_tables + (int64_t)seq * p.bt_stride;
   auto tile_slot = [&](int tile16) {
-    const int key = min(kstart + kTileKeys * tile16, (kend - 1) & ~(kTileKeys - 1));
+    const int key = min(kstart + kTileKeys * tile16, (it.kend - 1) & ~(kTileKeys - 1));
     return bt[key / p.block_size] * p.block_size + key % p.block_size;
   };
   // the first two stages' slots and this wave's Q rows are requested together; Q is
   // converted behind the first stage's loads
   int slot0 = 0;
   if (tid < 16) slot0 = tile_slot(tid);
+  QtTiles my{};
+  if (whole) my = qt_my_tiles(p);
+  __asm__ __volatile__("" ::: "memory");  // these loads are waited for before the Q rows
   u32x4 raw[kQtMT][4];
 #pragma unroll
   for (int mt = 0; mt < kQtMT; ++mt) {
     const int row = wrow0 + kRows * mt + r;
     const bool valid = row < it.rows_total;
     const int qi = valid ? row / p.group : 0;
-    kend_row[mt] = valid ? min(kend, it.ctx - it.ql + qi + 1) : kend;
     // a row past the last reads the sequence's first row; its results are never stored
-    const uint16_t* src = p.q + (int64_t)(it.qs + qi) * p.q_tok_stride +
+    const uint16_t* src = p.q + (int64_t)(qs + qi) * p.q_tok_stride +
                           (int64_t)(head * p.group + (valid ? row - qi * p.group : 0)) * p.q_head_stride + 8 * g;
 #pragma unroll
     for (int c = 0; c < 4; ++c) raw[mt][c] = *(const u32x4*)(src + 32 * c);
   }
+  if (whole) qt_sum_stages(p, my, kTileRows_, wave, lane, s_scan);
   if (tid < 16) s_slot[tid] = slot0;
   lds_barrier();
+  int S = 0;
+  if (whole) {
+    int longest;
+    S = qt_share(p, s_scan, longest);
+    parts = qt_parts(it.stages, S);
+  }
+  const int kend = min(it.kend, (int)((int64_t)it.stages * (part + 1) / parts) * kQtKeys);
+  const int n_stages = (kend - kstart + kQtKeys - 1) / kQtKeys;
+  int kend_wave = 0, kfull_wave = 0;  // keys some row of the wave sees; keys every row sees
+  if (wrow0 < it.rows_total) {
+    const int last = (min(wrow0 + kQtWaveRows, it.rows_total) - 1) / p.group;
+    kend_wave = min(kend, it.ctx - it.ql + last + 1);
+    kfull_wave = min(kend, it.ctx - it.ql + wrow0 / p.group + 1);
+  }
+  int kend_row[kQtMT];
+#pragma unroll
+  for (int mt = 0; mt < kQtMT; ++mt) {
+    const int row = wrow0 + kRows * mt + r;
+    kend_row[mt] = row < it.rows_total ? min(kend, it.ctx - it.ql + row / p.group + 1) : kend;
+  }
   QtRegs<INT8> R;
   qt_load<INT8, SDT>(p, s_slot, kstart, kend, head, tid, R);
   __asm__ __volatile__("" ::: "memory");
@@ -1221,6 +1424,21 @@ __global__ __launch_bounds__(kQtThreads) void paged_attention_rows_kernel(AttnPa
     __syncthreads();
   }
 
+  // a split tile's own work-group: the slot of its partial, and the tile's entry in the list of merges
+  if (whole && parts > 1) {
+    QtSplit sp;
+    qt_find_split(p, qt_my_tiles(p), kTileRows_, S, 0, seq * p.row_tiles + tile, wave, lane, s_scan + 2 * kQtWaves, sp);
+    slot = sp.parts_before * p.num_kv_heads + head;
+    if (tid == 0) {
+      int32_t* list = p.rows_list + (sp.tiles_before * p.num_kv_heads + head + 1) * kQtListInts;
+      list[0] = seq;
+      list[1] = tile;
+      list[2] = head;
+      list[3] = slot;
+      list[4] = parts;
+    }
+  }
+
   // ---- merge the key groups through LDS (the stages are done) ----
 #pragma unroll
   for (int mt = 0; mt < kQtMT; ++mt) {
@@ -1265,9 +1483,9 @@ __global__ __launch_bounds__(kQtThreads) void paged_attention_rows_kernel(AttnPa
   for (int mt = 0; mt < kQtMT; ++mt) {
     const int row = wrow0 + kRows * mt + r;
     if (row >= it.rows_total) continue;
-    if (it.n_splits == 1) {
+    if (parts == 1) {
       const int qi = row / p.group;
-      uint16_t* dst = p.out + (int64_t)(it.qs + qi) * p.o_tok_stride +
+      uint16_t* dst = p.out + (int64_t)(qs + qi) * p.o_tok_stride +
                       (int64_t)(head * p.group + row - qi * p.group) * p.o_head_stride + 4 * g;
       const float inv = 1.f / st.l[mt];
 #pragma unroll
@@ -1275,8 +1493,7 @@ __global__ __launch_bounds__(kQtThreads) void paged_attention_rows_kernel(AttnPa
         *(u32x2*)(dst + 16 * j) = u32x2{pack_bf16x2(st.o[mt][j][0] * inv, st.o[mt][j][1] * inv),
                                         pack_bf16x2(st.o[mt][j][2] * inv, st.o[mt][j][3] * inv)};
     } else {
-      const int64_t part = (((int64_t)(seq * p.row_tiles + tile) * p.num_kv_heads + head) * p.max_splits + split) *
-                               kTileRows_ + row - it.row0;
+      const int64_t part = (int64_t)slot * kTileRows_ + row - it.row0;
       float* po = p.part_o + part * kHeadDim + 4 * g;
 #pragma unroll
       for (int j = 0; j < 8; ++j) *(floatx4*)(po + 16 * j) = st.o[mt][j];
@@ -2405,30 +2622,33 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnParams p) {
   merge_partials(p, n_splits, cd, [&](int s) { return ubase + (int64_t)s * kRows; }, dst);
 }
 
-// Combines the split partials of the query-tile kernel: one work-group per (sequence,
-// tile, KV head, 16 rows), 16 threads per row, 8 dims per thread.
+// Combines the parts' partials of the query-tile kernel's split tiles: 16 rows of a (tile, KV
+// head) at a time, 16 threads per row, 8 dims per thread.  The grid is bounded, since few of
+// the tiles that could be split are.
+constexpr int kQtMergeGrid = 4 * kNumCu;
 __global__ __launch_bounds__(256) void attention_rows_merge_kernel(AttnParams p, int tile_rows) {
   const int blocks = tile_rows / kRows;
-  int b = blockIdx.x;
-  const int row = (b % blocks) * kRows + (threadIdx.x >> 4);
-  b /= blocks;
-  const int head = b % p.num_kv_heads;
-  b /= p.num_kv_heads;
-  const int tile = b % p.row_tiles;
-  const int seq = b / p.row_tiles;
-  const QtItem it = qt_item(p, seq, tile, tile_rows);
-  if (it.n_splits <= 1 || it.row0 + row >= it.rows_total) return;
-  const int cd = (threadIdx.x & 15) * 8;
-  const int64_t base = ((int64_t)(seq * p.row_tiles + tile) * p.num_kv_heads + head) * p.max_splits * tile_rows + row;
-  const int qi = (it.row0 + row) / p.group;
-  uint16_t* dst = p.out + (int64_t)(it.qs + qi) * p.o_tok_stride +
-                  (int64_t)(head * p.group + it.row0 + row - qi * p.group) * p.o_head_stride + cd;
-  merge_partials(p, it.n_splits, cd, [&](int s) { return base + (int64_t)s * tile_rows; }, dst);
+  const ConstI32* all = (const ConstI32*)p.rows_list;  // written by the kernel before
+  const int items = all[0] * blocks;
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
+    const ConstI32* list = all + (1 + item / blocks) * kQtListInts;
+    const int seq = list[0], tile = list[1], head = list[2], slot = list[3], parts = list[4];
+    const int row = item % blocks * kRows + (threadIdx.x >> 4);
+    const QtItem it = qt_item(p, seq, tile, tile_rows);
+    if (it.row0 + row >= it.rows_total) continue;
+    const int cd = (threadIdx.x & 15) * 8;
+    const int qi = (it.row0 + row) / p.group;
+    const int qs = ((const ConstI32*)p.q_start)[seq];
+    uint16_t* dst = p.out + (int64_t)(qs + qi) * p.o_tok_stride +
+                    (int64_t)(head * p.group + it.row0 + row - qi * p.group) * p.o_head_stride + cd;
+    merge_partials(p, parts, cd, [&](int s) { return (int64_t)(slot + s * p.num_kv_heads) * tile_rows + row; }, dst);
+  }
 }
 
 struct Layout {
   int group, mtiles, units, split_len, max_splits, plan_grid, plan_w;
-  int rows_kg, row_tiles;  // query-tile kernel: key groups per work-group (0: not its shape), tiles per sequence
+  // query-tile kernel: key groups per work-group (0: not its shape), tiles per sequence, split slots
+  int rows_kg, row_tiles, row_slots, row_share, row_extra;
   size_t part_o_off, part_ml_off, error_off, plan_off, desc_off, slots_off, total;
 };
 
@@ -2472,6 +2692,20 @@ int rows_key_groups(int64_t rows, int64_t seq_heads, int max_ctx) {
   return 1;
 }
 
+// Whether the query-tile kernel may split keys: not where a tile has at most two stages, nor
+// where the tiles may fill the chip (more than half of the CUs, if every row is there) and no
+// context has more than kQtWholeStages stages: an uneven batch then loses a few stages at most
+// (64 slots of 17 queries, one sequence of 1,024 keys and the others idle: 22 us, with splits
+// at twice the length 21), while every call would pay ~2 us for a merge kernel that finds
+// nothing (64 x 17 queries after 288 keys, bound 4,096: 28.3 -> 30.2 us).  (The last condition
+// keeps the kernel's sum of stages in 31 bits.)
+constexpr int kQtWholeStages = 8;
+bool rows_split(int64_t tiles, int max_ctx) {
+  const int stages = ceil_div(max(max_ctx, 1), kQtKeys);
+  return stages > kQtMinSplitStages && (2 * tiles <= kPlanCUs || stages > kQtWholeStages) &&
+         tiles * stages < (int64_t(1) << 31);
+}
+
 // Whether the query-tile kernel serves a shape: more rows per KV head than the DMA kernel
 // takes and no split length asked for.  Contexts of at most 64 keys stay with the register
 // kernel, which has one split of them and no staging to pay for: 7.4 us against 9.0-9.9 us
@@ -2488,22 +2722,26 @@ Layout make_layout(int num_seqs, int num_q_heads, int num_kv_heads, int max_q_le
   L.mtiles = ceil_div((int64_t)L.group * max_q_len, kRows);
   L.units = num_seqs * num_kv_heads * L.mtiles;
   if (rows_path && rows_serves(L.mtiles, split_len, max_ctx)) {
-    // one work-group per CU: where the tiles give fewer, the keys are split over the rest
     const int64_t rows = (int64_t)L.group * max_q_len;
     L.rows_kg = rows_key_groups(rows, (int64_t)num_seqs * num_kv_heads, max_ctx);
     const int tile_rows = qt_rows(L.rows_kg);
     L.row_tiles = ceil_div(rows, tile_rows);
-    const int64_t groups = (int64_t)num_seqs * num_kv_heads * L.row_tiles;
-    const int want = (int)max((int64_t)1, (int64_t)kPlanCUs / groups);
-    L.split_len = max(kQtMinSplit, ceil_div(ceil_div(max(max_ctx, 1), want), kQtKeys) * kQtKeys);
-    L.max_splits = ceil_div(max(max_ctx, 1), L.split_len);
-    const size_t parts = L.max_splits > 1 ? (size_t)groups * L.max_splits * tile_rows : 0;
+    const int64_t tiles = (int64_t)num_seqs * num_kv_heads * L.row_tiles;
+    if (rows_split(tiles, max_ctx)) {
+      const int stages = ceil_div(max_ctx, kQtKeys);
+      L.row_share = 2 * tiles <= kPlanCUs ? kQtMinSplitStages : kQtManySplitStages;
+      L.row_slots = (int)min((int64_t)kQtMaxSlots, tiles * ((stages + 1) / kQtMinSplitStages));
+      L.row_extra = (int)min((int64_t)kNumCu, tiles * ((stages - 1) / kQtMinSplitStages));
+    }
+    const size_t parts = (size_t)L.row_slots * tile_rows;
     size_t at = 256;  // the error flag
     L.part_o_off = at;
     at += parts * kHeadDim * sizeof(float);
     L.part_ml_off = at;
     at += (parts * 2 * sizeof(float) + 255) & ~(size_t)255;
-    L.plan_off = L.desc_off = L.slots_off = L.total = at;
+    L.desc_off = at;  // the merges' list
+    at += L.row_slots > 0 ? ((size_t)(1 + L.row_slots / 2) * kQtListInts * sizeof(int32_t) + 255) & ~(size_t)255 : 0;
+    L.plan_off = L.slots_off = L.total = at;
     return L;
   }
   const int fixed_split = split_len > 0 ? split_len : 0;  // 0: the caller left it to us
@@ -2553,14 +2791,13 @@ int launch_attention_rows_kg(const AttnParams& p, hipStream_t s) {
     set_error("paged_attention_rows_kernel: cannot reserve %d bytes of LDS: %s", kQtLds, hipGetErrorString(attr));
     return NE_ELAUNCH;
   }
-  const int64_t tiles = (int64_t)p.num_seqs * p.row_tiles * p.num_kv_heads;
-  const int64_t merges = tiles * (qt_rows(KG) / kRows);
-  NE_CHECK_SUPPORTED(tiles * p.max_splits < (int64_t(1) << 31) && merges < (int64_t(1) << 31),
-                     "too many query tiles (%lld)", (long long)tiles);
-  hipLaunchKernelGGL((paged_attention_rows_kernel<INT8, SDT, KG>), dim3((unsigned)(tiles * p.max_splits)),
-                     dim3(kQtThreads), kQtLds, s, p);
+  const int64_t grid = (int64_t)p.num_seqs * p.row_tiles * p.num_kv_heads + p.row_extra;
+  NE_CHECK_SUPPORTED(grid < (int64_t(1) << 31), "too many query tiles (%lld)", (long long)grid);
+  hipLaunchKernelGGL((paged_attention_rows_kernel<INT8, SDT, KG>), dim3((unsigned)grid), dim3(kQtThreads), kQtLds, s,
+                     p);
   const int rc = check_launch("paged_attention_rows_kernel");
-  if (rc != NE_OK || p.max_splits == 1) return rc;
+  if (rc != NE_OK || p.row_slots == 0) return rc;
+  const int merges = min(kQtMergeGrid, p.row_slots / 2 * (qt_rows(KG) / kRows));
   hipLaunchKernelGGL(attention_rows_merge_kernel, dim3((unsigned)merges), dim3(256), 0, s, p, qt_rows(KG));
   return check_launch("attention_rows_merge_kernel");
 }
@@ -2750,6 +2987,10 @@ int make_params(const void* q, int64_t q_token_stride, int64_t q_head_stride, co
   set_split_plan(p, split_len);
   p.rows_kg = L.rows_kg;
   p.row_tiles = L.row_tiles;
+  p.row_slots = L.row_slots;
+  p.row_share = L.row_share;
+  p.row_extra = L.row_extra;
+  p.rows_list = (int32_t*)(ws + L.desc_off);
   return NE_OK;
 }
 
