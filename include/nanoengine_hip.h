@@ -95,7 +95,9 @@ int ne_kv_write(const void* vectors, int32_t vec_dtype, int64_t n, int32_t num_h
  *   q, out       bf16, element (row, head, d) at row*token_stride + head*head_stride + d
  *   k/v_cache    [num_slots+1, num_kv_heads, 128] bf16 or int8 (kv_dtype)
  *   k/v_scale    [num_slots+1, num_kv_heads] bf16 or fp16 (int8 cache only)
- *   workspace    ne_paged_attention_workspace_size() bytes.  Bytes 0..3 hold an
+ *   workspace    ne_paged_attention_workspace_size() bytes; with split_len 0 a prefill
+ *                shape's size also covers every shape of no more sequences, queries and
+ *                keys, so one buffer can serve prefill and verify.  Bytes 0..3 hold an
  *                error flag, set non-zero when a sequence's context exceeded
  *                max_ctx_len (its keys past max_ctx_len, or past the split grid,
  *                are then dropped); the caller clears it.  The rest holds the work

@@ -2783,6 +2783,18 @@ Layout make_layout(int num_seqs, int num_q_heads, int num_kv_heads, int max_q_le
   return L;
 }
 
+// Bytes that hold the query-tile kernel's workspace of every shape up to this one.  Its own
+// need is not monotone (more tiles are split less, and take another tile size), and a caller
+// may size one buffer for the largest of its shapes.
+size_t rows_workspace_bound(int num_seqs, int num_kv_heads, int64_t rows, int max_ctx) {
+  const int64_t parts_per_tile = (ceil_div(max(max_ctx, 1), kQtKeys) + 1) / kQtMinSplitStages;
+  const int64_t padded_rows = (int64_t)ceil_div(rows, qt_rows(1)) * qt_rows(1);
+  const int64_t most = (int64_t)kQtMaxSlots * qt_rows(1);
+  const int64_t parts = min(most, (int64_t)num_seqs * num_kv_heads * min(parts_per_tile, most) * min(padded_rows, most));
+  const size_t list = (size_t)(1 + kQtMaxSlots / 2) * kQtListInts * sizeof(int32_t);
+  return 256 + (size_t)parts * (kHeadDim + 2) * sizeof(float) + 256 + ((list + 255) & ~(size_t)255);
+}
+
 template <bool INT8, int SDT, int KG>
 int launch_attention_rows_kg(const AttnParams& p, hipStream_t s) {
   static const hipError_t attr = hipFuncSetAttribute((const void*)paged_attention_rows_kernel<INT8, SDT, KG>,
@@ -3064,7 +3076,18 @@ extern "C" size_t ne_paged_attention_workspace_size(int32_t num_seqs, int32_t nu
                                split_len, NE_DTYPE_INT8).total;
   const size_t b = make_layout(num_seqs, num_q_heads, num_kv_heads, max_q_len, max_ctx_len,
                                split_len, NE_DTYPE_BF16).total;
-  return a > b ? a : b;
+  size_t bytes = a > b ? a : b;
+  // a prefill shape: also what every smaller one needs, the verify shapes of at most 32 rows
+  // per KV head among them
+  const int group = num_q_heads / num_kv_heads;
+  const int64_t rows = (int64_t)group * max_q_len;
+  if (split_len == 0 && ceil_div(rows, kRows) > kMaxRowTiles) {
+    bytes = max(bytes, rows_workspace_bound(num_seqs, num_kv_heads, rows, max_ctx_len));
+    const int verify_q = kMaxRowTiles * kRows / group;
+    if (verify_q > 0)
+      bytes = max(bytes, ne_paged_attention_workspace_size(num_seqs, num_q_heads, num_kv_heads, verify_q, max_ctx_len, 0));
+  }
+  return bytes;
 }
 
 extern "C" int ne_paged_verify_attention(

@@ -40,3 +40,15 @@ def test_the_split_rule_needs_no_more_parts_than_there_is_room_for():
         assert heads * sum(parts.values()) <= 341
         assert heads * sum(k - 1 for k in parts.values()) <= 256
         assert heads * len(parts) <= 341 // 2
+
+
+# (8, 2,048, 4,096): a prefill chunk whose engine verifies 8 sequences of 5 rows in the same
+# buffer; (64, 17, 4,096): 16 guesses, and fewer
+@pytest.mark.parametrize("heads", [(16, 8), (8, 8), (24, 2), (40, 1)])
+@pytest.mark.parametrize("largest", [(8, 2048, 4096), (64, 17, 4096), (64, 895, 895), (1, 8192, 16384), (256, 300, 300)])
+def test_a_buffer_for_the_largest_shape_holds_every_smaller_one(size, heads, largest):
+    rng = random.Random(sum(largest))
+    bound = size(largest[0], *heads, *largest[1:], 0)
+    for _ in range(4000):
+        seqs, q, ctx = (max(1, min(n, int(n * 2 ** -rng.uniform(0, 12)))) for n in largest)
+        assert size(seqs, *heads, q, ctx, 0) <= bound, (seqs, q, ctx)
