@@ -135,10 +135,11 @@ int ne_paged_verify_attention(const void* q, int64_t q_token_stride, int64_t q_h
  * OR-ed in as in the workspace's flag; the caller clears it).  A call whose splits need more
  * scratch than NE_NOALLOC_SCRATCH_BYTES returns NE_EWORKSPACE without launching: with at
  * most 32 query rows per KV head, one whose ne_paged_attention_workspace_size() is larger;
- * with more rows, one whose partials of fixed splits (256 keys of int8, 128 of bf16) are.  It allocates nothing: the scratch address is looked up once per
- * device (hipGetSymbolAddress) on the first call with that device current.  Every call on
- * one GPU shares that GPU's scratch, so calls that overlap on one GPU (concurrent streams)
- * race; calls ordered on one stream do not.
+ * with more rows, one whose partials of fixed splits (256 keys of int8, 128 of bf16) are
+ * (the limit, not what the call uses).  It allocates nothing: the scratch address is looked
+ * up once per device (hipGetSymbolAddress) on the first call with that device current.
+ * Every call on one GPU shares that GPU's scratch, so calls that overlap on one GPU
+ * (concurrent streams) race; calls ordered on one stream do not.
  */
 #define NE_NOALLOC_SCRATCH_BYTES (64u << 20)
 int ne_paged_verify_attention_noalloc(

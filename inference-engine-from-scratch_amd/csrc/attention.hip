@@ -3011,6 +3011,8 @@ int make_params(const void* q, int64_t q_token_stride, int64_t q_head_stride, co
 // never passes `scratch` itself (a host-side stand-in for the symbol): it passes the
 // device address hipGetSymbolAddress gives for the current device.
 constexpr size_t kNoAllocScratchBytes = (size_t)NE_NOALLOC_SCRATCH_BYTES;
+static_assert((size_t)kQtMaxSlots * qt_rows(1) * (kHeadDim + 2) * sizeof(float) + (64 << 10) < kNoAllocScratchBytes,
+              "the query-tile kernel's partials fit");
 static __device__ __align__(256) char scratch[kNoAllocScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -3127,8 +3129,9 @@ extern "C" int ne_paged_verify_attention_noalloc(
   NE_CHECK_ARG(num_q_heads > 0 && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 && max_q_len > 0 &&
                    max_ctx_len > 0,
                "bad attention shape");
-  // the limit is the fixed-split layout's, whichever kernel serves the shape (the query-tile
-  // kernel's layout is the smaller one)
+  // the limit is the fixed-split layout's, whichever kernel serves the shape, so that the calls
+  // refused do not depend on that choice; the query-tile kernel's own need (which can be the
+  // larger of the two) is at most rows_workspace_bound's 45.4 MB, and make_params checks it
   const Layout L = make_layout(num_seqs, num_q_heads, num_kv_heads, max_q_len, max_ctx_len, split_len, kv_dtype,
                                /*rows_path=*/false);
   if (L.total > kNoAllocScratchBytes) {
