@@ -1566,12 +1566,19 @@ constexpr int kWholeMaxTiles = 64;                    // longest context of a wh
 // 27.9 -> 24.5 us; one sequence of 17,408 keys 41.8 -> 26.9 us (int8); 8 of 2,000-8,000 34.0
 // -> 28.8; 24 of 300-2,000 24.3 -> 24.2 (bf16 33.0 -> 31.4).  32 such sequences lose with 4
 // (28.8 -> 29.5) and gain with 2 (25.8); 48 are even with 2 (34.4, 34.8) and 64 lose
-// (200-1,500 keys 34.2 -> 37.1).  From 641 keys on 4 also beats one whole item per sequence
-// (16 sequences of 200-800 keys 15.6 -> 14.8, bf16 20.3 -> 15.8; at 640 13.7 and 14.1, bf16
-// 16.8 and 14.3; at 512 12.4 and 13.8).
+// (200-1,500 keys 34.2 -> 37.1).
+// From 641 to 1,024 keys a planned call can also give every sequence one whole item, without
+// partials and merge.  Measured with bounds of 700 and 1,000 keys, whole -> split, int8 / bf16:
+// contexts of 25-100 % of 1,000 keys 2 sequences 15.2 -> 10.9 / 13.6 -> 10.4 us, 12 15.3 ->
+// 11.7 / 15.4 -> 12.6, 16 15.6 -> 12.2 / 16.0 -> 14.8, 24 15.9 -> 14.6 / 17.1 -> 17.7; of
+// 60-100 % of 700 keys 12 13.0 -> 11.5 / 12.6 -> 11.8, 16 13.1 -> 11.9 / 13.1 -> 13.4, 24
+// 13.7 -> 14.1 / 14.8 -> 17.5.  Contexts far below the bound pay for the merge kernel in vain
+// whatever their number (100-250 keys of 1,000: 8.2 -> 9.6).  So up to 12 sequences are split,
+// more stay whole.  An unplanned call has no whole items and splits all of them.
 constexpr int kSplitKs4MaxSeqs = 24;
 constexpr int kSplitKs2MaxSeqs = 40;
 constexpr int kSplitKs4MinTiles = 40;
+constexpr int kSplitOverWholeMaxSeqs = 12;
 constexpr int kSplitKsFloorTiles = 4;  // per wave: its ring
 int split_plan_grid(int num_seqs, int ks) { return max(kPlanCUs / ks, 2 * num_seqs); }  // items
 int split_plan_ks(int num_seqs, int max_ctx, int split_len, int mtiles) {
@@ -1588,7 +1595,7 @@ int split_plan_ks(int num_seqs, int max_ctx, int split_len, int mtiles) {
 // whole work item, served by that many work-groups (one per CU at most): no split
 // partials and no merge kernel.  0 when the split plan serves the shape better.
 int whole_plan_ks(int num_seqs, int max_ctx, int split_len, int mtiles) {
-  if (split_plan_ks(num_seqs, max_ctx, split_len, mtiles) > 1) return 0;
+  if (num_seqs <= kSplitOverWholeMaxSeqs && split_plan_ks(num_seqs, max_ctx, split_len, mtiles) > 1) return 0;
   if (split_len != 0 || mtiles != 1 || (max_ctx + kTileKeys - 1) / kTileKeys > kWholeMaxTiles) return 0;
   if (num_seqs * 4 <= kPlanCUs) return 4;
   if (num_seqs * 2 <= kPlanCUs) return 2;

@@ -1,6 +1,7 @@
 """A6 on split plans with several waves per KV head (up to 24 sequences past 640 keys: four;
 up to 40 past 1,024: two) against the oracle, planned and unplanned (the same items and sums,
-so the same bits), at the rule's edges and with sequences far shorter than the longest.
+so the same bits), at the rule's edges and with sequences far shorter than the longest; planned
+calls of more than 12 sequences keep whole items up to 1,024 keys.
 
 Bar: 6e-3 relative, four roundings of 2^-9 (output, probabilities, the oracle's dequantised
 keys and values; 1.1e-3 rms each) with a factor of 2.6 to spare.
@@ -19,7 +20,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("kv", ["bf16", "int8"])
-@pytest.mark.parametrize("seqs,longest", [(1, 641), (1, 2500), (3, 640), (24, 700), (25, 1024), (25, 1025), (40, 1100),
+@pytest.mark.parametrize("seqs,longest", [(1, 641), (1, 2500), (3, 640), (12, 700), (13, 700), (24, 700), (25, 1024), (25, 1025), (40, 1100),
                                           (41, 1100)])
 def test_split_items(device, kv, seqs, longest):
     ctx = [longest] + [1 + 37 * i % 300 for i in range(seqs - 1)]
@@ -43,5 +44,20 @@ def test_split_items(device, kv, seqs, longest):
                                     model_dtype=torch.bfloat16 if kv == "bf16" else torch.float16)
     assert rel_err(planned.cpu()[idx], ref[idx]) < 6e-3
     assert rel_err(unplanned.cpu()[idx], ref[idx]) < 6e-3
-    if not (25 <= seqs and longest <= 1024) and longest > 640:
+    if longest > 1024 or (seqs <= 12 and longest > 640):
         assert torch.equal(planned.cpu()[idx], unplanned.cpu()[idx])
+
+
+@pytest.mark.parametrize("seqs,ctx,whole", [(12, 700, False), (13, 700, True), (24, 1024, True), (24, 1025, False)])
+def test_whole_items_write_no_partials(device, seqs, ctx, whole):
+    """A whole item's call leaves the workspace's partials (from byte 256 on) as they were."""
+    kc, vc, ks, vs = make_pool(seqs * -(-ctx // 16), 16, 8, "int8")
+    tables, ctx_t, qs, ql, rows = make_batch([ctx] * seqs, [5] * seqs, seqs * -(-ctx // 16), 16)
+    q = torch.randn(rows, 16, 128, generator=torch.Generator().manual_seed(44)).to(torch.bfloat16)
+    q, kc, vc, ks, vs, tables, ctx_t, qs, ql = (t.to(device) for t in (q, kc, vc, ks, vs, tables, ctx_t, qs, ql))
+    ws = kernels.AttentionWorkspace()
+    kernels.paged_attention_plan(tables, 16, ctx_t, qs, ql, 16, 8, 5, ctx, ws)
+    before = ws.buffer[256:1 << 16].clone()
+    kernels.paged_verify_attention(q, kc, vc, ks, vs, tables, 16, ctx_t, qs, ql, max_q_len=5, max_ctx_len=ctx,
+                                   workspace=ws, planned=True)
+    assert torch.equal(ws.buffer[256:1 << 16], before) == whole
