@@ -1161,8 +1161,12 @@ enum class ProjTile { kVerify, k128x128, k128x256, k256x256 };
 // 8,192 rows: 2.3 (256 x 256), 1.32 (128 x 256), 0.8 (128 x 128) and, for the verify step's
 // kernel, 0.39 (80 x 64) or 0.45 (SwiGLU's 80 x 96) with rounds that overlap.  At 512 rows
 // of N = 4,096 that kernel takes 12.6 us and 128 x 128 tiles 14.0, at 1,024 rows 22.9 and
-// 15.7; 2,048 rows of o 24.3 and 23.3, 4,096 rows 49 and 25.  The fused QKV product follows
-// the plain product's choice, so that both sum in one order and round to the same bits.
+// 15.7; 2,048 rows of o 24.3 and 23.3, 4,096 rows 49 and 25.  From N = 16,384 on the tiles also
+// win below 320 rows (K = 1,024: 200 rows of 16,384 18.2 and 14.8, 81 of 32,768 25.2 and 15.9,
+// 33 of 65,536 26.4 and 22.8, 17 of 131,072 47.9 and 43.2; 17 of 65,536 over K = 2,048 45.2 and
+// 40.8); up to 16 rows the few-rows kernel goes first (16 of 65,536: 18.6, tiles 22.6).  The
+// fused QKV product follows the plain product's choice, so that both sum in one order and round
+// to the same bits.
 ProjTile choose_proj_tile(int m, int n, bool swiglu) {
   const auto rounds = [&](int bm, int bn) {
     return (int64_t)ceil_div((int64_t)ceil_div(m, bm) * (n / bn), kNumCu);
@@ -1437,6 +1441,11 @@ int launch_few(const GemmParams& p, int splits, float* partial, hipStream_t s, c
 
 template <int SDT>
 int dispatch_qkv_fused(GemmParams p, const QkvRopeArgs& qa, int kv_mode, hipStream_t s) {
+  if (few_rows(p, 1)) {
+    if (kv_mode == 1) return launch_few<1, kKgQkv, 8, 4, 1>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
+    if (kv_mode == 2) return launch_few<1, kKgQkv, 8, 4, 2>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
+    return launch_few<1, kKgQkv, 8, 4, 3>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
+  }
   // the tiles' epilogue stores 4 or 8 bytes at a time where the row kernel's stores elements
   const bool aligned = (((uintptr_t)qa.q_out | (uintptr_t)qa.rope | (uintptr_t)qa.k_cache | (uintptr_t)qa.v_cache) % 8) == 0;
   const ProjTile tile = aligned ? choose_proj_tile(p.m, p.n, false) : ProjTile::kVerify;
@@ -1444,11 +1453,6 @@ int dispatch_qkv_fused(GemmParams p, const QkvRopeArgs& qa, int kv_mode, hipStre
     if (kv_mode == 1) return launch_proj_tile<4, 1>(tile, p, s, "w8a16_qkv_norm_rope_kv", qa);
     if (kv_mode == 2) return launch_proj_tile<4, 2>(tile, p, s, "w8a16_qkv_norm_rope_kv", qa);
     return launch_proj_tile<4, 3>(tile, p, s, "w8a16_qkv_norm_rope_kv", qa);
-  }
-  if (few_rows(p, 1)) {
-    if (kv_mode == 1) return launch_few<1, kKgQkv, 8, 4, 1>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
-    if (kv_mode == 2) return launch_few<1, kKgQkv, 8, 4, 2>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
-    return launch_few<1, kKgQkv, 8, 4, 3>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
   }
   switch (kv_mode) {
     // 48-row tiles: 7 x 32 = 224 work-groups for 320 rows, 3 rows per wave in the epilogue
@@ -1460,16 +1464,16 @@ int dispatch_qkv_fused(GemmParams p, const QkvRopeArgs& qa, int kv_mode, hipStre
 
 template <int SDT>
 int dispatch_w8a16(GemmParams p, int epilogue, int splits, float* partial, hipStream_t s) {
+  if (few_rows(p, partial != nullptr ? splits : 1)) {
+    if (epilogue == NE_EPILOGUE_SWIGLU) return launch_few<2, kKgSwiglu, 2, 1, 0>(p, 1, nullptr, s, "w8a16_swiglu");
+    if (partial != nullptr) return launch_few<1, kKgPlain, 2, 3, 0>(p, splits, partial, s, "w8a16_splitk");
+    return launch_few<1, kKgPlain, 2, 0, 0>(p, 1, nullptr, s, "w8a16_gemm");
+  }
   if (partial == nullptr) {
     const bool swiglu = epilogue == NE_EPILOGUE_SWIGLU;
     const ProjTile tile = choose_proj_tile(p.m, p.n, swiglu);
     if (tile != ProjTile::kVerify)
       return swiglu ? launch_proj_tile<1, 0>(tile, p, s, "w8a16_swiglu") : launch_proj_tile<0, 0>(tile, p, s, "w8a16_gemm");
-  }
-  if (few_rows(p, partial != nullptr ? splits : 1)) {
-    if (epilogue == NE_EPILOGUE_SWIGLU) return launch_few<2, kKgSwiglu, 2, 1, 0>(p, 1, nullptr, s, "w8a16_swiglu");
-    if (partial != nullptr) return launch_few<1, kKgPlain, 2, 3, 0>(p, splits, partial, s, "w8a16_splitk");
-    return launch_few<1, kKgPlain, 2, 0, 0>(p, 1, nullptr, s, "w8a16_gemm");
   }
   if (epilogue == NE_EPILOGUE_SWIGLU) {
     if (p.n % 96 == 0)

@@ -181,3 +181,12 @@ def test_few_rows_give_the_bits_of_many(device, m):
                 assert not any(c[other].any() for c in caches)
         for a, b in zip(*results):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("m", [1, 16])
+def test_few_rows_of_a_wide_product_run_the_few_rows_kernel(device, m):
+    """One split of the split-K product is the plain product's sum, in fp32."""
+    w, s = weight(65536, 1024, device)
+    x = torch.randn(m, 1024, device=device, generator=torch.Generator(device=device).manual_seed(m)).to(torch.bfloat16)
+    assert torch.equal(kernels.w8a16_gemm(x, w, s),
+                       kernels.w8a16_gemm_splitk(x, w, s, 1).view(m, 65536).to(torch.bfloat16))
