@@ -246,6 +246,19 @@ int ne_w8a16_gemm_splitk(const void* x, int64_t ldx, const int8_t* w, const void
                          float* partials, void* stream);
 
 /*
+ * Which kernel serves a W8A16 product of these sizes (host only; for tests and
+ * measurements): ne_w8a16_gemm with `epilogue` for splits 0, ne_w8a16_gemm_splitk for
+ * splits >= 1.  ne_w8a16_qkv_norm_rope_kv follows the plain product of its n and k, except
+ * that pointers off their 8-byte alignment keep it from the tiles.
+ */
+#define NE_W8A16_STAGED 0
+#define NE_W8A16_FEW_ROWS 1
+#define NE_W8A16_TILE_128X128 2
+#define NE_W8A16_TILE_128X256 3
+#define NE_W8A16_TILE_256X256 4
+int32_t ne_w8a16_kernel(int32_t m, int32_t n, int32_t k, int32_t splits, int32_t epilogue);
+
+/*
  * A8b - bf16 GEMM for the tied LM head: logits[m, n] = bf16(sum_k x[m,k] w[n,k])
  * (replaces compute_logits, ne/models/qwen3.py:197-203).  Either output may be
  * null.  When argmax_partials is given, it receives per row ne_lm_head_num_tiles(n)

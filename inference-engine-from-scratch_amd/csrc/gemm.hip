@@ -1214,10 +1214,12 @@ struct FewLayout {
   static constexpr int kStage = kRows * 256;         // X rows of a 128-wide stage
   static constexpr int kX = KT * kStage;
   static constexpr int kCopies = KT * PM * 4;        // 1 KiB copies: 4 rows of 256 B
-  static constexpr int kPerWave = kCopies / WAVES;
+  static constexpr int kPerWave = (kCopies + WAVES - 1) / WAVES;
   static constexpr int kLoads = NPW * KT * 2;        // 16-byte weight loads per lane
-  static_assert(kCopies % WAVES == 0 && kLoads < 64, "copies split evenly; vmcnt range");
-  static_assert(kX <= 160 * 1024, "LDS");
+  static constexpr int kRowF = 132;                  // floats per row of the QKV epilogue's fp32 rows
+  static constexpr int kLds = kX > kRows * kRowF * 4 ? kX : kRows * kRowF * 4;
+  static_assert(kLoads < 64, "vmcnt range");
+  static_assert(kLds <= 160 * 1024, "LDS");
 };
 
 template <typename L, int EPI, int KV>
@@ -1238,6 +1240,7 @@ __global__ __launch_bounds__(L::WAVES* kWave) void proj_few_rows_kernel(GemmPara
 #pragma unroll
     for (int j = 0; j < L::kPerWave; ++j) {
       const int i = j * L::WAVES + wave;  // KiB: stage i / (4 PM), rows 4 (i % (4 PM)) .. + 4
+      if (i >= L::kCopies) break;         // wave-uniform
       const int t = i / (4 * PM);
       const int row = (i % (4 * PM)) * 4 + (lane >> 4);
       // rows past m re-read row m - 1 and are never stored
@@ -1353,8 +1356,7 @@ __global__ __launch_bounds__(L::WAVES* kWave) void proj_few_rows_kernel(GemmPara
     // the head's rows through LDS (fp32 [row][128 + 4], over X once every wave has read it),
     // then wave w takes rows w, w + WAVES, .. as the row kernel does
     static_assert(NPW == 1 && L::WAVES == 8, "one head per work-group");
-    constexpr int kRowF = 132;
-    static_assert(L::kRows * kRowF * 4 <= L::kX, "the rows fit over X");
+    constexpr int kRowF = L::kRowF;
     float* rows = (float*)smem;
     lds_barrier();
 #pragma unroll
@@ -1400,13 +1402,13 @@ template <typename L, int EPI, int KV>
 int launch_few_as(const GemmParams& p, int splits, float* partial, hipStream_t stream, const char* name,
                   const QkvRopeArgs& qa) {
   static const hipError_t attr = hipFuncSetAttribute((const void*)proj_few_rows_kernel<L, EPI, KV>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, L::kX);
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, L::kLds);
   if (attr != hipSuccess) {
-    set_error("%s: cannot reserve %d bytes of LDS: %s", name, L::kX, hipGetErrorString(attr));
+    set_error("%s: cannot reserve %d bytes of LDS: %s", name, L::kLds, hipGetErrorString(attr));
     return NE_ELAUNCH;
   }
   hipLaunchKernelGGL((proj_few_rows_kernel<L, EPI, KV>),
-                     dim3((unsigned)(p.n / (L::WAVES * L::NPW * 16)), (unsigned)splits), dim3(L::WAVES * kWave), L::kX,
+                     dim3((unsigned)(p.n / (L::WAVES * L::NPW * 16)), (unsigned)splits), dim3(L::WAVES * kWave), L::kLds,
                      stream, p, partial, qa);
   return check_launch(name);
 }
@@ -1419,24 +1421,26 @@ constexpr int kKgPlain = 2, kNpwPlain = 1;
 constexpr int kKgQkv = 2, kNpwQkv = 2;
 constexpr int kKgSwiglu = 4, kNpwSwiglu = 2;
 
-// Whether the few-rows kernel serves a product: one token subtile, and a K (per split) of
-// 1,024 (or 512 / 768 of a split one), i.e. 8, 4 or 6 stages.  With three subtiles it lost to
-// the staged kernel at 48 rows (QKV 10.4 -> 12.2 us, gate|up 8.2 -> 9.4, down 5.6 -> 6.8:
-// every wave then waits for 96 KB of X before its first product).
-bool few_rows(const GemmParams& p, int splits) {
-  const int kt = p.k / splits / kStageK;
-  return p.m <= 16 && (splits > 1 ? kt == 4 || kt == 6 || kt == 8 : kt == 8);
-}
+// Whether the few-rows kernel serves a product: one token subtile, and a K (per split) of up
+// to kFewMaxStages stages, whose weights a wave holds in registers (128 of them for SwiGLU's
+// two subtiles).  Per launch at 5 rows, weights in turn from a HIP graph (us, staged -> here):
+// N = 4,096 K = 128 3.5 -> 2.6, 384 4.7 -> 3.3, 640 5.7 -> 3.9, 896 6.7 -> 5.0, 1,024 6.2 -> 5.3;
+// SwiGLU N = 6,144 4.5 -> 3.3, 5.8 -> 4.3, 7.2 -> 5.7, 8.4 -> 6.9 and 7.6 -> 7.6; four splits of
+// them at N = 1,024 3.2 -> 2.7, 4.2 -> 3.3, 5.0 -> 3.9, 5.9 -> 4.9 and 5.2 -> 5.3.  A larger K
+// would need a second burst behind the first.  With three subtiles it lost to the staged kernel at 48 rows (QKV 10.4 ->
+// 12.2 us, gate|up 8.2 -> 9.4, down 5.6 -> 6.8: every wave then waits for 96 KB of X before its
+// first product).
+constexpr int kFewMaxStages = 8;
+bool few_rows(const GemmParams& p, int splits) { return p.m <= 16 && p.k / splits <= kFewMaxStages * kStageK; }
 
-template <int NPW, int KG, int WAVES, int EPI, int KV>
+template <int NPW, int KG, int WAVES, int EPI, int KV, int KT = kFewMaxStages>
 int launch_few(const GemmParams& p, int splits, float* partial, hipStream_t s, const char* name,
                const QkvRopeArgs& qa = QkvRopeArgs{}) {
-  const int kt = p.k / splits / kStageK;
-  if constexpr (EPI == 3) {
-    if (kt == 4) return launch_few_as<FewLayout<1, NPW, KG, WAVES, 4>, EPI, KV>(p, splits, partial, s, name, qa);
-    if (kt == 6) return launch_few_as<FewLayout<1, NPW, KG, WAVES, 6>, EPI, KV>(p, splits, partial, s, name, qa);
+  if constexpr (KT > 1) {
+    if (p.k / splits / kStageK < KT)
+      return launch_few<NPW, KG, WAVES, EPI, KV, KT - 1>(p, splits, partial, s, name, qa);
   }
-  return launch_few_as<FewLayout<1, NPW, KG, WAVES, 8>, EPI, KV>(p, splits, partial, s, name, qa);
+  return launch_few_as<FewLayout<1, NPW, KG, WAVES, KT>, EPI, KV>(p, splits, partial, s, name, qa);
 }
 
 template <int SDT>
@@ -2006,6 +2010,22 @@ int w8a16_common(const void* x, int64_t ldx, const int8_t* w, const void* scale,
 }
 
 }  // namespace
+
+extern "C" int32_t ne_w8a16_kernel(int32_t m, int32_t n, int32_t k, int32_t splits, int32_t epilogue) {
+  if (m <= 0 || n <= 0 || k <= 0 || splits < 0) return NE_W8A16_STAGED;
+  GemmParams p{};
+  p.m = m;
+  p.n = n;
+  p.k = k;
+  if (few_rows(p, splits > 0 ? splits : 1)) return NE_W8A16_FEW_ROWS;
+  if (splits > 0) return NE_W8A16_STAGED;
+  switch (choose_proj_tile(m, n, epilogue == NE_EPILOGUE_SWIGLU)) {
+    case ProjTile::k128x128: return NE_W8A16_TILE_128X128;
+    case ProjTile::k128x256: return NE_W8A16_TILE_128X256;
+    case ProjTile::k256x256: return NE_W8A16_TILE_256X256;
+    default: return NE_W8A16_STAGED;
+  }
+}
 
 extern "C" int ne_w8a16_gemm(const void* x, int64_t ldx, const int8_t* w, const void* scale,
                              int32_t scale_dtype, int32_t m, int32_t n, int32_t k, void* y,

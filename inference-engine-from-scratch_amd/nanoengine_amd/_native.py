@@ -87,6 +87,7 @@ SIGNATURES: dict[str, tuple] = {
         ctypes.c_int,
         [_vp, _i64, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp],
     ),
+    "ne_w8a16_kernel": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "ne_lm_head_num_tiles": (_i32, [_i32]),
     "ne_lm_head": (ctypes.c_int, [_vp, _i64, _vp, _i32, _i32, _i32, _vp, _i64, _u64p, _vp]),
     "ne_rmsnorm": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i32, _f32, _vp]),

@@ -12,7 +12,7 @@ import pytest
 import torch
 
 from helpers import rel_err
-from nanoengine_amd import kernels
+from nanoengine_amd import _native, kernels
 from nanoengine_amd._native import EPILOGUE_SWIGLU
 
 pytestmark = pytest.mark.gpu
@@ -190,3 +190,41 @@ def test_few_rows_of_a_wide_product_run_the_few_rows_kernel(device, m):
     x = torch.randn(m, 1024, device=device, generator=torch.Generator(device=device).manual_seed(m)).to(torch.bfloat16)
     assert torch.equal(kernels.w8a16_gemm(x, w, s),
                        kernels.w8a16_gemm_splitk(x, w, s, 1).view(m, 65536).to(torch.bfloat16))
+
+
+FEW_ROWS = 1
+
+
+# stage counts other than the benchmark model's 8 (K = 1,024) and 4, 6, 8 of a split product
+@pytest.mark.parametrize("k", [128, 256, 384, 512, 640, 768, 896, 1024])
+def test_few_rows_over_any_k(device, k):
+    """Every K (per split) of up to 1,024 runs the few-rows kernel and gives a row the bits it
+    has among 320, plain, paired, split and through the fused QKV epilogue."""
+    choice = _native.load().ne_w8a16_kernel
+    m, g = 5, torch.Generator(device=device).manual_seed(k)
+    x = torch.randn(320, 4 * k, device=device, generator=g).to(torch.bfloat16)
+    for n, epilogue in ((4096, 0), (6144, EPILOGUE_SWIGLU)):
+        assert choice(m, n, k, 0, epilogue) == FEW_ROWS and choice(320, n, k, 0, epilogue) == 0
+        w, s = weight(n, k, device)
+        few = kernels.w8a16_gemm(x[:m, :k], w, s, epilogue=epilogue)
+        assert torch.equal(few, kernels.w8a16_gemm(x[:, :k], w, s, epilogue=epilogue)[:m])
+        if epilogue == 0:
+            assert rel_err(few, product(x[:m, :k], w, s)) < 2.5e-3
+    assert choice(m, 1024, 4 * k, 4, 0) == FEW_ROWS and choice(320, 1024, 4 * k, 4, 0) == 0
+    w, s = weight(1024, 4 * k, device)
+    few, many = kernels.w8a16_gemm_splitk(x[:m], w, s, 4), kernels.w8a16_gemm_splitk(x, w, s, 4)
+    assert torch.equal(few.view(4, m, 1024), many.view(4, 320, 1024)[:, :m])
+    w, s = weight(4096, k, device)
+    norms = [(1 + 0.1 * torch.randn(128, device=device, generator=g)).to(torch.bfloat16) for _ in range(2)]
+    positions = torch.randint(0, 3000, (m,), generator=g, dtype=torch.int32, device=device)
+    rope = kernels.rope_table(3000, 1e6).to(device)
+    slots = torch.randperm(40, generator=g, device=device)[:m].to(torch.int32)
+    pools = [[torch.zeros(40, 8, 128, dtype=torch.int8, device=device) for _ in range(2)]
+             + [torch.zeros(40, 8, dtype=torch.bfloat16, device=device) for _ in range(2)] for _ in range(2)]
+    q_ref = kernels.qk_norm_rope_kv_write(kernels.w8a16_gemm(x[:m, :k], w, s), 16, 8, *norms, 1e-6, positions, rope,
+                                          slots, *pools[0])
+    q = torch.zeros(m + 1, 16, 128, dtype=torch.bfloat16, device=device)
+    kernels.w8a16_qkv_norm_rope_kv(x[:m, :k], w, s, 16, 8, *norms, 1e-6, positions, rope, slots, *pools[1], q_out=q[:m])
+    assert torch.equal(q[:m], q_ref) and not q[m].any()
+    for a, b in zip(*pools):
+        assert torch.equal(a, b)
