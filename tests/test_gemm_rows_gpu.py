@@ -1,7 +1,7 @@
 """A8 over many rows (prefill): the large-tile projection kernels against Int8Linear in fp32.
 
 Sizes reach each tile (128 x 128, 128 x 256, 256 x 256) with row counts one below, at and one
-past its edges.  Bars: 2.5e-3 relative for a plain product, whose only rounding beside fp32
+past its edges; every case pins the kernel that serves it.  Bars: 2.5e-3 relative for a plain product, whose only rounding beside fp32
 sums is the bf16 output (2^-9, 1.1e-3 rms); 5e-3 for SwiGLU, which rounds gate, up, silu and
 the product (four such, 2.3e-3).
 """
@@ -29,12 +29,23 @@ def product(x, w, s):
     return (x.float() @ w.float().t()) * s.float()
 
 
-# N = 4,096 at 897-1,024 rows: 128 x 128; at 2,047-2,048: 128 x 256; at 3,841-4,096: 256 x 256
-@pytest.mark.parametrize("m,n,k", [
-    (897, 4096, 1024), (1024, 4096, 128), (1023, 4096, 256), (1000, 4096, 384), (2047, 4096, 1024), (2048, 4096, 128),
-    (2000, 4096, 384), (3841, 4096, 1024), (4096, 4096, 128), (4095, 4096, 256), (4097, 1024, 2048), (8191, 1024, 3072),
+STAGED, FEW_ROWS, TILE_128X128, TILE_128X256, TILE_256X256 = range(5)
+
+
+def kernel_of(m, n, k, splits=0, epilogue=0):
+    return _native.load().ne_w8a16_kernel(m, n, k, splits, epilogue)
+
+
+@pytest.mark.parametrize("tile,m,n,k", [
+    (TILE_128X128, 897, 4096, 1024), (TILE_128X128, 1024, 4096, 128), (TILE_128X128, 1023, 4096, 256),
+    (TILE_128X128, 1000, 4096, 384), (TILE_128X128, 641, 4096, 1024), (TILE_128X128, 2561, 1024, 2048),
+    (TILE_128X256, 2047, 4096, 1024), (TILE_128X256, 2048, 4096, 128), (TILE_128X256, 2000, 4096, 384),
+    (TILE_128X256, 4321, 1024, 2048), (TILE_128X256, 8191, 1024, 3072),
+    (TILE_256X256, 3841, 4096, 1024), (TILE_256X256, 4096, 4096, 128), (TILE_256X256, 4095, 4096, 256),
+    (STAGED, 4097, 1024, 2048), (TILE_128X256, 17, 65536, 1024),
 ])
-def test_product(device, m, n, k):
+def test_product(device, tile, m, n, k):
+    assert kernel_of(m, n, k) == tile
     w, s = weight(n, k, device)
     x = torch.randn(m, k, device=device, generator=torch.Generator(device=device).manual_seed(m)).to(torch.bfloat16)
     out = kernels.w8a16_gemm(x, w, s)
@@ -52,8 +63,14 @@ def test_scale_types_and_strides(device, scale_dtype):
     assert not out[1001].any()  # the row after the last
 
 
-@pytest.mark.parametrize("m", [1025, 1537, 2049])
-def test_swiglu(device, m):
+# the two-k-group tile at its first and last rows, one row past and one before the others' edges
+@pytest.mark.parametrize("tile,m", [
+    (TILE_128X128, 561), (TILE_128X128, 600), (TILE_128X128, 639), (TILE_128X128, 640), (STAGED, 641),
+    (TILE_128X256, 881), (TILE_128X256, 1025), (TILE_128X256, 1280), (STAGED, 1537), (TILE_256X256, 1601),
+    (TILE_256X256, 2049), (TILE_256X256, 2560),
+])
+def test_swiglu(device, tile, m):
+    assert kernel_of(m, 6144, 1024, epilogue=EPILOGUE_SWIGLU) == tile
     gate, gs = weight(3072, 1024, device, seed=1)
     up, us = weight(3072, 1024, device, seed=2)
     pair = lambda a, b: torch.stack([a.view(-1, 16, *a.shape[1:]), b.view(-1, 16, *b.shape[1:])], 1).flatten(0, 2)
@@ -64,11 +81,12 @@ def test_swiglu(device, m):
 
 
 @pytest.mark.parametrize("kv", ["int8-bf16-scales", "int8-fp16-scales", "bf16"])
-@pytest.mark.parametrize("m", [1000, 2047, 3900])
-def test_fused_qkv_equals_gemm_then_row_kernel(device, kv, m):
+@pytest.mark.parametrize("tile,m", [(TILE_128X128, 1000), (TILE_128X256, 2047), (TILE_256X256, 3900)])
+def test_fused_qkv_equals_gemm_then_row_kernel(device, kv, tile, m):
     """The tiles' QK-norm + RoPE + KV-write epilogue gives the bits of the plain product
     followed by the row kernel, rows past the last written nowhere."""
     hq, hkv, k, slots_n = 16, 8, 1024, 5000
+    assert kernel_of(m, 4096, k) == tile
     g = torch.Generator(device=device).manual_seed(m)
     w, s = weight(4096, k, device)
     x = torch.randn(m, k, device=device, generator=g).to(torch.bfloat16)
@@ -192,25 +210,21 @@ def test_few_rows_of_a_wide_product_run_the_few_rows_kernel(device, m):
                        kernels.w8a16_gemm_splitk(x, w, s, 1).view(m, 65536).to(torch.bfloat16))
 
 
-FEW_ROWS = 1
-
-
 # stage counts other than the benchmark model's 8 (K = 1,024) and 4, 6, 8 of a split product
 @pytest.mark.parametrize("k", [128, 256, 384, 512, 640, 768, 896, 1024])
 def test_few_rows_over_any_k(device, k):
     """Every K (per split) of up to 1,024 runs the few-rows kernel and gives a row the bits it
     has among 320, plain, paired, split and through the fused QKV epilogue."""
-    choice = _native.load().ne_w8a16_kernel
     m, g = 5, torch.Generator(device=device).manual_seed(k)
     x = torch.randn(320, 4 * k, device=device, generator=g).to(torch.bfloat16)
     for n, epilogue in ((4096, 0), (6144, EPILOGUE_SWIGLU)):
-        assert choice(m, n, k, 0, epilogue) == FEW_ROWS and choice(320, n, k, 0, epilogue) == 0
+        assert kernel_of(m, n, k, 0, epilogue) == FEW_ROWS and kernel_of(320, n, k, 0, epilogue) == STAGED
         w, s = weight(n, k, device)
         few = kernels.w8a16_gemm(x[:m, :k], w, s, epilogue=epilogue)
         assert torch.equal(few, kernels.w8a16_gemm(x[:, :k], w, s, epilogue=epilogue)[:m])
         if epilogue == 0:
             assert rel_err(few, product(x[:m, :k], w, s)) < 2.5e-3
-    assert choice(m, 1024, 4 * k, 4, 0) == FEW_ROWS and choice(320, 1024, 4 * k, 4, 0) == 0
+    assert kernel_of(m, 1024, 4 * k, 4) == FEW_ROWS and kernel_of(320, 1024, 4 * k, 4) == STAGED
     w, s = weight(1024, 4 * k, device)
     few, many = kernels.w8a16_gemm_splitk(x[:m], w, s, 4), kernels.w8a16_gemm_splitk(x, w, s, 4)
     assert torch.equal(few.view(4, m, 1024), many.view(4, 320, 1024)[:, :m])
