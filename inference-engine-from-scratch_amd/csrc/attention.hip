@@ -1607,8 +1607,8 @@ int whole_plan_ks(int num_seqs, int max_ctx, int split_len, int mtiles) {
 // covers tiles [tiles_b s / n_b, tiles_b (s+1) / n_b)).  W is p.plan_w when the
 // caller fixed the split length; else 16 when every context fits in 16 tiles (one
 // split per sequence, so no partials and no merge kernel); else
-// max(8, ceil(T / (G - B))) (16 with four waves per KV head) for T = sum_b tiles_b, G =
-// p.plan_grid items and B sequences -- splitting is paid for already, so W only balances
+// max(p.plan_floor, ceil(T / (G - B))) (a floor of 8, or of 16 with four waves per KV head)
+// for T = sum_b tiles_b, G = p.plan_grid items and B sequences -- splitting is paid for already, so W only balances
 // the longest split against the mean.  Both keep sum_b n_b <= G:
 // the longest sequence is spread over as many work-groups as its share of T asks
 // for instead of one per fixed-length split, and no CU waits for a second round
@@ -2065,10 +2065,11 @@ __device__ __forceinline__ void compute_iter_bf(const IterRegs<false>& R, const 
 // output instead of being derived here (one round trip instead of two).
 // MT: row tiles of 16 per KV head handled by each wave (1, or 2 for up to 32 rows).
 // KS: waves per KV head.  KS = 1: the 8 waves are the 8 KV heads of one work item.
-// KS > 1 (planned, one row tile, items of whole sequences): KS work-groups share an
-// item, each taking 8 / KS heads, and a head's KS waves take consecutive parts of the
-// item's tiles, their (m, l, O) merged through LDS before the store -- so that short
-// contexts fill KS times as many CUs without a merge kernel.
+// KS > 1 (one row tile; items of whole sequences of a planned call, or split items of any):
+// KS work-groups share an item, each taking 8 / KS heads, and a head's KS waves take
+// consecutive parts of the item's tiles, their (m, l, O) merged through LDS before the store
+// -- so that short contexts fill KS times as many CUs without a merge kernel, and split ones
+// write 1 / KS of the partials.
 // BF16: a bf16 cache (SDT unused): two-tile rings, bf16 MFMA scores (compute_iter_bf).
 template <int SDT, bool PLANNED, int MT, int KS = 1, bool BF16 = false>
 __global__ __launch_bounds__((DmaShape<KS, BF16>::waves * kWave)) void paged_attention_dma_kernel(AttnParams p) {
@@ -2715,8 +2716,9 @@ bool rows_split(int64_t tiles, int max_ctx) {
 
 // Whether the query-tile kernel serves a shape: more rows per KV head than the DMA kernel
 // takes and no split length asked for.  Contexts of at most 64 keys stay with the register
-// kernel, which has one split of them and no staging to pay for: 7.4 us against 9.0-9.9 us
-// at 17-32 queries of a bf16 cache, 9.5-9.7 us against 9.0-9.9 us at 17-64 of an int8 one.
+// kernel, which has one split of them and no staging to pay for: 7.4 us against 9.0-9.9 us at
+// 17-32 queries of a bf16 cache.  Of an int8 one the two are even there (9.5-9.7 us against
+// 9.0-9.9 us at 17-64 queries); one line serves both.
 bool rows_serves(int mtiles, int split_len, int max_ctx) {
   return mtiles > kMaxRowTiles && split_len <= 0 && max_ctx > 4 * kTileKeys;
 }
