@@ -96,6 +96,54 @@ def test_uneven_contexts_split_by_their_work(device, q_lens, pasts, heads, kv):
     assert rel_err(got, ref) < TOL
 
 
+def test_captured_and_allocation_free_calls_split_by_the_lengths_of_the_replay(device):
+    """A graph captured once with bounds serves batches of other lengths, with eager work between
+    its replays; the library's own scratch gives the same bits as a workspace."""
+    n, bound = 17, 2300
+    blocks = -(-bound // 16)
+    kc, vc, ks, vs = make_pool(n * blocks, 16, 8, "int8", seed=61)
+    tables = torch.randperm(n * blocks, generator=torch.Generator().manual_seed(62)).to(torch.int32).view(n, blocks)
+    q = torch.randn(n * 20, 16, 128, generator=torch.Generator().manual_seed(63)).to(torch.bfloat16)
+    starts = torch.arange(n, dtype=torch.int32) * 20
+    batches = [([30 + i for i in range(n)], [17] * n), ([40] * (n - 1) + [bound], [20] * n), ([1800, bound, 2100, 90] * 4 + [700], [20] * n),
+               ([0] * 5 + [2250] + [0] * (n - 6), [0] * 5 + [18] + [0] * (n - 6))]
+    d = lambda t: t.to(device)
+    ctx, ql = (torch.zeros(n, dtype=torch.int32, device=device) for _ in range(2))
+    args = [d(t) for t in (q, kc, vc, ks, vs, tables)] + [16, ctx, d(starts), ql]
+    out = torch.zeros(n * 20, 16, 128, dtype=torch.bfloat16, device=device)
+    ws = kernels.AttentionWorkspace()
+
+    def call():
+        kernels.paged_verify_attention(*args, max_q_len=20, max_ctx_len=bound, out=out, workspace=ws)
+
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for lens, queries in batches * 2:
+        ctx.copy_(torch.tensor(lens, dtype=torch.int32))
+        ql.copy_(torch.tensor(queries, dtype=torch.int32))
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        replayed = out.clone()
+        out.zero_()
+        call()
+        flag = torch.zeros(1, dtype=torch.int32, device=device)
+        scratch = torch.zeros_like(out)
+        kernels.paged_verify_attention_noalloc(*args, max_q_len=20, max_ctx_len=bound, out=scratch, error_flag=flag)
+        torch.cuda.synchronize()
+        assert int(flag) == 0 and ws.error_flag() == 0
+        assert torch.equal(replayed, out) and torch.equal(replayed, scratch)
+        t = lambda v: torch.tensor(v, dtype=torch.int32)
+        idx = real_rows(starts, t(queries))
+        keep = [i for i, m in enumerate(queries) if m]
+        ref = paged_attention_reference(q, kc, vc, ks, vs, tables[keep], 16, t(lens)[keep], starts[keep], t(queries)[keep],
+                                        model_dtype=torch.bfloat16)
+        assert rel_err(replayed.cpu()[idx], ref[idx]) < TOL
+
+
 @pytest.mark.parametrize("scale_dtype", [torch.float16, torch.float32])
 def test_scale_types(device, scale_dtype):
     got, ref = run(device, [70, 40], [30, 300], "int8", scale_dtype)
