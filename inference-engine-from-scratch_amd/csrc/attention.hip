@@ -107,6 +107,7 @@ struct AttnParams {
   int32_t row_tiles;   // query-tile kernel: tiles of query rows per sequence
   int32_t row_slots;   // query-tile kernel: partials of split tiles (0: no splits)
   int32_t row_share;   // query-tile kernel: least stages per work-group of a split tile
+  int32_t row_parts;   // query-tile kernel: work-groups of every tile where row_share is the batch's share (else 0)
   int32_t row_extra;   // query-tile kernel: work-groups for the parts after a tile's first
   int32_t* rows_list;  // query-tile kernel: the split tiles' merges, [1 + row_slots / 2][kQtListInts], the count first
   int32_t* plan_desc;  // precomputed plan: [plan_grid][8] work items (seq < 0: none)
@@ -857,13 +858,16 @@ static_assert(kQtLds <= 160 * 1024, "LDS of one CU");
 // twelve prompts of 300 522 -> 69, 64 slots of 17 queries with one sequence of 16,384 keys
 // 253 -> 44 (the fixed-split kernel: 208 and 50), eight times 64 queries after 0-6,000 keys
 // 47 -> 32.
-// Every work-group derives S from the lengths (a load per thread, a sum in registers and one
-// in LDS, under the first loads).  A tile's own work-group serves its first part, which needs S
-// only to know where to end; the other parts have work-groups at the end of the grid, so that
-// those without a part (most calls split nothing) leave while the last tiles run.  In front of
-// the tiles they balance a little better (63 instead of 69 us above) and cost every call
-// ~3 us; as a second pass of the tiles' own work-groups they cost the main loop 13 % (the
-// lane addresses of both passes held in registers or computed again).
+// Where even full tiles of the longest context give the least share, the host knows S, and the
+// parts of a tile have work-groups side by side.  Elsewhere every work-group derives S from the
+// lengths: a load per thread, a sum in registers and one in LDS, under the first loads (8 x 48
+// queries of 400 keys paid 2.3 us of 19.5 for it, one sequence of 17 after 4,096 1.9 of 19.2).
+// A tile's own work-group then serves its first part, which needs S only to know where to end;
+// the other parts have work-groups at the end of the grid, so that those without a part (most
+// calls split nothing) leave while the last tiles run.  In front of the tiles they balance a
+// little better (63 instead of 69 us above) and cost every call ~3 us; as a second pass of the
+// tiles' own work-groups they cost the main loop 13 % (the lane addresses of both passes held in
+// registers or computed again).
 constexpr int kQtMinSplitStages = 2;             // a shorter part is mostly prologue and partials
 constexpr int kQtManySplitStages = 4;            // where the tiles may fill the chip: tiles of up to 5 need no S
 constexpr int kQtMaxSlots = 4 * kNumCu / 3;      // parts of split tiles, each with a partial's room
@@ -1130,7 +1134,7 @@ __device__ __forceinline__ QtItem qt_item(const AttnParams& p, int seq, int tile
 }
 
 // Parts of a tile of n stages when a work-group's share is S.
-__device__ __forceinline__ int qt_parts(int n, int S) { return 2 * (int64_t)n >= 3 * (int64_t)S ? (n + S / 2) / S : 1; }
+__host__ __device__ inline int qt_parts(int n, int S) { return 2 * (int64_t)n >= 3 * (int64_t)S ? (n + S / 2) / S : 1; }
 
 // The batch's tiles f = sequence * row_tiles + tile, a consecutive range for each thread (one
 // tile, up to kQtThreads of them), and the lengths of the first one's sequence.
@@ -1277,10 +1281,15 @@ __global__ __launch_bounds__(kQtThreads) void paged_attention_rows_kernel(AttnPa
   const int tiles = p.num_seqs * p.row_tiles * p.num_kv_heads;
   int* s_scan = (int*)(smem + kQtScanOff);
   int seq, tile, head, part = 0, parts = 1, slot = 0;
-  if ((int)blockIdx.x < tiles) {
+  if (p.row_parts > 0 || (int)blockIdx.x < tiles) {
     int b = blockIdx.x;
     head = b % p.num_kv_heads;
     b /= p.num_kv_heads;
+    if (p.row_parts > 0) {  // the parts of a tile side by side
+      slot = blockIdx.x;
+      part = b % p.row_parts;
+      b /= p.row_parts;
+    }
     seq = b % p.num_seqs;
     tile = p.row_tiles - 1 - b / p.num_seqs;
   } else {
@@ -1306,10 +1315,14 @@ __global__ __launch_bounds__(kQtThreads) void paged_attention_rows_kernel(AttnPa
   const QtItem it = qt_item(p, seq, tile, kTileRows_);
   const int qs = ((const ConstI32*)p.q_start)[seq];
   if (it.stages == 0) return;
+  if (p.row_parts > 0) {
+    parts = qt_parts(it.stages, p.row_share);
+    if (part >= parts) return;
+  }
   if (tid == 0 && it.ctx > p.max_ctx) atomicOr(p.error_flag, 1u);
   const int kstart = (int)((int64_t)it.stages * part / parts) * kQtKeys;
   // whether S decides where this tile's work-group ends
-  const bool whole = part == 0 && p.row_slots > 0 && qt_parts(it.stages, p.row_share) > 1;
+  const bool whole = part == 0 && p.row_extra > 0 && qt_parts(it.stages, p.row_share) > 1;
 
   // ---- this wave's rows ----
   const int r = lane & 15;
@@ -2631,16 +2644,29 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnParams p) {
 }
 
 // Combines the parts' partials of the query-tile kernel's split tiles: 16 rows of a (tile, KV
-// head) at a time, 16 threads per row, 8 dims per thread.  The grid is bounded, since few of
-// the tiles that could be split are.
+// head) at a time, 16 threads per row, 8 dims per thread.  With row_parts every tile is looked
+// at, else those of the list; its grid is bounded, since few of the tiles that could be split are.
 constexpr int kQtMergeGrid = 4 * kNumCu;
 __global__ __launch_bounds__(256) void attention_rows_merge_kernel(AttnParams p, int tile_rows) {
   const int blocks = tile_rows / kRows;
   const ConstI32* all = (const ConstI32*)p.rows_list;  // written by the kernel before
-  const int items = all[0] * blocks;
+  const int entries = p.row_parts > 0 ? p.num_seqs * p.row_tiles * p.num_kv_heads : all[0];
+  const int items = entries * blocks;
   for (int item = blockIdx.x; item < items; item += gridDim.x) {
-    const ConstI32* list = all + (1 + item / blocks) * kQtListInts;
-    const int seq = list[0], tile = list[1], head = list[2], slot = list[3], parts = list[4];
+    const int entry = item / blocks;
+    int seq, tile, head, slot, parts;
+    if (p.row_parts > 0) {
+      head = entry % p.num_kv_heads;
+      const int f = entry / p.num_kv_heads;  // the kernel's order: tiles from the last down, then the sequences
+      seq = f % p.num_seqs;
+      tile = p.row_tiles - 1 - f / p.num_seqs;
+      slot = f * p.row_parts * p.num_kv_heads + head;
+      parts = qt_parts(qt_item(p, seq, tile, tile_rows).stages, p.row_share);
+      if (parts == 1) continue;
+    } else {
+      const ConstI32* list = all + (1 + entry) * kQtListInts;
+      seq = list[0], tile = list[1], head = list[2], slot = list[3], parts = list[4];
+    }
     const int row = item % blocks * kRows + (threadIdx.x >> 4);
     const QtItem it = qt_item(p, seq, tile, tile_rows);
     if (it.row0 + row >= it.rows_total) continue;
@@ -2656,7 +2682,7 @@ __global__ __launch_bounds__(256) void attention_rows_merge_kernel(AttnParams p,
 struct Layout {
   int group, mtiles, units, split_len, max_splits, plan_grid, plan_w;
   // query-tile kernel: key groups per work-group (0: not its shape), tiles per sequence, split slots
-  int rows_kg, row_tiles, row_slots, row_share, row_extra;
+  int rows_kg, row_tiles, row_slots, row_share, row_parts, row_extra;
   size_t part_o_off, part_ml_off, error_off, plan_off, desc_off, slots_off, total;
 };
 
@@ -2740,7 +2766,12 @@ Layout make_layout(int num_seqs, int num_q_heads, int num_kv_heads, int max_q_le
       const int stages = ceil_div(max_ctx, kQtKeys);
       L.row_share = 2 * tiles <= kPlanCUs ? kQtMinSplitStages : kQtManySplitStages;
       L.row_slots = (int)min((int64_t)kQtMaxSlots, tiles * ((stages + 1) / kQtMinSplitStages));
-      L.row_extra = (int)min((int64_t)kNumCu, tiles * ((stages - 1) / kQtMinSplitStages));
+      // the share is at most ceil(tiles stages / 256): where that is the least one the host knows
+      // it, and no work-group has to add up the lengths
+      if (tiles * stages <= (int64_t)L.row_share * kNumCu)
+        L.row_parts = qt_parts(stages, L.row_share);
+      else
+        L.row_extra = (int)min((int64_t)kNumCu, tiles * ((stages - 1) / kQtMinSplitStages));
     }
     const size_t parts = (size_t)L.row_slots * tile_rows;
     size_t at = 256;  // the error flag
@@ -2812,13 +2843,15 @@ int launch_attention_rows_kg(const AttnParams& p, hipStream_t s) {
     set_error("paged_attention_rows_kernel: cannot reserve %d bytes of LDS: %s", kQtLds, hipGetErrorString(attr));
     return NE_ELAUNCH;
   }
-  const int64_t grid = (int64_t)p.num_seqs * p.row_tiles * p.num_kv_heads + p.row_extra;
+  const int64_t tiles = (int64_t)p.num_seqs * p.row_tiles * p.num_kv_heads;
+  const int64_t grid = p.row_parts > 0 ? tiles * p.row_parts : tiles + p.row_extra;
   NE_CHECK_SUPPORTED(grid < (int64_t(1) << 31), "too many query tiles (%lld)", (long long)grid);
   hipLaunchKernelGGL((paged_attention_rows_kernel<INT8, SDT, KG>), dim3((unsigned)grid), dim3(kQtThreads), kQtLds, s,
                      p);
   const int rc = check_launch("paged_attention_rows_kernel");
   if (rc != NE_OK || p.row_slots == 0) return rc;
-  const int merges = min(kQtMergeGrid, p.row_slots / 2 * (qt_rows(KG) / kRows));
+  const int64_t entries = p.row_parts > 0 ? tiles : p.row_slots / 2;
+  const int merges = (int)min((int64_t)kQtMergeGrid, entries * (qt_rows(KG) / kRows));
   hipLaunchKernelGGL(attention_rows_merge_kernel, dim3((unsigned)merges), dim3(256), 0, s, p, qt_rows(KG));
   return check_launch("attention_rows_merge_kernel");
 }
@@ -3010,6 +3043,7 @@ int make_params(const void* q, int64_t q_token_stride, int64_t q_head_stride, co
   p.row_tiles = L.row_tiles;
   p.row_slots = L.row_slots;
   p.row_share = L.row_share;
+  p.row_parts = L.row_parts;
   p.row_extra = L.row_extra;
   p.rows_list = (int32_t*)(ws + L.desc_off);
   return NE_OK;
