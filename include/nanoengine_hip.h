@@ -107,7 +107,8 @@ int ne_kv_write(const void* vectors, int32_t vec_dtype, int64_t n, int32_t num_h
  * int8 / 8-KV-head path then sizes each sequence's splits from the total work, at
  * least 256 keys each).  head_dim must be 128 and block_size a multiple of 16.  One
  * work-group serves every KV head of a sequence's split, or, with more than 32 query rows
- * per KV head and split_len 0 (prefill), one KV head of a tile of 64 to 256 query rows,
+ * per KV head and split_len 0 (prefill, but for many contexts of at most 256 keys), one KV
+ * head of a tile of 64 to 256 query rows,
  * its keys split where they exceed the batch's mean work per CU; splits are combined by a
  * second kernel on the same stream.
  */

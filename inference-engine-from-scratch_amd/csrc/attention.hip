@@ -21,7 +21,8 @@
 //           work-group derives from the context lengths (plan_item); the register
 //           kernels use fixed `split_len` splits.
 //           Prefill (more than 32 rows per KV head) runs a kernel of its own, one KV
-//           head of a tile of query rows per work-group (paged_attention_rows_kernel).
+//           head of a tile of query rows per work-group (paged_attention_rows_kernel),
+//           except for many short contexts (register_serves).
 //   merge = splits store fp32 partials (reference max, sum, unnormalised output;
 //           real rows only) and a second kernel combines them.  No fences or
 //           atomics order the work-groups: the kernel boundary does, which on an
@@ -2740,13 +2741,29 @@ bool rows_split(int64_t tiles, int max_ctx) {
          tiles * stages < (int64_t(1) << 31);
 }
 
-// Whether the query-tile kernel serves a shape: more rows per KV head than the DMA kernel
-// takes and no split length asked for.  Contexts of at most 64 keys stay with the register
-// kernel, which has one split of them and no staging to pay for: 7.4 us against 9.0-9.9 us at
-// 17-32 queries of a bf16 cache.  Of an int8 one the two are even there (9.5-9.7 us against
-// 9.0-9.9 us at 17-64 queries); one line serves both.
-bool rows_serves(int mtiles, int split_len, int max_ctx) {
-  return mtiles > kMaxRowTiles && split_len <= 0 && max_ctx > 4 * kTileKeys;
+// Whether the register kernel serves a prefill shape better than the query-tile kernel: a single
+// split (256 keys of int8, 128 of bf16) in fewer rounds of work-groups.  A work-group of the
+// query-tile kernel fills its CU and takes ~9-12 us for a stage or two however few its rows; one
+// of the register kernel serves 16 rows of all 8 heads, and a round of them costs w times as much:
+// 1 up to 128 int8 keys, 1.5 up to 256 and up to 96 bf16 ones, a little less there with tiles of at
+// most 64 rows (96 x 17 of 65 25.6 / 27.9, 96 x 33 of 96 32.5 / 28.3), and 2 up to 128 bf16 ones, of
+// such tiles alone (48 x 33 23.2 / 19.3).  The line is within 3 % of the
+// better kernel in 97 of 100 shapes measured.  Measured at 33-256 sequences of 17-128 queries, us, register /
+// query-tile kernel, int8: 33 x 17 of 65 keys 12.9 / 18.2, 64 x 32 of 128 18.0 / 21.1, 200 x 17 of
+// 65 33.4 / 62.0, 128 x 24 of 200 39.7 / 45.0, 100 x 48 of 96 35.0 / 38.1; but 32 x 17 of 65 12.8 /
+// 10.2, 64 x 33 of 65 22.5 / 17.9, 96 x 17 of 256 40.3 / 34.7, 150 x 64 of 128 64.3 / 56.0.  bf16:
+// 64 x 17 of 65 16.1 / 18.4, 200 x 24 of 96 43.9 / 64.2, 100 x 32 of 128 36.1 / 40.4; 64 x 17 of 160
+// 44.2 / 24.7 (two splits), 64 x 48 of 96 27.9 / 21.3.  Contexts of at most 64 keys always go there
+// (one sequence of 17-32 queries, bf16, 7.4 us against 9.0-9.9; int8 even, 9.5-9.7 against 9.0-9.9).
+bool register_serves(int kv_dtype, int64_t mtiles, int num_seqs, int num_kv_heads, int64_t tiles, int max_ctx) {
+  if (max_ctx <= 4 * kTileKeys) return true;
+  const bool int8 = kv_dtype == NE_DTYPE_INT8;
+  if (max_ctx > (int8 ? 256 : 128)) return false;
+  const bool one_tile = mtiles * kRows <= qt_rows(4);
+  if (!int8 && max_ctx > 96 && !one_tile) return false;
+  const double w = int8 ? (max_ctx <= 128 ? 1.0 : 1.5) : (max_ctx > 96 ? 1.95 : one_tile ? 1.45 : 1.5);
+  const int64_t rounds = (int64_t)ceil_div(num_seqs * mtiles, kNumCu) * ceil_div(num_kv_heads, kHeadWaves);
+  return w * (double)rounds < (double)ceil_div(tiles, kNumCu);
 }
 
 // rows_path: whether the query-tile kernel may serve the shape.
@@ -2756,12 +2773,21 @@ Layout make_layout(int num_seqs, int num_q_heads, int num_kv_heads, int max_q_le
   L.group = num_q_heads / num_kv_heads;
   L.mtiles = ceil_div((int64_t)L.group * max_q_len, kRows);
   L.units = num_seqs * num_kv_heads * L.mtiles;
-  if (rows_path && rows_serves(L.mtiles, split_len, max_ctx)) {
+  if (rows_path && L.mtiles > kMaxRowTiles && split_len <= 0) {
     const int64_t rows = (int64_t)L.group * max_q_len;
-    L.rows_kg = rows_key_groups(rows, (int64_t)num_seqs * num_kv_heads, max_ctx);
-    const int tile_rows = qt_rows(L.rows_kg);
-    L.row_tiles = ceil_div(rows, tile_rows);
-    const int64_t tiles = (int64_t)num_seqs * num_kv_heads * L.row_tiles;
+    const int kg = rows_key_groups(rows, (int64_t)num_seqs * num_kv_heads, max_ctx);
+    const int tile_rows = qt_rows(kg);
+    const int row_tiles = ceil_div(rows, tile_rows);
+    const int64_t tiles = (int64_t)num_seqs * num_kv_heads * row_tiles;
+    size_t at = 256;  // the error flag
+    if (register_serves(kv_dtype, L.mtiles, num_seqs, num_kv_heads, tiles, max_ctx)) {
+      L.split_len = default_split_len(kv_dtype, max_ctx);
+      L.max_splits = 1;
+      L.part_o_off = L.part_ml_off = L.plan_off = L.desc_off = L.slots_off = L.total = at;
+      return L;
+    }
+    L.rows_kg = kg;
+    L.row_tiles = row_tiles;
     if (rows_split(tiles, max_ctx)) {
       const int stages = ceil_div(max_ctx, kQtKeys);
       L.row_share = 2 * tiles <= kPlanCUs ? kQtMinSplitStages : kQtManySplitStages;
@@ -2774,7 +2800,6 @@ Layout make_layout(int num_seqs, int num_q_heads, int num_kv_heads, int max_q_le
         L.row_extra = (int)min((int64_t)kNumCu, tiles * ((stages - 1) / kQtMinSplitStages));
     }
     const size_t parts = (size_t)L.row_slots * tile_rows;
-    size_t at = 256;  // the error flag
     L.part_o_off = at;
     at += parts * kHeadDim * sizeof(float);
     L.part_ml_off = at;

@@ -96,6 +96,33 @@ def test_uneven_contexts_split_by_their_work(device, q_lens, pasts, heads, kv):
     assert rel_err(got, ref) < TOL
 
 
+# many short sequences: the register kernel's fewer rounds, on both sides of the rule's lines
+@pytest.mark.parametrize("kv,seqs,q,ctx,register", [
+    ("int8", 33, 17, 65, True), ("int8", 64, 32, 128, True), ("int8", 130, 24, 200, True), ("int8", 64, 17, 256, True),
+    ("int8", 32, 17, 65, False), ("int8", 64, 33, 128, False), ("int8", 64, 17, 257, False), ("int8", 96, 17, 250, False),
+    ("bf16", 64, 17, 65, True), ("bf16", 100, 32, 128, True), ("bf16", 64, 17, 129, False), ("bf16", 64, 48, 96, False),
+    ("bf16", 96, 17, 65, True), ("bf16", 48, 33, 128, False),
+])
+def test_many_short_sequences_run_the_register_kernel(device, kv, seqs, q, ctx, register):
+    """Where the register kernel serves a call it gives the bits of a call that asks for its
+    split; the query-tile kernel adds in another order."""
+    blocks = -(-ctx // 16)
+    kc, vc, ks, vs = make_pool(seqs * blocks, 16, 8, kv, seed=71)
+    q_lens = [q - i % 3 for i in range(seqs)]
+    tables, ctx_t, qs, ql, rows = make_batch([ctx - i % 40 for i in range(seqs)][:seqs - 1] + [ctx], q_lens,
+                                             seqs * blocks, 16, seed=72)
+    x = torch.randn(rows, 16, 128, generator=torch.Generator().manual_seed(73)).to(torch.bfloat16)
+    d = lambda t: None if t is None else t.to(device)
+    args = [d(t) for t in (x, kc, vc, ks, vs, tables)] + [16] + [d(t) for t in (ctx_t, qs, ql)]
+    ws = kernels.AttentionWorkspace()
+    got = kernels.paged_verify_attention(*args, max_q_len=q, max_ctx_len=ctx, workspace=ws)
+    asked = kernels.paged_verify_attention(*args, max_q_len=q, max_ctx_len=ctx, split_len=256 if kv == "int8" else 128)
+    torch.cuda.synchronize()
+    assert ws.error_flag() == 0 and torch.equal(got, asked) == register
+    ref = paged_attention_reference(x, kc, vc, ks, vs, tables, 16, ctx_t, qs, ql, model_dtype=torch.bfloat16)
+    assert rel_err(got.cpu(), ref) < TOL
+
+
 def test_captured_and_allocation_free_calls_split_by_the_lengths_of_the_replay(device):
     """A graph captured once with bounds serves batches of other lengths, with eager work between
     its replays; the library's own scratch gives the same bits as a workspace."""
