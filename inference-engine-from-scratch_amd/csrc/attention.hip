@@ -1581,6 +1581,11 @@ constexpr int kWholeMaxTiles = 64;                    // longest context of a wh
 // -> 28.8; 24 of 300-2,000 24.3 -> 24.2 (bf16 33.0 -> 31.4).  32 such sequences lose with 4
 // (28.8 -> 29.5) and gain with 2 (25.8); 48 are even with 2 (34.4, 34.8) and 64 lose
 // (200-1,500 keys 34.2 -> 37.1).
+// Four waves leave 64 items, so past 12 sequences a long one is cut too coarsely: 24 of
+// 4,800-8,000 keys take 66.5 us with one wave, 75.2 with four and 65 with two, 20 of 4,800-16,000
+// (int8, ratio to one wave) 1.07-1.11 with four and 0.97-1.01 with two.  16 sequences keep four up
+// to 8,192 keys (0.91-0.97 of one wave's time at 8,000, 1.03 at 16,000), 17-24 up to 4,608 tiles in
+// all (24 x 3,072 keys), and take two beyond.
 // From 641 to 1,024 keys a planned call can also give every sequence one whole item, without
 // partials and merge.  Measured with bounds of 700 and 1,000 keys, whole -> split, int8 / bf16:
 // contexts of 25-100 % of 1,000 keys 2 sequences 15.2 -> 10.9 / 13.6 -> 10.4 us, 12 15.3 ->
@@ -1590,6 +1595,9 @@ constexpr int kWholeMaxTiles = 64;                    // longest context of a wh
 // whatever their number (100-250 keys of 1,000: 8.2 -> 9.6).  So up to 12 sequences are split,
 // more stay whole.  An unplanned call has no whole items and splits all of them.
 constexpr int kSplitKs4MaxSeqs = 24;
+constexpr int kSplitKs4AnySeqs = 12;
+constexpr int kSplitKs4MaxTiles16 = 8192;  // of all sequences, at the bound
+constexpr int kSplitKs4MaxTiles24 = 4608;
 constexpr int kSplitKs2MaxSeqs = 40;
 constexpr int kSplitKs4MinTiles = 40;
 constexpr int kSplitOverWholeMaxSeqs = 12;
@@ -1598,7 +1606,10 @@ int split_plan_grid(int num_seqs, int ks) { return max(kPlanCUs / ks, 2 * num_se
 int split_plan_ks(int num_seqs, int max_ctx, int split_len, int mtiles) {
   const int64_t tiles = ((int64_t)max_ctx + kTileKeys - 1) / kTileKeys;
   if (split_len != 0 || mtiles != 1) return 1;
-  const int ks = num_seqs <= kSplitKs4MaxSeqs ? 4 : num_seqs <= kSplitKs2MaxSeqs ? 2 : 1;
+  const bool four = num_seqs <= kSplitKs4AnySeqs ||
+                    (num_seqs <= kSplitKs4MaxSeqs &&
+                     num_seqs * tiles <= (num_seqs <= 16 ? kSplitKs4MaxTiles16 : kSplitKs4MaxTiles24));
+  const int ks = four ? 4 : num_seqs <= kSplitKs2MaxSeqs ? 2 : 1;
   if (tiles <= (ks == 4 ? kSplitKs4MinTiles : kWholeMaxTiles)) return 1;
   // every item's slot list holds its tiles
   const int64_t need = num_seqs + (num_seqs * tiles + kPlanMaxTiles - 1) / kPlanMaxTiles;

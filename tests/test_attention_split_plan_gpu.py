@@ -21,7 +21,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("kv", ["bf16", "int8"])
 @pytest.mark.parametrize("seqs,longest", [(1, 641), (1, 2500), (3, 640), (12, 700), (13, 700), (24, 700), (25, 1024), (25, 1025), (40, 1100),
-                                          (41, 1100)])
+                                          (41, 1100), (16, 8192), (16, 8193), (24, 3072), (24, 3073)])
 def test_split_items(device, kv, seqs, longest):
     ctx = [longest] + [1 + 37 * i % 300 for i in range(seqs - 1)]
     ctx[-1] = longest - 1 if seqs > 1 else longest
