@@ -106,13 +106,14 @@ struct AttnParams {
   int32_t max_ctx;     // the caller's bound on ctx_len
   int32_t rows_kg;     // query-tile kernel: key groups per work-group (0: another kernel serves the call)
   int32_t row_tiles;   // query-tile kernel: tiles of query rows per sequence
+  int32_t* plan_desc;  // precomputed plan: [plan_grid][8] work items (seq < 0: none)
+  int32_t* plan_slots; // precomputed plan: [plan_grid][kPlanMaxTiles] first slot of each tile
+  // (the query-tile kernel's own, last: the other kernels' arguments keep their places)
   int32_t row_slots;   // query-tile kernel: partials of split tiles (0: no splits)
   int32_t row_share;   // query-tile kernel: least stages per work-group of a split tile
   int32_t row_parts;   // query-tile kernel: work-groups of every tile where row_share is the batch's share (else 0)
   int32_t row_extra;   // query-tile kernel: work-groups for the parts after a tile's first
   int32_t* rows_list;  // query-tile kernel: the split tiles' merges, [1 + row_slots / 2][kQtListInts], the count first
-  int32_t* plan_desc;  // precomputed plan: [plan_grid][8] work items (seq < 0: none)
-  int32_t* plan_slots; // precomputed plan: [plan_grid][kPlanMaxTiles] first slot of each tile
 };
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));

@@ -1240,7 +1240,7 @@ __global__ __launch_bounds__(L::WAVES* kWave) void proj_few_rows_kernel(GemmPara
 #pragma unroll
     for (int j = 0; j < L::kPerWave; ++j) {
       const int i = j * L::WAVES + wave;  // KiB: stage i / (4 PM), rows 4 (i % (4 PM)) .. + 4
-      if (i >= L::kCopies) break;         // wave-uniform
+      if (L::kCopies % L::WAVES != 0 && i >= L::kCopies) break;  // wave-uniform
       const int t = i / (4 * PM);
       const int row = (i % (4 * PM)) * 4 + (lane >> 4);
       // rows past m re-read row m - 1 and are never stored
