@@ -1445,48 +1445,50 @@ int launch_few(const GemmParams& p, int splits, float* partial, hipStream_t s, c
 
 template <int SDT>
 int dispatch_qkv_fused(GemmParams p, const QkvRopeArgs& qa, int kv_mode, hipStream_t s) {
-  if (few_rows(p, 1)) {
-    if (kv_mode == 1) return launch_few<1, kKgQkv, 8, 4, 1>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
-    if (kv_mode == 2) return launch_few<1, kKgQkv, 8, 4, 2>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
-    return launch_few<1, kKgQkv, 8, 4, 3>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
-  }
+  const char* name = "w8a16_qkv_norm_rope_kv";
+  const bool few = few_rows(p, 1);
   // the tiles' epilogue stores 4 or 8 bytes at a time where the row kernel's stores elements
   const bool aligned = (((uintptr_t)qa.q_out | (uintptr_t)qa.rope | (uintptr_t)qa.k_cache | (uintptr_t)qa.v_cache) % 8) == 0;
-  const ProjTile tile = aligned ? choose_proj_tile(p.m, p.n, false) : ProjTile::kVerify;
-  if (tile != ProjTile::kVerify) {
-    if (kv_mode == 1) return launch_proj_tile<4, 1>(tile, p, s, "w8a16_qkv_norm_rope_kv", qa);
-    if (kv_mode == 2) return launch_proj_tile<4, 2>(tile, p, s, "w8a16_qkv_norm_rope_kv", qa);
-    return launch_proj_tile<4, 3>(tile, p, s, "w8a16_qkv_norm_rope_kv", qa);
+  const ProjTile tile = !few && aligned ? choose_proj_tile(p.m, p.n, false) : ProjTile::kVerify;
+  if (!few && tile == ProjTile::kVerify) {
+    switch (kv_mode) {
+      // 48-row tiles: 7 x 32 = 224 work-groups for 320 rows, 3 rows per wave in the epilogue
+      case 1: return launch_proj<8, SDT, 4, 1, 3, kKgQkv, kNpwQkv>(p, 1, nullptr, s, name, qa);
+      case 2: return launch_proj<8, SDT, 4, 2, 3, kKgQkv, kNpwQkv>(p, 1, nullptr, s, name, qa);
+      default: return launch_proj<8, SDT, 4, 3, 3, kKgQkv, kNpwQkv>(p, 1, nullptr, s, name, qa);
+    }
   }
-  switch (kv_mode) {
-    // 48-row tiles: 7 x 32 = 224 work-groups for 320 rows, 3 rows per wave in the epilogue
-    case 1: return launch_proj<8, SDT, 4, 1, 3, kKgQkv, kNpwQkv>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
-    case 2: return launch_proj<8, SDT, 4, 2, 3, kKgQkv, kNpwQkv>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
-    default: return launch_proj<8, SDT, 4, 3, 3, kKgQkv, kNpwQkv>(p, 1, nullptr, s, "w8a16_qkv_norm_rope_kv", qa);
+  if (few) {
+    if (kv_mode == 1) return launch_few<1, kKgQkv, 8, 4, 1>(p, 1, nullptr, s, name, qa);
+    if (kv_mode == 2) return launch_few<1, kKgQkv, 8, 4, 2>(p, 1, nullptr, s, name, qa);
+    return launch_few<1, kKgQkv, 8, 4, 3>(p, 1, nullptr, s, name, qa);
   }
+  if (kv_mode == 1) return launch_proj_tile<4, 1>(tile, p, s, name, qa);
+  if (kv_mode == 2) return launch_proj_tile<4, 2>(tile, p, s, name, qa);
+  return launch_proj_tile<4, 3>(tile, p, s, name, qa);
 }
 
 template <int SDT>
 int dispatch_w8a16(GemmParams p, int epilogue, int splits, float* partial, hipStream_t s) {
-  if (few_rows(p, partial != nullptr ? splits : 1)) {
-    if (epilogue == NE_EPILOGUE_SWIGLU) return launch_few<2, kKgSwiglu, 2, 1, 0>(p, 1, nullptr, s, "w8a16_swiglu");
+  const bool swiglu = epilogue == NE_EPILOGUE_SWIGLU;
+  const bool few = few_rows(p, partial != nullptr ? splits : 1);
+  const ProjTile tile = !few && partial == nullptr ? choose_proj_tile(p.m, p.n, swiglu) : ProjTile::kVerify;
+  if (!few && tile == ProjTile::kVerify) {
+    if (swiglu) {
+      if (p.n % 96 == 0)
+        return launch_proj<6, SDT, 1, 0, kPM, kKgSwiglu, kNpwSwiglu>(p, 1, nullptr, s, "w8a16_swiglu");
+      return launch_proj<4, SDT, 1, 0, kPM, kKgSwiglu, kNpwSwiglu>(p, 1, nullptr, s, "w8a16_swiglu");
+    }
+    if (partial != nullptr)
+      return launch_proj<4, SDT, 3, 0, kSplitPM, kKgPlain, kNpwPlain>(p, splits, partial, s, "w8a16_splitk");
+    return launch_proj<4, SDT, 0, 0, kPM, kKgPlain, kNpwPlain>(p, 1, nullptr, s, "w8a16_gemm");
+  }
+  if (few) {
+    if (swiglu) return launch_few<2, kKgSwiglu, 2, 1, 0>(p, 1, nullptr, s, "w8a16_swiglu");
     if (partial != nullptr) return launch_few<1, kKgPlain, 2, 3, 0>(p, splits, partial, s, "w8a16_splitk");
     return launch_few<1, kKgPlain, 2, 0, 0>(p, 1, nullptr, s, "w8a16_gemm");
   }
-  if (partial == nullptr) {
-    const bool swiglu = epilogue == NE_EPILOGUE_SWIGLU;
-    const ProjTile tile = choose_proj_tile(p.m, p.n, swiglu);
-    if (tile != ProjTile::kVerify)
-      return swiglu ? launch_proj_tile<1, 0>(tile, p, s, "w8a16_swiglu") : launch_proj_tile<0, 0>(tile, p, s, "w8a16_gemm");
-  }
-  if (epilogue == NE_EPILOGUE_SWIGLU) {
-    if (p.n % 96 == 0)
-      return launch_proj<6, SDT, 1, 0, kPM, kKgSwiglu, kNpwSwiglu>(p, 1, nullptr, s, "w8a16_swiglu");
-    return launch_proj<4, SDT, 1, 0, kPM, kKgSwiglu, kNpwSwiglu>(p, 1, nullptr, s, "w8a16_swiglu");
-  }
-  if (partial != nullptr)
-    return launch_proj<4, SDT, 3, 0, kSplitPM, kKgPlain, kNpwPlain>(p, splits, partial, s, "w8a16_splitk");
-  return launch_proj<4, SDT, 0, 0, kPM, kKgPlain, kNpwPlain>(p, 1, nullptr, s, "w8a16_gemm");
+  return swiglu ? launch_proj_tile<1, 0>(tile, p, s, "w8a16_swiglu") : launch_proj_tile<0, 0>(tile, p, s, "w8a16_gemm");
 }
 
 // ---- LM head: persistent work-groups over the vocabulary -------------------------
