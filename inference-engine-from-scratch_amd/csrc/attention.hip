@@ -208,7 +208,7 @@ __device__ __forceinline__ UnitInfo unit_info(const AttnParams& p, int unit) {
     // the largest query index among this tile's rows bounds the keys it can see
     const int first_i = u.row0 % u.ql;
     const int max_i = (first_i + rows_here > u.ql) ? u.ql - 1 : first_i + rows_here - 1;
-    u.kend_unit = u.ctx - u.ql + max_i + 1;
+    u.kend_unit = min(u.ctx - u.ql + max_i + 1, p.max_ctx);  // keys past the caller's bound are dropped
     u.n_splits = max(0, (u.kend_unit + p.split_len - 1) / p.split_len);
   }
   return u;
@@ -646,11 +646,8 @@ __global__ __launch_bounds__(kHeadWaves * KG * kWave) void paged_attention_kerne
   // the geometry below does not depend on the head
   const UnitInfo u0 = unit_info(p, seq * p.num_kv_heads * p.mtiles + mt);
   if (u0.row0 >= u0.rows_total) return;
-  int n_splits = u0.n_splits;
-  if (n_splits > p.max_splits) {
-    if (tid == 0 && split == 0) atomicOr(p.error_flag, 1u);
-    n_splits = p.max_splits;
-  }
+  if (tid == 0 && split == 0 && u0.ctx > p.max_ctx) atomicOr(p.error_flag, 1u);
+  const int n_splits = u0.n_splits;  // at most max_splits: kend_unit is at most max_ctx
   if (split >= n_splits) return;
   const int kstart = split * p.split_len;
   const int kend = min(u0.kend_unit, kstart + p.split_len);
@@ -2643,7 +2640,7 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnParams p) {
   const int unit = blockIdx.x;
   const UnitInfo u = unit_info(p, unit);
   if (u.row0 >= u.rows_total) return;
-  const int n_splits = min(u.n_splits, p.max_splits);
+  const int n_splits = u.n_splits;
   if (n_splits <= 1) return;
   const int crow = threadIdx.x >> 4;
   const int cd = (threadIdx.x & 15) * 8;

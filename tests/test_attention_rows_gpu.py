@@ -241,13 +241,16 @@ def test_context_past_the_bound_is_flagged(device):
 
 
 # contexts past the bound: the first rows see keys up to their own position, the others those
-# below the bound; a bound shorter than the queries
+# below the bound; a bound shorter than the queries; many short contexts (the register kernel,
+# whose one split of 256 or 128 keys reaches past the bound)
 @pytest.mark.parametrize("kv", ["bf16", "int8"])
-@pytest.mark.parametrize("q_lens,ctx_lens,bound", [([40, 40], [500, 60], 400), ([300, 70], [330, 70], 200)])
+@pytest.mark.parametrize("q_lens,ctx_lens,bound", [
+    ([40, 40], [500, 60], 400), ([300, 70], [330, 70], 200), ([17] * 40, [30] * 38 + [140, 125], 120),
+])
 def test_keys_past_the_bound_are_dropped(device, kv, q_lens, ctx_lens, bound):
     ws = kernels.AttentionWorkspace()
-    kc, vc, ks, vs = make_pool(64, 16, 8, kv)
-    tables, ctx, qs, ql, rows = make_batch(ctx_lens, q_lens, 64, 16)
+    kc, vc, ks, vs = make_pool(128, 16, 8, kv)
+    tables, ctx, qs, ql, rows = make_batch(ctx_lens, q_lens, 128, 16)
     q = torch.randn(rows, 16, 128, generator=torch.Generator().manual_seed(51)).to(torch.bfloat16)
     # every query as a sequence of its own, which sees min(position + 1, bound) keys
     seq = torch.repeat_interleave(torch.arange(len(q_lens)), ql.long())
